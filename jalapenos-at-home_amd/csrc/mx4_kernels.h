@@ -151,9 +151,12 @@ hipError_t launch_synth_bf16(uint64_t seed, double sigma, uint64_t start, uint64
                              uint16_t* out, hipStream_t s);
 hipError_t launch_synth_weight(uint64_t seed, double sigma, uint32_t rows, uint32_t cols,
                                uint8_t* packed, uint8_t* scales, hipStream_t s);
-// Smallest scale byte of a resident weight (flags subnormal-scale blocks)
-hipError_t launch_min_max_scale(const uint8_t* scales, uint64_t count, uint32_t* out2,
-                                hipStream_t s);
+// Smallest and largest scale byte of a resident weight, one pair per block of
+// the launch (min_max_scale_blocks(count), at most kMinMaxBlocks): the caller
+// folds the pairs out[2 b], out[2 b + 1].
+constexpr uint32_t kMinMaxBlocks = 256;
+uint32_t min_max_scale_blocks(uint64_t count);
+hipError_t launch_min_max_scale(const uint8_t* scales, uint64_t count, uint32_t* out, hipStream_t s);
 // Hardware-converter table for the exhaustive decode check: out[s*16 + c]
 hipError_t launch_decode_table(int mode, float* out, hipStream_t s);
 // Matrix-core ceiling probe (probe.hip): back-to-back scaled FP4 MFMAs

@@ -423,34 +423,62 @@ hipError_t launch_decode_table(int mode, float* out, hipStream_t s) {
     return hipGetLastError();
 }
 
-// Smallest and largest scale byte (out2[0] = min, out2[1] = max); out2 must
-// start at {255, 0}.
-__global__ __launch_bounds__(256) void min_max_scale_kernel(const uint8_t* __restrict__ scales,
-                                                            uint64_t count, uint32_t* out2) {
+// Smallest and largest scale byte: block b writes its own pair to out[2 b],
+// out[2 b + 1] and the host, which waits for the result anyway, folds the
+// pairs. Bound by the read of the scales (1.5 MiB for 12288 x 4096), so the
+// bytes come in 16 at a time and nothing is written twice: a byte per thread
+// with two atomics per wave on one word each serialised on those words (16
+// thousand of them: 189 us at 12288 x 4096, and 318 -> 129 us for a quantize +
+// wrap + dequantize of that weight without them). The bytes before the
+// first and after the last whole 16-byte piece go one per thread to block 0.
+__global__ __launch_bounds__(256) void min_max_scale_kernel(const uint8_t* __restrict__ scales, uint64_t count,
+                                                            uint32_t* __restrict__ out) {
+    uint64_t head = (16 - ((uintptr_t)scales & 15)) & 15;
+    head = head < count ? head : count;
+    const uint64_t pieces = (count - head) / 16, tail = head + 16 * pieces;
     uint32_t lo = 255, hi = 0;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count;
+    // (a thread without a byte keeps {255, 0}: its lo may not count as a maximum, nor its hi as a minimum)
+    auto take = [&](uint32_t a, uint32_t b) {
+        lo = a < lo ? a : lo;
+        hi = b > hi ? b : hi;
+    };
+    if (blockIdx.x == 0) {
+        if (threadIdx.x < head) take(scales[threadIdx.x], scales[threadIdx.x]);
+        if (tail + threadIdx.x < count) take(scales[tail + threadIdx.x], scales[tail + threadIdx.x]);
+    }
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < pieces;
          i += (uint64_t)gridDim.x * blockDim.x) {
-        uint32_t v = scales[i];
-        lo = v < lo ? v : lo;
-        hi = v > hi ? v : hi;
+        const u32x4 v = load_u32x4(scales + head + 16 * i);
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) take((v[d] >> (8 * e)) & 0xffu, (v[d] >> (8 * e)) & 0xffu);
     }
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {
-        uint32_t a = __shfl_xor(lo, off, 64), b = __shfl_xor(hi, off, 64);
-        lo = a < lo ? a : lo;
-        hi = b > hi ? b : hi;
+        take(__shfl_xor(lo, off, 64), __shfl_xor(hi, off, 64));
     }
+    __shared__ uint32_t part[4][2];
     if (threadIdx.x % 64 == 0) {
-        atomicMin(out2, lo);
-        atomicMax(out2 + 1, hi);
+        part[threadIdx.x / 64][0] = lo;
+        part[threadIdx.x / 64][1] = hi;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int w = 1; w < 4; ++w) take(part[w][0], part[w][1]);
+        out[2 * blockIdx.x] = lo;
+        out[2 * blockIdx.x + 1] = hi;
     }
 }
 
-hipError_t launch_min_max_scale(const uint8_t* scales, uint64_t count, uint32_t* out2, hipStream_t s) {
-    uint64_t groups = (count + 255) / 256;
-    if (groups > 2048) groups = 2048;
-    if (groups == 0) groups = 1;
-    hipLaunchKernelGGL(min_max_scale_kernel, dim3((unsigned)groups), dim3(256), 0, s, scales, count, out2);
+uint32_t min_max_scale_blocks(uint64_t count) {
+    const uint64_t blocks = (count / 16 + 255) / 256;
+    return (uint32_t)(blocks < 1 ? 1 : blocks > kMinMaxBlocks ? kMinMaxBlocks : blocks);
+}
+
+hipError_t launch_min_max_scale(const uint8_t* scales, uint64_t count, uint32_t* out, hipStream_t s) {
+    hipLaunchKernelGGL(min_max_scale_kernel, dim3(min_max_scale_blocks(count)), dim3(256), 0, s, scales, count, out);
     return hipGetLastError();
 }
 

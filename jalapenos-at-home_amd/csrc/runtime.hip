@@ -59,6 +59,7 @@ struct CacheKeyHash {
 };
 
 constexpr uint64_t kDefaultCacheLimit = 64ull << 30;
+constexpr uint32_t kMinMaxAt = 64;  // first min/max word of mx4_context::flags
 
 }  // namespace
 
@@ -100,7 +101,7 @@ struct mx4_context {
     hipStream_t own = nullptr;
     hipStream_t stream = nullptr;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
-    uint32_t* flags = nullptr;  // device scratch: [0] bad flag, [1..2] min/max scale
+    uint32_t* flags = nullptr;  // device scratch: [0] bad flag, [kMinMaxAt..] min/max scale pairs
     // per-call drop-in state
     std::unordered_map<CacheKey, CacheEntry, CacheKeyHash> cache;
     std::list<CacheKey> lru;
@@ -471,7 +472,7 @@ mx4_status mx4_create(int device, mx4_context** out) {
     if (hipGetDeviceProperties(&prop, device) == hipSuccess) ctx->cus = prop.multiProcessorCount;
     if (hipStreamCreateWithFlags(&ctx->own, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreate(&ctx->ev0) != hipSuccess || hipEventCreate(&ctx->ev1) != hipSuccess ||
-        hipMalloc((void**)&ctx->flags, 256) != hipSuccess ||
+        hipMalloc((void**)&ctx->flags, (kMinMaxAt + 2 * mx4::kMinMaxBlocks) * 4) != hipSuccess ||
         hipMalloc((void**)&ctx->am_partial, kArgmaxPartials * sizeof(uint64_t)) != hipSuccess ||
         hipMalloc((void**)&ctx->split_part, (size_t)kSplitPartBytes) != hipSuccess ||
         hipMalloc((void**)&ctx->split_count, kSplitCounts * sizeof(uint32_t)) != hipSuccess ||
@@ -641,12 +642,15 @@ mx4_status mx4_weight_wrap(mx4_context* ctx, const uint8_t* packed_dev, const ui
     if (((uintptr_t)packed_dev & 15) != 0) return fail(MX4_ERR_ARGUMENT, "packed data must be 16-byte aligned");
     DeviceGuard g(ctx->device);
     const uint64_t sbytes = (uint64_t)rows * cols / 32;
-    HIP_TRY(mx4::launch_fill_u32(ctx->flags + 1, 2, 0, ctx->stream));
-    HIP_TRY(mx4::launch_fill_u32(ctx->flags + 1, 1, 255, ctx->stream));
-    HIP_TRY(mx4::launch_min_max_scale(scales_dev, sbytes, ctx->flags + 1, ctx->stream));
-    uint32_t mm[2];
-    HIP_TRY(hipMemcpyAsync(mm, ctx->flags + 1, 8, hipMemcpyDeviceToHost, ctx->stream));
+    HIP_TRY(mx4::launch_min_max_scale(scales_dev, sbytes, ctx->flags + kMinMaxAt, ctx->stream));
+    const uint32_t pairs = mx4::min_max_scale_blocks(sbytes);
+    uint32_t mm[2 * mx4::kMinMaxBlocks];
+    HIP_TRY(hipMemcpyAsync(mm, ctx->flags + kMinMaxAt, pairs * 8, hipMemcpyDeviceToHost, ctx->stream));
     HIP_TRY(hipStreamSynchronize(ctx->stream));
+    for (uint32_t b = 1; b < pairs; ++b) {
+        mm[0] = std::min(mm[0], mm[2 * b]);
+        mm[1] = std::max(mm[1], mm[2 * b + 1]);
+    }
     if (mm[1] == 255) return fail(MX4_ERR_NAN_SCALE, "MXFP4 checkpoint contains a NaN scale");
     mx4_weight* w = nullptr;
     mx4_status st = new_weight(ctx, rows, cols, &w);
