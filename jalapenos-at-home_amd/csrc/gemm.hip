@@ -27,7 +27,10 @@
 //    reference's sequential loop (engine/src/lib.rs:240-266);
 //  * every global load goes through a buffer resource: token rows >= M and
 //    weight rows >= N read as zeros without touching memory, and their outputs
-//    are not stored.
+//    are not stored;
+//  * widths that are no whole number of stages (any K % 32 == 0: the ANY
+//    instances) zero the last stage's columns past K the same way, and take
+//    the scale bytes, whose rows then start at any byte, as aligned words.
 #include <type_traits>
 #include "mx4_device.h"
 #include "mx4_kernels.h"
@@ -73,6 +76,8 @@ __device__ __forceinline__ void mfma_drain() {
 
 constexpr int kBK = 128;  // K elements per stage
 
+typedef double f64x16 __attribute__((ext_vector_type(16)));
+
 // Stage layout in LDS (no padding): activations BM rows x A_CPR 16-byte slots,
 // packed weights BN rows x 4 slots, then BN scale words. Slots are written by
 // direct-to-LDS buffer loads, lane l of a load instruction at slot base + l,
@@ -80,19 +85,23 @@ constexpr int kBK = 128;  // K elements per stage
 // of row r sits in slot c ^ (r % 16) of an activation row and c ^ ((r / 4) % 4)
 // of a weight row. The MFMA-operand reads (32 rows, one logical chunk) then
 // spread over all LDS banks.
-template <bool XBF16, int WM, int WN, int TM, int TN, int D>
+//
+// ANY: K is any multiple of 32. A stage's four scale bytes of a row then lie
+// anywhere in two aligned words, so the stage holds both and the reader shifts.
+template <bool XBF16, int WM, int WN, int TM, int TN, int D, bool ANY>
 struct Geometry {
     static constexpr int NW = WM * WN, NT = 64 * NW;
     static constexpr int BM = 32 * TM * WM, BN = 32 * TN * WN;
     static constexpr int XB = XBF16 ? 2 : 4;              // bytes per activation element
     static constexpr int A_CPR = kBK * XB / 16;           // 16-byte chunks per activation row
-    static constexpr int A_BYTES = BM * A_CPR * 16, B_BYTES = BN * 4 * 16, S_BYTES = BN * 4;
+    static constexpr int A_BYTES = BM * A_CPR * 16, B_BYTES = BN * 4 * 16, S_BYTES = BN * (ANY ? 8 : 4);
     static constexpr int STAGE = A_BYTES + B_BYTES + S_BYTES;
     static constexpr int A_INSTR = BM * A_CPR / NT;       // 64-lane loads per wave per stage
     static constexpr int B_INSTR = BN * 4 / NT;
-    static constexpr int S_ROWS = BN / NW;                // scale words per wave per stage
-    static constexpr int LPS = A_INSTR + B_INSTR + 1;     // vector memory instructions per stage
-    static_assert(BM * A_CPR % NT == 0 && BN * 4 % NT == 0 && BN % NW == 0 && S_ROWS <= 64, "stage split");
+    static constexpr int S_WORDS = BN / NW * (ANY ? 2 : 1);  // scale words per wave per stage
+    static constexpr int S_INSTR = (S_WORDS + 63) / 64;
+    static constexpr int LPS = A_INSTR + B_INSTR + S_INSTR;  // vector memory instructions per stage
+    static_assert(BM * A_CPR % NT == 0 && BN * 4 % NT == 0 && BN % NW == 0, "stage split");
     static_assert(D >= 2 && D <= 4 && (D - 2) * LPS <= 63, "vmcnt range");
     static_assert(D * STAGE <= 160 * 1024, "the stages must fit the LDS");
 };
@@ -112,7 +121,9 @@ struct GemmSegs {
     uint32_t count;
 };
 
-template <bool XBF16, int WM, int WN, int TM, int TN, int D, class SG = NoGemmSegs>
+constexpr uint32_t kPastEnd = 0xffffff00u;  // past every buffer resource: a load there returns zeros
+
+template <bool XBF16, int WM, int WN, int TM, int TN, int D, bool ANY = false, class SG = NoGemmSegs>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_exact_kernel(const uint8_t* __restrict__ packed,
                                                                   const uint8_t* __restrict__ scales,
                                                                   const void* __restrict__ x, float* __restrict__ y,
@@ -120,7 +131,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_exact_kernel(const uint8_t*
                                                                   uint32_t tiles_n, uint32_t tiles,
                                                                   uint32_t kslice, float* __restrict__ part,
                                                                   const SG group) {
-    using G = Geometry<XBF16, WM, WN, TM, TN, D>;
+    using G = Geometry<XBF16, WM, WN, TM, TN, D, ANY>;
     __shared__ __attribute__((aligned(16))) uint8_t lds[D * G::STAGE];
     const uint32_t lane = threadIdx.x % 64, h = lane / 32, r32 = lane % 32;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -149,53 +160,84 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_exact_kernel(const uint8_t*
         tn -= t0;
     }
     const uint32_t row0 = tm * G::BM, col0 = tn * G::BN;
-    const uint32_t k0 = slice * kslice, stages = kslice / kBK;
+    // (ANY: the last slice may be shorter, and its last stage ragged)
+    const uint32_t k0 = slice * kslice;
+    const uint32_t klen = ANY ? (k - k0 < kslice ? k - k0 : kslice) : kslice;
+    const uint32_t stages = ANY ? (klen + kBK - 1) / kBK : klen / kBK;
     if (part) y = part + (size_t)slice * m * n;
 
     const __amdgpu_buffer_rsrc_t xr = rsrc(x, m * k * G::XB);
     const __amdgpu_buffer_rsrc_t pr = rsrc(packed, n * (k / 2));
-    const __amdgpu_buffer_rsrc_t sr = rsrc(scales, n * (k / 32));
+    // ANY: whole aligned words from the one that holds the first scale byte on
+    const uint32_t mis = ANY ? (uint32_t)((uintptr_t)scales & 3) : 0u;
+    const __amdgpu_buffer_rsrc_t sr =
+        ANY ? rsrc(scales - mis, (n * (k / 32) + mis + 3) & ~3u) : rsrc(scales, n * (k / 32));
 
     // this lane's global offsets (stage 0) of its loads; LDS slot p = (q NW + wave) 64 + lane
-    uint32_t a_goff[G::A_INSTR], b_goff[G::B_INSTR];
+    uint32_t a_goff[G::A_INSTR], b_goff[G::B_INSTR], s_goff[G::S_INSTR];
+    uint32_t a_col[G::A_INSTR], b_col[G::B_INSTR];  // first element within the stage (ANY)
 #pragma unroll
     for (int q = 0; q < G::A_INSTR; ++q) {
         const uint32_t p = (q * G::NW + wave) * 64 + lane, row = p / G::A_CPR, c = (p % G::A_CPR) ^ (row % 16);
         a_goff[q] = (row0 + row) * k * G::XB + k0 * G::XB + c * 16;
+        a_col[q] = c * 16 / G::XB;
     }
 #pragma unroll
     for (int q = 0; q < G::B_INSTR; ++q) {
         const uint32_t p = (q * G::NW + wave) * 64 + lane, row = p / 4, c = (p % 4) ^ ((row >> 2) & 3);
         b_goff[q] = (col0 + row) * (k / 2) + k0 / 2 + c * 16;
+        b_col[q] = c * 32;
     }
-    const uint32_t s_row = wave * G::S_ROWS + lane;
-    const uint32_t s_goff = (col0 + s_row) * (k / 32) + k0 / 32;
+#pragma unroll
+    for (int q = 0; q < G::S_INSTR; ++q) {
+        const uint32_t p = wave * G::S_WORDS + q * 64 + lane, row = ANY ? p / 2 : p;
+        s_goff[q] = (col0 + row) * (k / 32) + k0 / 32 + mis;
+        if (ANY) s_goff[q] = (s_goff[q] & ~3u) + 4 * (p % 2);
+    }
 
     auto issue = [&](uint32_t st, uint32_t slot) {
         uint8_t* base = lds + slot * G::STAGE;
+        const uint32_t live = klen - st * kBK;  // ANY: columns of the stage before K's end
 #pragma unroll
-        for (int q = 0; q < G::A_INSTR; ++q)
-            load_lds16(xr, (lds_ptr)(base + (q * G::NW + wave) * 1024), a_goff[q] + st * kBK * G::XB);
+        for (int q = 0; q < G::A_INSTR; ++q) {
+            uint32_t off = a_goff[q] + st * kBK * G::XB;
+            if (ANY) off = a_col[q] < live ? off : kPastEnd;
+            load_lds16(xr, (lds_ptr)(base + (q * G::NW + wave) * 1024), off);
+        }
 #pragma unroll
-        for (int q = 0; q < G::B_INSTR; ++q)
-            load_lds16(pr, (lds_ptr)(base + G::A_BYTES + (q * G::NW + wave) * 1024), b_goff[q] + st * (kBK / 2));
-        // the wave's S_ROWS scale words; lanes past them stay inactive, so they
+        for (int q = 0; q < G::B_INSTR; ++q) {
+            uint32_t off = b_goff[q] + st * (kBK / 2);
+            if (ANY) off = b_col[q] < live ? off : kPastEnd;
+            load_lds16(pr, (lds_ptr)(base + G::A_BYTES + (q * G::NW + wave) * 1024), off);
+        }
+        // the wave's scale words; lanes past them stay inactive, so they
         // write nothing into the next wave's words (the instruction still
         // counts once in vmcnt: lane 0 is always active)
-        if (lane < (uint32_t)G::S_ROWS)
-            load_lds4(sr, (lds_ptr)(base + G::A_BYTES + G::B_BYTES + wave * G::S_ROWS * 4), s_goff + st * (kBK / 32));
+#pragma unroll
+        for (int q = 0; q < G::S_INSTR; ++q)
+            if (q * 64 + lane < (uint32_t)G::S_WORDS)
+                load_lds4(sr, (lds_ptr)(base + G::A_BYTES + G::B_BYTES + (wave * G::S_WORDS + q * 64) * 4),
+                          s_goff[q] + st * (kBK / 32));
     };
 
-    f32x16 acc[TM][TN];
+    using Acc = std::conditional_t<ANY, f64x16, f32x16>;
+    Acc acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
 
-    auto compute = [&](uint32_t slot) {
+    uint32_t s_shift[TN];  // ANY: bits before row j's first scale byte in its two words
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+        s_shift[j] = 8 * (((col0 + (wn * TN + j) * 32 + r32) * (k / 32) + k0 / 32 + mis) & 3);
+    auto compute = [&](uint32_t st, uint32_t slot) {
         const uint8_t* base = lds + slot * G::STAGE;
+        // ANY: blocks past K keep scale byte 0 (what follows the row in memory is no scale of theirs)
+        const uint32_t live = klen - st * kBK;
+        const uint32_t s_mask = ANY && live < (uint32_t)kBK ? (1u << (live / 4)) - 1 : ~0u;
         u32x4 wq[TN][2];
         uint32_t sw[TN];
 #pragma unroll
@@ -204,8 +246,32 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_exact_kernel(const uint8_t*
             const uint8_t* bp = base + G::A_BYTES + r * 64;
             wq[j][0] = *reinterpret_cast<const u32x4*>(bp + ((2 * h) ^ f) * 16);
             wq[j][1] = *reinterpret_cast<const u32x4*>(bp + ((2 * h + 1) ^ f) * 16);
-            sw[j] = *reinterpret_cast<const uint32_t*>(base + G::A_BYTES + G::B_BYTES + r * 4);
+            if constexpr (ANY) {
+                const uint2 two = *reinterpret_cast<const uint2*>(base + G::A_BYTES + G::B_BYTES + r * 8);
+                sw[j] = __builtin_amdgcn_alignbit(two.y, two.x, s_shift[j]) & s_mask;
+            } else {
+                sw[j] = *reinterpret_cast<const uint32_t*>(base + G::A_BYTES + G::B_BYTES + r * 4);
+            }
         }
+        // ANY: a stage is summed from zero and the stages are summed in 64
+        // bits. The kernel that ran these widths before summed K / 64 products
+        // per lane and the lanes in a tree; one MFMA chain over all of K is
+        // 1.2 to 2.5 times as far from the exact sum as that (K = 1600, bf16 /
+        // f32 x: 1.5e-7 / 3.9e-7 against 6e-8 / 1.6e-7 relative), stages added
+        // in 32 bits up to 1.7 times, in 64 bits no further. (The chains of
+        // the other instances are what those widths always had.)
+        f32x16 sum[ANY ? TM : 1][ANY ? TN : 1];
+        auto mac = [&](int s, int i, int j, bf16x8 a, bf16x8 w, bool first) {
+            if constexpr (ANY) {
+                f32x16 c;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) c[r] = 0.0f;
+                if (!(s == 0 && first)) c = sum[i][j];
+                sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, w, c, 0, 0, 0);
+            } else {
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, w, acc[i][j], 0, 0, 0);
+            }
+        };
 #pragma unroll
         for (int s = 0; s < 8; ++s) {
             bf16x8 b[TN];
@@ -223,8 +289,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_exact_kernel(const uint8_t*
                     const uint32_t c = (8 * h + s) ^ sw16;
                     const bf16x8 a = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(ap + c * 16));
 #pragma unroll
-                    for (int j = 0; j < TN; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b[j], acc[i][j], 0, 0, 0);
+                    for (int j = 0; j < TN; ++j) mac(s, i, j, a, b[j], true);
                 } else {
                     const uint32_t c0 = (16 * h + 2 * s) ^ sw16, c1 = (16 * h + 2 * s + 1) ^ sw16;
                     const f32x4 v0 = __builtin_bit_cast(f32x4, *reinterpret_cast<const u32x4*>(ap + c0 * 16));
@@ -233,12 +298,21 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_exact_kernel(const uint8_t*
                     split3x8(v0, v1, hi, mid, lo);
 #pragma unroll
                     for (int j = 0; j < TN; ++j) {
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(hi, b[j], acc[i][j], 0, 0, 0);
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(mid, b[j], acc[i][j], 0, 0, 0);
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lo, b[j], acc[i][j], 0, 0, 0);
+                        mac(s, i, j, hi, b[j], true);
+                        mac(s, i, j, mid, b[j], false);
+                        mac(s, i, j, lo, b[j], false);
                     }
                 }
             }
+        }
+        if constexpr (ANY) {
+            mfma_drain();
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[i][j][r] += (double)sum[i][j][r];
         }
     };
 
@@ -255,7 +329,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_exact_kernel(const uint8_t*
         else wait_vm<0>();
         lds_barrier();
         if (st + D - 1 < stages) issue(st + D - 1, (st + D - 1) % D);
-        compute(st % D);
+        compute(st, st % D);
     }
     mfma_drain();
 
@@ -270,9 +344,22 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_exact_kernel(const uint8_t*
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const uint32_t row = row0 + (wm * TM + i) * 32 + 8 * (r / 4) + 4 * h + r % 4;
-                if (row < m) y[(size_t)row * n + col] = acc[i][j][r];
+                if (row < m) y[(size_t)row * n + col] = (float)acc[i][j][r];
             }
         }
+}
+
+// K of one of ks slices: whole stages, the last slice taking what is left.
+uint32_t slice_k(uint32_t k, uint32_t ks) {
+    const uint32_t stages = (k + kBK - 1) / kBK;
+    return (stages + ks - 1) / ks * kBK;
+}
+
+// Can K be cut into ks slices that the kernel takes: equal ones of whole
+// stages, or (K no whole number of stages) none of them empty.
+bool slices_fit(uint32_t k, uint32_t ks) {
+    if (k % kBK == 0) return k % (ks * kBK) == 0;
+    return (uint64_t)(ks - 1) * slice_k(k, ks) < k;
 }
 
 // y = sum over the slices of part[s] (count floats each), in slice order.
@@ -292,13 +379,13 @@ __global__ __launch_bounds__(256) void split_sum_kernel(const float* __restrict_
     }
 }
 
-template <bool XBF16, int WM, int WN, int TM, int TN>
+template <bool XBF16, int WM, int WN, int TM, int TN, bool ANY>
 hipError_t go(const GemvArgs& a, uint32_t ks, float* part) {
     // deepest ring that fits: 3 stages of a 128 x 128 bf16 tile (121.5 KiB)
-    constexpr int D3 = Geometry<XBF16, WM, WN, TM, TN, 2>::STAGE * 3 <= 160 * 1024 ? 3 : 2;
-    constexpr int D = (Geometry<XBF16, WM, WN, TM, TN, 2>::STAGE * 4 <= 160 * 1024 &&
-                       2 * Geometry<XBF16, WM, WN, TM, TN, 2>::LPS <= 63) ? 4 : D3;
-    using G = Geometry<XBF16, WM, WN, TM, TN, D>;
+    using G2 = Geometry<XBF16, WM, WN, TM, TN, 2, ANY>;
+    constexpr int D3 = G2::STAGE * 3 <= 160 * 1024 ? 3 : 2;
+    constexpr int D = (G2::STAGE * 4 <= 160 * 1024 && 2 * G2::LPS <= 63) ? 4 : D3;
+    using G = Geometry<XBF16, WM, WN, TM, TN, D, ANY>;
     const uint32_t tiles_m = (a.m + G::BM - 1) / G::BM;
     if (a.group) {
         // each weight of the group a run of column tiles; no K split
@@ -315,16 +402,16 @@ hipError_t go(const GemvArgs& a, uint32_t ks, float* part) {
             tiles_n += (sg.n[s] + G::BN - 1) / G::BN;
         }
         const uint32_t tiles = tiles_n * tiles_m;
-        hipLaunchKernelGGL((gemm_exact_kernel<XBF16, WM, WN, TM, TN, D, GemmSegs>), dim3(tiles), dim3(G::NT), 0,
+        hipLaunchKernelGGL((gemm_exact_kernel<XBF16, WM, WN, TM, TN, D, ANY, GemmSegs>), dim3(tiles), dim3(G::NT), 0,
                            a.stream, nullptr, nullptr, a.x, nullptr, a.m, 0u, a.k, tiles_n, tiles, a.k, nullptr, sg);
         return hipGetLastError();
     }
     const uint32_t tiles_n = (a.n + G::BN - 1) / G::BN;
     const uint32_t tiles = tiles_n * tiles_m;
     if (ks < 1) ks = 1;
-    hipLaunchKernelGGL((gemm_exact_kernel<XBF16, WM, WN, TM, TN, D>), dim3(tiles * ks), dim3(G::NT), 0, a.stream,
-                       a.packed, a.scales, a.x, a.y, a.m, a.n, a.k, tiles_n, tiles, a.k / ks, ks > 1 ? part : nullptr,
-                       NoGemmSegs{});
+    hipLaunchKernelGGL((gemm_exact_kernel<XBF16, WM, WN, TM, TN, D, ANY>), dim3(tiles * ks), dim3(G::NT), 0, a.stream,
+                       a.packed, a.scales, a.x, a.y, a.m, a.n, a.k, tiles_n, tiles, slice_k(a.k, ks),
+                       ks > 1 ? part : nullptr, NoGemmSegs{});
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || ks == 1) return e;
     const uint32_t count = a.m * a.n, threads = count % 4 == 0 ? count / 4 : count;
@@ -332,25 +419,33 @@ hipError_t go(const GemvArgs& a, uint32_t ks, float* part) {
     return hipGetLastError();
 }
 
+// the instances that the shape rule picks from, for widths of whole stages and for any
+template <bool XBF16, bool ANY>
+hipError_t dispatch_rule(const GemvArgs& a, const GemmConfig& c, uint32_t ks, float* part) {
+    if (c.wm == 2 && c.wn == 2 && c.tm == 2 && c.tn == 3) return go<XBF16, 2, 2, 2, 3, ANY>(a, ks, part);
+    if (c.wm == 2 && c.wn == 2 && c.tm == 2 && c.tn == 2) return go<XBF16, 2, 2, 2, 2, ANY>(a, ks, part);
+    if (c.wm == 2 && c.wn == 2 && c.tm == 1 && c.tn == 1) return go<XBF16, 2, 2, 1, 1, ANY>(a, ks, part);
+    if (c.wm == 1 && c.wn == 4 && c.tm == 2 && c.tn == 2) return go<XBF16, 1, 4, 2, 2, ANY>(a, ks, part);
+    if (c.wm == 1 && c.wn == 4 && c.tm == 2 && c.tn == 1) return go<XBF16, 1, 4, 2, 1, ANY>(a, ks, part);
+    // a 128 x 256 tile of f32 activations would leave room for one stage only,
+    // and 64-bit sums do not fit the registers of its eight waves
+    if constexpr (XBF16 && !ANY)
+        if (c.wm == 2 && c.wn == 4 && c.tm == 2 && c.tn == 2) return go<XBF16, 2, 4, 2, 2, ANY>(a, ks, part);
+    return hipErrorNotSupported;
+}
+
 template <bool XBF16>
 hipError_t dispatch(const GemvArgs& a, const GemmConfig& c, float* part) {
     // instances: (waves along M x along N, MFMA tiles per wave along M x N)
     const uint32_t ks = c.ks < 1 ? 1u : (uint32_t)c.ks;
-    if (c.wm == 2 && c.wn == 2 && c.tm == 2 && c.tn == 3) return go<XBF16, 2, 2, 2, 3>(a, ks, part);
-    if (c.wm == 2 && c.wn == 2 && c.tm == 2 && c.tn == 2) return go<XBF16, 2, 2, 2, 2>(a, ks, part);
-    if (c.wm == 2 && c.wn == 2 && c.tm == 2 && c.tn == 1) return go<XBF16, 2, 2, 2, 1>(a, ks, part);
-    if (c.wm == 2 && c.wn == 2 && c.tm == 1 && c.tn == 2) return go<XBF16, 2, 2, 1, 2>(a, ks, part);
-    if (c.wm == 4 && c.wn == 1 && c.tm == 1 && c.tn == 2) return go<XBF16, 4, 1, 1, 2>(a, ks, part);
-    if (c.wm == 2 && c.wn == 2 && c.tm == 1 && c.tn == 1) return go<XBF16, 2, 2, 1, 1>(a, ks, part);
-    if (c.wm == 1 && c.wn == 4 && c.tm == 2 && c.tn == 2) return go<XBF16, 1, 4, 2, 2>(a, ks, part);
-    if (c.wm == 1 && c.wn == 4 && c.tm == 2 && c.tn == 1) return go<XBF16, 1, 4, 2, 1>(a, ks, part);
-    if (c.wm == 1 && c.wn == 4 && c.tm == 1 && c.tn == 2) return go<XBF16, 1, 4, 1, 2>(a, ks, part);
-    if (c.wm == 1 && c.wn == 4 && c.tm == 1 && c.tn == 1) return go<XBF16, 1, 4, 1, 1>(a, ks, part);
-    // a 128 x 256 tile of f32 activations would leave room for one stage only
-    if constexpr (XBF16)
-        if (c.wm == 2 && c.wn == 4 && c.tm == 2 && c.tn == 2) return go<XBF16, 2, 4, 2, 2>(a, ks, part);
-    if (c.wm == 2 && c.wn == 4 && c.tm == 1 && c.tn == 2) return go<XBF16, 2, 4, 1, 2>(a, ks, part);
-    return hipErrorNotSupported;
+    if (a.k % kBK != 0) return dispatch_rule<XBF16, true>(a, c, ks, part);
+    if (c.wm == 2 && c.wn == 2 && c.tm == 2 && c.tn == 1) return go<XBF16, 2, 2, 2, 1, false>(a, ks, part);
+    if (c.wm == 2 && c.wn == 2 && c.tm == 1 && c.tn == 2) return go<XBF16, 2, 2, 1, 2, false>(a, ks, part);
+    if (c.wm == 4 && c.wn == 1 && c.tm == 1 && c.tn == 2) return go<XBF16, 4, 1, 1, 2, false>(a, ks, part);
+    if (c.wm == 1 && c.wn == 4 && c.tm == 1 && c.tn == 2) return go<XBF16, 1, 4, 1, 2, false>(a, ks, part);
+    if (c.wm == 1 && c.wn == 4 && c.tm == 1 && c.tn == 1) return go<XBF16, 1, 4, 1, 1, false>(a, ks, part);
+    if (c.wm == 2 && c.wn == 4 && c.tm == 1 && c.tn == 2) return go<XBF16, 2, 4, 1, 2, false>(a, ks, part);
+    return dispatch_rule<XBF16, false>(a, c, ks, part);
 }
 
 }  // namespace
@@ -359,6 +454,13 @@ bool gemm_exact_supported(uint32_t m, uint32_t n, uint32_t k, bool x_bf16) {
     // 32-bit buffer offsets over x and the packed weights
     const uint64_t xb = (uint64_t)m * k * (x_bf16 ? 2 : 4);
     return m >= 1 && n >= 1 && k % kBK == 0 && k >= kBK && xb + 256 * k * 4 < (1ull << 31) &&
+           (uint64_t)(n + 256) * (k / 2) < (1ull << 31);
+}
+
+bool gemm_any_supported(uint32_t m, uint32_t n, uint32_t k, bool x_bf16) {
+    if (k % kBK == 0) return gemm_exact_supported(m, n, k, x_bf16);
+    const uint64_t xb = (uint64_t)m * k * (x_bf16 ? 2 : 4);
+    return m >= 1 && n >= 1 && k % 32 == 0 && k >= 32 && xb + 256 * k * 4 < (1ull << 31) &&
            (uint64_t)(n + 256) * (k / 2) < (1ull << 31);
 }
 
@@ -372,8 +474,8 @@ hipError_t launch_gemm_exact(const GemvArgs& a, int cus, const GemmConfig* force
         if (forced && forced->wm) return hipErrorNotSupported;
         if (a.group->count < 1 || a.group->count > 4) return hipErrorNotSupported;
         for (uint32_t s = 0; s < a.group->count; ++s)
-            if (!gemm_exact_supported(a.m, a.group->n[s], a.k, a.x_bf16)) return hipErrorNotSupported;
-    } else if (!gemm_exact_supported(a.m, a.n, a.k, a.x_bf16)) {
+            if (!gemm_any_supported(a.m, a.group->n[s], a.k, a.x_bf16)) return hipErrorNotSupported;
+    } else if (!gemm_any_supported(a.m, a.n, a.k, a.x_bf16)) {
         return hipErrorNotSupported;
     }
     // column tiles of width bn over the weight (or over each weight of a group)
@@ -408,10 +510,12 @@ hipError_t launch_gemm_exact(const GemvArgs& a, int cus, const GemmConfig* force
                               {1, 4, 2, 1, 64, 128, 22.0},  {2, 2, 1, 1, 64, 64, 16.5}};
         const uint64_t nc = (uint64_t)(cus > 0 ? cus : 256);
         const uint64_t want = nc * 3 / 4;
+        // 128 x 256 has an instance for bf16 x and whole stages only
+        auto wide = [&](const Cand& cd) { return cd.bn == 256 && cd.bm == 128 && (!a.x_bf16 || a.k % kBK != 0); };
         const Cand* best = nullptr;
         double best_t = 0.0;
         for (const Cand& cd : cands) {
-            if (!a.x_bf16 && cd.wn == 4 && cd.wm == 2) continue;  // no f32 instance of 128 x 256
+            if (wide(cd)) continue;
             const uint64_t tiles = (uint64_t)((a.m + cd.bm - 1) / cd.bm) * col_tiles(cd.bn);
             const double t = (double)((tiles + nc - 1) / nc) * cd.round_us;
             if (!best || t < best_t) {
@@ -433,10 +537,10 @@ hipError_t launch_gemm_exact(const GemvArgs& a, int cus, const GemmConfig* force
             uint32_t sel_ks = 0;
             uint64_t sel_area = 0, sel_wgs = 0;
             for (const Cand& cd : cands) {
-                if (!a.x_bf16 && cd.wn == 4 && cd.wm == 2) continue;
+                if (wide(cd)) continue;
                 const uint64_t tiles = (uint64_t)((a.m + cd.bm - 1) / cd.bm) * col_tiles(cd.bn);
                 for (uint32_t ks = 1; ks <= 4; ++ks) {
-                    if (a.k % (ks * kBK) != 0) continue;
+                    if (!slices_fit(a.k, ks)) continue;
                     if (ks > 1 && (a.group || !part || (uint64_t)ks * a.m * a.n * 4 > part_bytes)) continue;
                     const uint64_t wgs = tiles * ks, area = (uint64_t)cd.bm * cd.bn;
                     if (wgs > nc || wgs < want) continue;
@@ -467,7 +571,7 @@ hipError_t launch_gemm_exact(const GemvArgs& a, int cus, const GemmConfig* force
         // q|k|v at 64 token rows: 96 tiles)
         if (a.group) return a.x_bf16 ? dispatch<true>(a, c, nullptr) : dispatch<false>(a, c, nullptr);
         for (uint32_t ks = 4; ks >= 2 && tiles < want; --ks) {
-            if (a.k % (ks * kBK) == 0 && part && (uint64_t)ks * a.m * a.n * 4 <= kFewRowsSplitBytes) {
+            if (slices_fit(a.k, ks) && part && (uint64_t)ks * a.m * a.n * 4 <= kFewRowsSplitBytes) {
                 c.ks = (int)ks;
                 break;
             }

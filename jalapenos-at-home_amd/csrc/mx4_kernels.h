@@ -87,6 +87,9 @@ struct GemmConfig {
     int wm = 0, wn = 0, tm = 0, tn = 0, ks = 0;
 };
 bool gemm_exact_supported(uint32_t m, uint32_t n, uint32_t k, bool x_bf16);
+// The same kernel for any K % 32 == 0 (no explicit configuration where K is no
+// multiple of 128).
+bool gemm_any_supported(uint32_t m, uint32_t n, uint32_t k, bool x_bf16);
 hipError_t launch_gemm_exact(const GemvArgs& a, int cus, const GemmConfig* forced, float* part, uint64_t part_bytes);
 
 // bf16 weights [n][k] (engine/src/lib.rs:255, None arm), any m, f32 accumulation.

@@ -344,7 +344,8 @@ mx4_status run_matmul(mx4_context* ctx, const void* x, mx4_dtype xt, uint32_t m,
         return MX4_OK;
     }
     mx4::GemvArgs a{w->packed, w->scales, x, y, m, w->rows, w->cols, xt == MX4_BF16, ctx->stream};
-    if (path == MX4_PATH_AUTO) {
+    const bool chosen = path == MX4_PATH_AUTO;
+    if (chosen) {
         // 2..4 bf16 token rows: the few-token GEMV where it measured faster
         // than the skinny kernel on the Qwen3 1.7B/8B shapes: 2 tokens below
         // vocabulary-sized weights, and 3-4 tokens on 1024-row weights at
@@ -355,8 +356,8 @@ mx4_status run_matmul(mx4_context* ctx, const void* x, mx4_dtype xt, uint32_t m,
             path = MX4_PATH_GEMV;
         else if (m >= 2 && mx4::skinny_supported(m, w->cols) && scales_foldable(w))
             path = MX4_PATH_SKINNY;
-        else if (m > 32 && mx4::gemm_exact_supported(m, w->rows, w->cols, xt == MX4_BF16) && scales_foldable(w))
-            path = MX4_PATH_GEMM;
+        else if (m > 32 && mx4::gemm_any_supported(m, w->rows, w->cols, xt == MX4_BF16) && scales_foldable(w))
+            path = MX4_PATH_GEMM;  // (asked for by name, the path takes K % 128 == 0 only)
         else
             path = MX4_PATH_GENERIC;
     }
@@ -379,7 +380,7 @@ mx4_status run_matmul(mx4_context* ctx, const void* x, mx4_dtype xt, uint32_t m,
             e = mx4::launch_skinny(a, ctx->cus, {ctx->split_part, ctx->split_count, kSplitPartTiles, kSplitCounts});
             break;
         case MX4_PATH_GEMM:
-            if (!mx4::gemm_exact_supported(m, w->rows, w->cols, xt == MX4_BF16))
+            if (!chosen && !mx4::gemm_exact_supported(m, w->rows, w->cols, xt == MX4_BF16))
                 return fail(MX4_ERR_UNSUPPORTED, "GEMM path needs K %% 128 == 0 and operands under 2 GiB");
             if (!scales_foldable(w))
                 return fail(MX4_ERR_UNSUPPORTED, "GEMM path folds scales into bf16; scale bytes outside 2..252 need GENERIC");

@@ -4,7 +4,7 @@ their ranges. Bars as in test_gpu_parity (assert_close)."""
 import numpy as np
 import pytest
 
-from test_gpu_parity import ctx, mx4  # noqa: F401  (fixtures)
+from test_gpu_parity import assert_close, ctx, mx4  # noqa: F401  (ctx, mx4: fixtures)
 
 pytestmark = pytest.mark.gpu
 
@@ -40,3 +40,67 @@ def test_wrapped_scale_range(mx4, ctx, rows, cols, shift):
                 with pytest.raises(mx4.Mx4Error, match="2..252"):
                     ctx.matmul(x, mx4.F32, 64, w, y, mx4.PATH_GEMM)
             w.release()
+
+
+def planted(rng, n, k):
+    """Random codes and scales of an n x k weight (scale bytes 118..129)."""
+    packed = rng.integers(0, 256, (n, k // 2), dtype=np.uint8)
+    scales = rng.integers(118, 130, (n, k // 32), dtype=np.uint8)
+    return packed, scales
+
+
+def wrapped(ctx, packed, scales, shift):
+    """The weight in device memory, its scales `shift` bytes off a word and NaN
+    scale bytes and full codes all around both arrays."""
+    n, k = packed.shape[0], 2 * packed.shape[1]
+    pb = np.full(packed.size + 64, 0xff, np.uint8)
+    pb[:packed.size] = packed.reshape(-1)
+    sb = np.full(scales.size + shift + 64, 0xff, np.uint8)
+    sb[shift:shift + scales.size] = scales.reshape(-1)
+    return ctx.wrap_weight(ctx.to_device(pb), ctx.to_device(sb), n, k, 0, shift)
+
+
+def activations(mx4, ctx, rng, m, k, xt):
+    """(device buffer, f32 values): m rows with NaN rows behind them."""
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    if xt == mx4.BF16:
+        bits = (x.view(np.uint32) >> 16).astype(np.uint16)
+        x = (bits.astype(np.uint32) << 16).view(np.float32)
+        return ctx.to_device(np.concatenate([bits.reshape(-1), np.full(2 * k, 0x7fc0, np.uint16)])), x
+    return ctx.to_device(np.concatenate([x.reshape(-1), np.full(2 * k, np.nan, np.float32)])), x
+
+
+def check_any_width(mx4, ctx, oracle, seed, m, ns, k, shift):
+    """One weight (ns[0]) and the group of all of ns through the default path,
+    bf16 and f32 activations, against the oracle. Scaled: the planted scale
+    bytes make outputs of any size."""
+    rng = np.random.default_rng(seed)
+    stored = [planted(rng, n, k) for n in ns]
+    ws = [wrapped(ctx, p, s, shift) for p, s in stored]
+    for xt in (mx4.BF16, mx4.F32):
+        xb, x = activations(mx4, ctx, rng, m, k, xt)
+        refs = [oracle.matmul(x, p.reshape(-1), s.reshape(-1)) for p, s in stored]
+        what = f"m={m} ns={ns} k={k} shift={shift} xt={xt}"
+        y = ctx.to_device(np.full(m * ns[0] + 64, 7.0, np.float32))
+        ctx.matmul(xb, xt, m, ws[0], y)
+        out = y.download(np.float32)
+        assert np.all(out[m * ns[0]:] == 7.0), f"{what}: written past the output"
+        assert_close(out[:m * ns[0]].reshape(m, ns[0]), refs[0], what, scaled=True)
+        ys = [ctx.to_device(np.full(m * n + 64, 7.0, np.float32)) for n in ns]
+        ctx.matmul_group(xb.ptr, xt, m, ws, [b.ptr for b in ys])
+        for n, b, ref in zip(ns, ys, refs):
+            out = b.download(np.float32)
+            assert np.all(out[m * n:] == 7.0), f"{what}: written past a group's output"
+            assert_close(out[:m * n].reshape(m, n), ref, f"{what} group", scaled=True)
+    for w in ws:
+        w.release()
+
+
+# more than 32 token rows: K below, at and past a 128-element stage and with 1
+# to 3 blocks left in the last one; rows and columns around the 64, 128 and
+# 192-wide tiles; enough stages that the K split's last slice is short
+@pytest.mark.parametrize("m,ns,k,shift", [
+    (33, (1, 65, 31), 32, 0), (64, (64, 192), 96, 1), (65, (129, 3), 160, 2), (77, (320, 64, 64), 416, 3),
+    (129, (50, 257), 352, 0), (40, (193, 33, 7, 64), 1600, 1), (200, (640, 96), 544, 2), (260, (2100,), 288, 3)])
+def test_prompt_any_width(mx4, ctx, oracle, m, ns, k, shift):
+    check_any_width(mx4, ctx, oracle, m + k, m, ns, k, shift)
