@@ -121,7 +121,7 @@ struct GemmSegs {
     uint32_t count;
 };
 
-constexpr uint32_t kPastEnd = 0xffffff00u;  // past every buffer resource: a load there returns zeros
+constexpr uint32_t kPastEnd = 0x80000000u;  // past every buffer resource: a load there returns zeros
 
 template <bool XBF16, int WM, int WN, int TM, int TN, int D, bool ANY = false, class SG = NoGemmSegs>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_exact_kernel(const uint8_t* __restrict__ packed,

@@ -17,7 +17,10 @@
 //  * the next row-set's loads are issued before the current one is reduced
 //    (register double-buffering), keeping R*BPL KiB in flight per wave;
 //  * E2M1 -> bf16/f32 by the hardware converter, bf16 dot2 (or f32 FMA)
-//    accumulation, wave reduction through lane shuffles, cross-wave through LDS.
+//    accumulation, wave reduction through lane shuffles, cross-wave through LDS;
+//  * widths that no team of whole lanes covers (SUB > 0: any K % 32 == 0) run
+//    the same kernel with lanes past the row reading zeros, and rows of at
+//    most 32 or 16 blocks two or four side by side in a wave.
 #include <type_traits>
 #include "mx4_device.h"
 #include "mx4_kernels.h"
@@ -44,6 +47,17 @@ struct LaneX<true, BPL> {
                 p[j][4 * q + 3] = v[3];
             }
         }
+    }
+    // through a buffer resource of x's size: blocks past the row are zeros
+    __device__ __forceinline__ void load_bounded(__amdgpu_buffer_rsrc_t r, uint32_t blk0, uint32_t stride) {
+#pragma unroll
+        for (int j = 0; j < BPL; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, (blk0 + j * stride) * 64 + 16 * q, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) p[j][4 * q + e] = v[e];
+            }
     }
     // the same blocks from a copy of x staged in LDS
     __device__ __forceinline__ void load_lds(const uint8_t* xl, uint32_t blk0, uint32_t stride) {
@@ -80,6 +94,16 @@ struct LaneX<false, BPL> {
                 f[j][4 * q + 3] = v[3];
             }
         }
+    }
+    __device__ __forceinline__ void load_bounded(__amdgpu_buffer_rsrc_t r, uint32_t blk0, uint32_t stride) {
+#pragma unroll
+        for (int j = 0; j < BPL; ++j)
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, (blk0 + j * stride) * 128 + 16 * q, 0, 0);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) f[j][4 * q + e] = __uint_as_float(v[e]);
+            }
     }
     __device__ __forceinline__ void load_lds(const uint8_t* xl, uint32_t blk0, uint32_t stride) {
 #pragma unroll
@@ -174,15 +198,17 @@ __device__ __forceinline__ void swap_stage(float (&v)[R], int& n) {
 
 constexpr int kDppHalfMirror = 0x141, kDppQuadXor1 = 0xB1, kDppQuadXor2 = 0x4E, kDppRowRor8 = 0x128;
 
-template <int R>
+// SUB rows side by side: the sum over each 64 / SUB lanes only (SUB 2 or 4;
+// lane l's row is then reduced_row_of_lane<R>(l) of its part of the wave).
+template <int R, int SUB = 1>
 __device__ __forceinline__ float wave_reduce_rows(float (&v)[R], uint32_t lane) {
     int n = R;
     dpp_stage<kDppHalfMirror, R>(v, n, (lane & 4) != 0);
     dpp_stage<kDppQuadXor1, R>(v, n, (lane & 1) != 0);
     dpp_stage<kDppQuadXor2, R>(v, n, (lane & 2) != 0);
     dpp_stage<kDppRowRor8, R>(v, n, (lane & 8) != 0);
-    swap_stage<16, R>(v, n);
-    swap_stage<32, R>(v, n);
+    if constexpr (SUB < 4) swap_stage<16, R>(v, n);
+    if constexpr (SUB < 2) swap_stage<32, R>(v, n);
     return v[0];
 }
 
@@ -243,12 +269,23 @@ __device__ __forceinline__ Seg pick_seg(const Segs& sg, uint32_t rs) {
 // so the prefetch can be issued unconditionally. (A prefetch under a branch
 // makes the compiler's wait-count merge fall back to waiting for every load,
 // the prefetch included, which serialises streaming and compute.)
-template <bool XBF16, int WG, int BPL, int R>
+//
+// SUB = 0: K is 32 blocks of every lane, exactly. SUB >= 1: any K of at most
+// that many blocks; SUB rows lie side by side in a wave (64 / SUB lanes each),
+// row-set row i SUB + part is load i of part `part`, and lanes past the row's
+// blocks load zeros (codes and scale byte 0, so they add nothing).
+constexpr uint32_t kPastEnd = 0x80000000u;  // past every buffer resource
+template <int SUB>
+constexpr uint32_t kLanes = 64 / (SUB > 1 ? SUB : 1);  // lanes per row of a wave
+template <int R, int SUB>
+constexpr uint32_t kSetRows = R * (SUB > 1 ? SUB : 1);  // rows of a row-set
+
+template <bool XBF16, int WG, int BPL, int R, int SUB = 0>
 __device__ __forceinline__ void load_rowset_in(const Seg& sgm, uint32_t rs, uint32_t rowsets, uint32_t t,
                                                uint32_t row_bytes, uint32_t nblk, RowSet<XBF16, BPL, R>& out) {
     const bool valid = rs < rowsets;
-    const uint32_t row0 = valid ? (rs - sgm.first) * R : 0;
-    uint32_t rows = sgm.n - row0 < (uint32_t)R ? sgm.n - row0 : (uint32_t)R;
+    const uint32_t row0 = valid ? (rs - sgm.first) * kSetRows<R, SUB> : 0;
+    uint32_t rows = sgm.n - row0 < kSetRows<R, SUB> ? sgm.n - row0 : kSetRows<R, SUB>;
     rows = valid ? rows : 0;
     const __amdgpu_buffer_rsrc_t wr = rsrc(sgm.packed + (size_t)row0 * row_bytes, rows * row_bytes);
     const __amdgpu_buffer_rsrc_t sr = rsrc(sgm.scales + (size_t)row0 * nblk, rows * nblk);
@@ -256,9 +293,16 @@ __device__ __forceinline__ void load_rowset_in(const Seg& sgm, uint32_t rs, uint
     for (int i = 0; i < R; ++i) {
 #pragma unroll
         for (int j = 0; j < BPL; ++j) {
-            const uint32_t b = t + j * 64 * WG;
-            out.w[i][j] = __builtin_amdgcn_raw_buffer_load_b128(wr, 16 * b, i * row_bytes, kNonTemporal);
-            out.s[i][j] = __builtin_amdgcn_raw_buffer_load_b8(sr, b, i * nblk, 0);
+            if constexpr (SUB == 0) {
+                const uint32_t b = t + j * 64 * WG;
+                out.w[i][j] = __builtin_amdgcn_raw_buffer_load_b128(wr, 16 * b, i * row_bytes, kNonTemporal);
+                out.s[i][j] = __builtin_amdgcn_raw_buffer_load_b8(sr, b, i * nblk, 0);
+            } else {
+                const uint32_t part = SUB > 1 ? t / kLanes<SUB> : 0, b = (SUB > 1 ? t % kLanes<SUB> : t) + j * 64 * WG;
+                const uint32_t at = b < nblk ? part * nblk + b : kPastEnd / 16;
+                out.w[i][j] = __builtin_amdgcn_raw_buffer_load_b128(wr, 16 * at, i * SUB * row_bytes, kNonTemporal);
+                out.s[i][j] = __builtin_amdgcn_raw_buffer_load_b8(sr, b < nblk ? at : kPastEnd, i * SUB * nblk, 0);
+            }
         }
     }
     // keep the stream ahead of the arithmetic that follows
@@ -281,10 +325,10 @@ struct OneSeg {
 
 __device__ __forceinline__ Seg pick_seg(const OneSeg& o, uint32_t) { return Seg{o.packed, o.scales, o.y, o.n, 0u}; }
 
-template <bool XBF16, int WG, int BPL, int R, class SG>
+template <bool XBF16, int WG, int BPL, int R, int SUB = 0, class SG>
 __device__ __forceinline__ void load_rowset(const SG& sg, uint32_t rs, uint32_t rowsets, uint32_t t,
                                             uint32_t row_bytes, uint32_t nblk, RowSet<XBF16, BPL, R>& out) {
-    load_rowset_in<XBF16, WG, BPL, R>(pick_seg(sg, rs), rs, rowsets, t, row_bytes, nblk, out);
+    load_rowset_in<XBF16, WG, BPL, R, SUB>(pick_seg(sg, rs), rs, rowsets, t, row_bytes, nblk, out);
 }
 
 // Sum over one row's blocks owned by this lane. The E8M0 scale is folded into
@@ -327,7 +371,7 @@ __device__ __forceinline__ float row_dot(const LaneX<XBF16, BPL>& xr, const u32x
     return acc;
 }
 
-template <bool XBF16, int WG, int BPL, int R, bool AM>
+template <bool XBF16, int WG, int BPL, int R, bool AM, int SUB>
 __device__ __forceinline__ void finish_rowset(const Segs& sg, uint32_t rs, const LaneX<XBF16, BPL>& xr,
                                               const RowSet<XBF16, BPL, R>& cur, uint32_t t,
                                               float (*red)[WG][R], uint32_t& parity, uint64_t& best) {
@@ -336,12 +380,13 @@ __device__ __forceinline__ void finish_rowset(const Segs& sg, uint32_t rs, const
 #pragma unroll
     for (int i = 0; i < R; ++i) acc[i] = row_dot<XBF16, BPL>(xr, cur.w[i], cur.s[i]);
     const Seg sgm = pick_seg(sg, rs);
-    const uint32_t row0 = (rs - sgm.first) * R;
+    const uint32_t row0 = (rs - sgm.first) * kSetRows<R, SUB>;
     const uint32_t n = sgm.n;
     float* y = sgm.y;
-    const float total = wave_reduce_rows<R>(acc, lane);
-    const uint32_t myrow = reduced_row_of_lane<R>(lane);
-    const bool writer = row_writer<R>(lane);
+    static_assert(SUB <= 1 || WG == 1, "rows side by side are one wave's");
+    const float total = wave_reduce_rows<R, SUB>(acc, lane);
+    const uint32_t myrow = SUB > 1 ? reduced_row_of_lane<R>(lane) * SUB + lane / kLanes<SUB> : reduced_row_of_lane<R>(lane);
+    const bool writer = row_writer<R>(lane % kLanes<SUB>);
     if constexpr (WG == 1) {
         if (writer && row0 + myrow < n) {
             if constexpr (AM) {
@@ -386,7 +431,7 @@ struct AllEarly {
     __device__ const Segs& operator()(const Segs& early) const { return early; }
 };
 
-template <bool XBF16, int WG, int BPL, int R, bool AM, bool HEAD0 = false, class Late = AllEarly>
+template <bool XBF16, int WG, int BPL, int R, bool AM, int SUB = 0, bool HEAD0 = false, class Late = AllEarly>
 __device__ __forceinline__ void gemv_m1_body(const Segs& early, const void* __restrict__ x, uint32_t k, uint32_t tpw,
                                              uint32_t grid, Late late = {}) {
     constexpr uint32_t T = 64 * WG;  // threads per team
@@ -406,6 +451,8 @@ __device__ __forceinline__ void gemv_m1_body(const Segs& early, const void* __re
     RowSet<XBF16, BPL, R> a, b;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
     const uint32_t xbytes = k * (XBF16 ? 2 : 4);
+    // the shared copy of x: the blocks of every lane, zeros past K
+    const uint32_t xcopy = SUB ? kLanes<SUB> * WG * BPL * (XBF16 ? 64 : 128) : xbytes;
     // K = 64 WG BPL blocks of 32. When several teams share one LDS copy of x,
     // x is fetched first from K = 6144 on (12 KiB of bf16 x per workgroup)
     // and for one-row teams: its direct-to-LDS loads go out before the first
@@ -415,11 +462,11 @@ __device__ __forceinline__ void gemv_m1_body(const Segs& early, const void* __re
     // 3.52 us and k, v 2.54 -> 2.29 us with four one-row teams sharing x).
     // With two-row teams at K = 4096 (gate, gate|up, lm_head) the same order
     // measured 0.05-0.13 us slower, so there x follows the weights.
-    constexpr bool XFIRST = WG * BPL >= 3 || R == 1;
+    constexpr bool XFIRST = WG * BPL >= 3 || R == 1 || SUB > 0;
     if (XFIRST && tpw > 1) {
         const __amdgpu_buffer_rsrc_t xres = rsrc(x, xbytes);
         const uint32_t lane = threadIdx.x % 64, wave0 = threadIdx.x - lane;
-        for (uint32_t c0 = wave0; c0 < xbytes / 16; c0 += tpw * T)
+        for (uint32_t c0 = wave0; c0 < xcopy / 16; c0 += tpw * T)
             load_lds16(xres, (lds_ptr)(smem + 16 * c0), 16 * (c0 + lane));
         __builtin_amdgcn_sched_barrier(0);
     }
@@ -427,7 +474,7 @@ __device__ __forceinline__ void gemv_m1_body(const Segs& early, const void* __re
         asm volatile("" ::"s"(early.packed[0]), "s"(early.scales[0]), "s"(early.n[0]), "s"(x), "s"(k), "s"(rowsets),
                      "s"(tpw));
         __builtin_amdgcn_sched_barrier(0);
-        load_rowset_in<XBF16, WG, BPL, R>(Seg{early.packed[0], early.scales[0], nullptr, early.n[0], 0u}, rs, rowsets,
+        load_rowset_in<XBF16, WG, BPL, R, SUB>(Seg{early.packed[0], early.scales[0], nullptr, early.n[0], 0u}, rs, rowsets,
                                           t, row_bytes, nblk, a);
     } else {
 #pragma unroll
@@ -436,19 +483,21 @@ __device__ __forceinline__ void gemv_m1_body(const Segs& early, const void* __re
                          "s"(early.first[q]));
         asm volatile("" ::"s"(x), "s"(early.count), "s"(k), "s"(tpw));
         __builtin_amdgcn_sched_barrier(0);
-        load_rowset<XBF16, WG, BPL, R>(early, rs, rowsets, t, row_bytes, nblk, a);
+        load_rowset<XBF16, WG, BPL, R, SUB>(early, rs, rowsets, t, row_bytes, nblk, a);
     }
     const Segs sg = late(early);
     LaneX<XBF16, BPL> xr;
     // the host sizes dynamic LDS as (tpw > 1 ? x : nothing) + tpw * 2 * WG * R floats
-    float(*red)[WG][R] = reinterpret_cast<float(*)[WG][R]>(smem + (tpw > 1 ? xbytes : 0)) + 2 * team;
+    float(*red)[WG][R] = reinterpret_cast<float(*)[WG][R]>(smem + (tpw > 1 ? xcopy : 0)) + 2 * team;
+    const uint32_t xt = SUB > 1 ? t % kLanes<SUB> : t;  // the lane's first block
     if (tpw == 1) {
-        xr.load(x, t, T);
+        if constexpr (SUB > 0) xr.load_bounded(rsrc(x, xbytes), xt, T);
+        else xr.load(x, t, T);
     } else if constexpr (XFIRST) {
         // x's loads were issued before the first row-set's 2 R BPL loads
         wait_vm<2 * R * BPL>();
         __syncthreads();
-        xr.load_lds(smem, t, T);
+        xr.load_lds(smem, xt, T);
     } else {
         const uint8_t* xg = static_cast<const uint8_t*>(x);
         for (uint32_t c = threadIdx.x; c < xbytes / 16; c += tpw * T)
@@ -465,14 +514,14 @@ __device__ __forceinline__ void gemv_m1_body(const Segs& early, const void* __re
     // loads zeros and writes nothing.
     for (uint32_t rf = first;;) {
         uint32_t nxt = rs + stride;
-        load_rowset<XBF16, WG, BPL, R>(sg, nxt, rowsets, t, row_bytes, nblk, b);
-        finish_rowset<XBF16, WG, BPL, R, AM>(sg, rs, xr, a, t, red, parity, best);
+        load_rowset<XBF16, WG, BPL, R, SUB>(sg, nxt, rowsets, t, row_bytes, nblk, b);
+        finish_rowset<XBF16, WG, BPL, R, AM, SUB>(sg, rs, xr, a, t, red, parity, best);
         rf += stride;
         if (rf >= rowsets) break;
         rs = nxt;
         nxt = rs + stride;
-        load_rowset<XBF16, WG, BPL, R>(sg, nxt, rowsets, t, row_bytes, nblk, a);
-        finish_rowset<XBF16, WG, BPL, R, AM>(sg, rs, xr, b, t, red, parity, best);
+        load_rowset<XBF16, WG, BPL, R, SUB>(sg, nxt, rowsets, t, row_bytes, nblk, a);
+        finish_rowset<XBF16, WG, BPL, R, AM, SUB>(sg, rs, xr, b, t, red, parity, best);
         rf += stride;
         if (rf >= rowsets) break;
         rs = nxt;
@@ -502,10 +551,10 @@ __device__ __forceinline__ void gemv_m1_body(const Segs& early, const void* __re
 // first weight load.
 //
 // A group of up to four weights (their table passed by value).
-template <bool XBF16, int WG, int BPL, int R, bool AM>
+template <bool XBF16, int WG, int BPL, int R, bool AM, int SUB = 0>
 __global__ __launch_bounds__(512) void gemv_m1_kernel(Segs sg, const void* __restrict__ x, uint32_t k, uint32_t tpw,
                                                       uint32_t grid) {
-    gemv_m1_body<XBF16, WG, BPL, R, AM>(sg, x, k, tpw, grid);
+    gemv_m1_body<XBF16, WG, BPL, R, AM, SUB>(sg, x, k, tpw, grid);
 }
 
 // A group whose teams all start in segment 0: what the first load needs --
@@ -555,7 +604,7 @@ struct HeadTail {
     }
 };
 
-template <bool XBF16, int WG, int BPL, int R>
+template <bool XBF16, int WG, int BPL, int R, int SUB = 0>
 __global__ __launch_bounds__(512) void gemv_m1_head_kernel(const uint8_t* __restrict__ packed0,
                                                            const uint8_t* __restrict__ scales0,
                                                            const void* __restrict__ x, uint32_t n0, uint32_t k,
@@ -566,7 +615,7 @@ __global__ __launch_bounds__(512) void gemv_m1_head_kernel(const uint8_t* __rest
     early.scales[0] = scales0;
     early.n[0] = n0;
     early.rowsets = rowsets;
-    gemv_m1_body<XBF16, WG, BPL, R, false, true>(early, x, k, tpw, grid, HeadTail{});
+    gemv_m1_body<XBF16, WG, BPL, R, false, SUB, true>(early, x, k, tpw, grid, HeadTail{});
 }
 
 // One weight, every argument a plain scalar: this file is built with kernel
@@ -574,7 +623,7 @@ __global__ __launch_bounds__(512) void gemv_m1_head_kernel(const uint8_t* __rest
 // in SGPRs and the first weight load issues without a memory round trip (a
 // by-value table cannot be preloaded; y and am_partial, needed only at the
 // first store, come last and may be fetched).
-template <bool XBF16, int WG, int BPL, int R, bool AM>
+template <bool XBF16, int WG, int BPL, int R, bool AM, int SUB = 0>
 __global__ __launch_bounds__(512) void gemv_m1_one_kernel(const uint8_t* __restrict__ packed,
                                                           const uint8_t* __restrict__ scales,
                                                           const void* __restrict__ x, uint32_t n, uint32_t k,
@@ -593,7 +642,7 @@ __global__ __launch_bounds__(512) void gemv_m1_one_kernel(const uint8_t* __restr
     sg.count = 1;
     sg.rowsets = rowsets;
     sg.am_partial = am_partial;
-    gemv_m1_body<XBF16, WG, BPL, R, AM>(sg, x, k, tpw, grid);
+    gemv_m1_body<XBF16, WG, BPL, R, AM, SUB>(sg, x, k, tpw, grid);
 }
 
 // A few tokens (speculative verify, 2 <= m <= MT, bf16 activations): the
@@ -818,18 +867,24 @@ __global__ __launch_bounds__(256) void gemv_generic_kernel(const uint8_t* __rest
 
 // ------------------------------------------------------------------ launchers
 
-template <bool XBF16, int WG, int BPL, int R>
+// Bytes of a workgroup's shared copy of x.
+template <bool XBF16, int WG, int BPL, int SUB>
+static size_t x_copy_bytes(uint32_t k) {
+    return SUB ? (size_t)kLanes<SUB> * WG * BPL * (XBF16 ? 64 : 128) : (size_t)k * (XBF16 ? 2 : 4);
+}
+
+template <bool XBF16, int WG, int BPL, int R, int SUB = 0>
 static hipError_t go_m1(const Segs& sg, const void* x, uint32_t k, uint32_t grid, int tpw, hipStream_t st) {
-    const size_t lds = (tpw > 1 ? (size_t)k * (XBF16 ? 2 : 4) : 0) + (size_t)tpw * 2 * WG * R * sizeof(float);
+    const size_t lds = (tpw > 1 ? x_copy_bytes<XBF16, WG, BPL, SUB>(k) : 0) + (size_t)tpw * 2 * WG * R * sizeof(float);
     if (sg.count == 1)
-        hipLaunchKernelGGL((gemv_m1_one_kernel<XBF16, WG, BPL, R, false>), dim3(grid), dim3(64 * WG * tpw), lds, st,
+        hipLaunchKernelGGL((gemv_m1_one_kernel<XBF16, WG, BPL, R, false, SUB>), dim3(grid), dim3(64 * WG * tpw), lds, st,
                            sg.packed[0], sg.scales[0], x, sg.n[0], k, sg.rowsets, (uint32_t)tpw, grid, sg.y[0],
                            (uint64_t*)nullptr);
     else if ((uint64_t)grid * tpw <= sg.first[1])
-        hipLaunchKernelGGL((gemv_m1_head_kernel<XBF16, WG, BPL, R>), dim3(grid), dim3(64 * WG * tpw), lds, st,
+        hipLaunchKernelGGL((gemv_m1_head_kernel<XBF16, WG, BPL, R, SUB>), dim3(grid), dim3(64 * WG * tpw), lds, st,
                            sg.packed[0], sg.scales[0], x, sg.n[0], k, sg.rowsets, (uint32_t)tpw, grid, sg);
     else
-        hipLaunchKernelGGL((gemv_m1_kernel<XBF16, WG, BPL, R, false>), dim3(grid), dim3(64 * WG * tpw), lds, st, sg,
+        hipLaunchKernelGGL((gemv_m1_kernel<XBF16, WG, BPL, R, false, SUB>), dim3(grid), dim3(64 * WG * tpw), lds, st, sg,
                            x, k, (uint32_t)tpw, grid);
     return hipGetLastError();
 }
@@ -908,12 +963,76 @@ static void default_m1_config(uint32_t k, uint32_t rows, int cus, M1Config& c) {
     }
 }
 
+// Any other width: the lanes that cover a row, and how many rows a wave holds
+// side by side (0 as the lane count stands for a width of whole lanes).
+static int any_sub(uint32_t nblk) { return nblk <= 16 ? 4 : nblk <= 32 ? 2 : 1; }
+
+bool gemv_any_supported(uint32_t k) { return k >= 32 && k % 32 == 0 && k <= 32 * 64 * 4 * 3; }
+
+// Bound by the launch and the first loads' latency up to a few thousand rows
+// (2.3-2.5 us), by HBM above (100000 x 3072 27 us, 6.0 TB/s); the generic
+// kernel it replaces here took 5 to 12 us and 105 us for 151936 x 1024. From a
+// sweep of rows, teams and grids at K = 480 .. 16384 and 1024 .. 100000 rows on
+// MI355X (cold weights, recorded passes), in teams per CU:
+//  * one block a lane: one-row teams up to 4096 of them, then two rows (16384 x
+//    1600 4.76 -> 4.55 us against one row, 100000 x 1600 16.5 -> 15.9 us
+//    against four);
+//  * two: one row a team up to 8192 (eight teams a workgroup against four: 4096
+//    x 2560 3.73 -> 3.36 us), then two;
+//  * three: one row, eight teams a workgroup, twice the teams on long weights
+//    (4096 / 100000 x 4288 4.52 / 56.6 -> 3.95 / 37.7 us against 1024 teams of
+//    four a workgroup);
+//  * more: as the tuned K = 12288, two- and four-wave teams of one row.
+// f32 x takes four teams a workgroup (twice the bytes of x in its copy: 1024 x
+// 480 2.66 -> 2.36 us, 16384 x 4288 12.6 -> 10.8 us against eight) and two rows
+// a team from 2048 on with two blocks a lane (4096 x 3072 4.47 -> 4.3 us).
+static void default_any_config(uint32_t k, uint32_t rows, bool x_bf16, int cus, M1Config& c) {
+    const uint32_t nblk = k / 32;
+    const uint32_t scale = (uint32_t)(cus > 0 ? cus : 256);
+    const uint32_t sets = rows / (uint32_t)any_sub(nblk);
+    c.wg = nblk <= 192 ? 1 : nblk <= 384 ? 2 : 4;
+    const uint32_t bpl = (nblk + 64 * c.wg - 1) / (64 * c.wg);
+    if (c.wg > 1) {
+        c.r = 1;
+        c.tpw = c.wg > 2 ? 2 : 4;
+        c.grid = (c.wg > 2 ? 2 : 4) * scale;
+    } else if (bpl == 1) {
+        c.r = sets <= 4096 ? 1 : 2;
+        c.tpw = sets <= 4096 && x_bf16 ? 8 : 4;
+        c.grid = (sets <= 4096 ? 8 : 16) * scale;
+    } else if (!x_bf16) {
+        c.r = bpl == 2 && sets > 2048 ? 2 : 1;
+        c.tpw = 4;
+        c.grid = (sets <= 32768 ? 8 : 12) * scale;
+    } else {
+        c.r = bpl == 2 && sets > 8192 ? 2 : 1;
+        c.tpw = sets <= 1024 ? 4 : 8;
+        c.grid = (sets <= 8192 ? 8 : 16) * scale;
+    }
+    // the shared copy of x must fit 64 KiB with the partial sums
+    if ((uint64_t)bpl * c.wg * 64 * (x_bf16 ? 64 : 128) + (uint64_t)c.tpw * 2 * c.wg * c.r * 4 > 65536) c.tpw = 1;
+}
+
+template <bool XBF16>
+static hipError_t go_any(const Segs& sg, const void* x, uint32_t k, uint32_t grid, int sub, int wg, int bpl, int r,
+                         int tpw, hipStream_t st) {
+#define MX4_ANY_CASE(S, W, B, R_) \
+    if (sub == S && wg == W && bpl == B && r == R_) return go_m1<XBF16, W, B, R_, S>(sg, x, k, grid, tpw, st);
+    MX4_ANY_CASE(4, 1, 1, 1) MX4_ANY_CASE(4, 1, 1, 2) MX4_ANY_CASE(2, 1, 1, 1) MX4_ANY_CASE(2, 1, 1, 2)
+    MX4_ANY_CASE(1, 1, 1, 1) MX4_ANY_CASE(1, 1, 1, 2) MX4_ANY_CASE(1, 1, 2, 1) MX4_ANY_CASE(1, 1, 2, 2) MX4_ANY_CASE(1, 1, 3, 1)
+    MX4_ANY_CASE(1, 2, 2, 1) MX4_ANY_CASE(1, 2, 3, 1) MX4_ANY_CASE(1, 4, 2, 1) MX4_ANY_CASE(1, 4, 3, 1)
+#undef MX4_ANY_CASE
+    return hipErrorNotSupported;
+}
+
 hipError_t launch_gemv_m1_group(const GemvGroup& g, int cus, const M1Config* forced) {
-    if (g.count < 1 || g.count > kMaxSegs || !gemv_m1_supported(g.k)) return hipErrorNotSupported;
+    const bool any = !gemv_m1_supported(g.k);
+    if (g.count < 1 || g.count > kMaxSegs || (any && !gemv_any_supported(g.k))) return hipErrorNotSupported;
     uint32_t rows = 0;
     for (uint32_t s = 0; s < g.count; ++s) rows += g.n[s];
     M1Config c;
-    default_m1_config(g.k, rows, cus, c);
+    if (any) default_any_config(g.k, rows, g.x_bf16, cus, c);
+    else default_m1_config(g.k, rows, cus, c);
     if (forced) {
         if (forced->wg) c.wg = forced->wg;
         if (forced->r) c.r = forced->r;
@@ -921,12 +1040,14 @@ hipError_t launch_gemv_m1_group(const GemvGroup& g, int cus, const M1Config* for
         if (forced->wg || forced->r || forced->grid) c.grid = forced->grid;
     }
     const uint32_t nblk = g.k / 32;
-    if (c.wg < 1 || nblk % (64u * c.wg) != 0) return hipErrorNotSupported;
+    if (c.wg < 1 || (!any && nblk % (64u * c.wg) != 0)) return hipErrorNotSupported;
     if (c.tpw < 1 || 64 * c.wg * c.tpw > 512) return hipErrorNotSupported;
-    // x staged in LDS with the partial sums: at most 64 KiB
-    if (c.tpw > 1 && (uint64_t)g.k * (g.x_bf16 ? 2 : 4) + (uint64_t)c.tpw * 2 * c.wg * c.r * 4 > 65536)
+    // x staged in LDS with the partial sums: at most 64 KiB (the rule for any width sees to it)
+    if (!any && c.tpw > 1 && (uint64_t)g.k * (g.x_bf16 ? 2 : 4) + (uint64_t)c.tpw * 2 * c.wg * c.r * 4 > 65536)
         return hipErrorNotSupported;
-    const int bpl = (int)(nblk / (64u * c.wg));
+    const int bpl = (int)((nblk + 64u * c.wg - 1) / (64u * c.wg));
+    const int sub = any ? any_sub(nblk) : 1;
+    const uint32_t set = (uint32_t)(c.r * sub);  // rows per row-set
     Segs sg{};
     sg.count = g.count;
     sg.first[0] = 0;
@@ -935,7 +1056,7 @@ hipError_t launch_gemv_m1_group(const GemvGroup& g, int cus, const M1Config* for
         sg.scales[s] = g.scales[s];
         sg.y[s] = g.y[s];
         sg.n[s] = g.n[s];
-        sg.first[s + 1] = sg.first[s] + (g.n[s] + c.r - 1) / c.r;
+        sg.first[s + 1] = sg.first[s] + (g.n[s] + set - 1) / set;
     }
     for (uint32_t s = g.count; s < (uint32_t)kMaxSegs; ++s) sg.first[s + 1] = sg.first[g.count];
     const uint32_t rowsets = sg.first[g.count];
@@ -946,6 +1067,9 @@ hipError_t launch_gemv_m1_group(const GemvGroup& g, int cus, const M1Config* for
     const uint32_t per = (rowsets + teams - 1) / teams;
     teams = (rowsets + per - 1) / per;
     const uint32_t grid = (teams + c.tpw - 1) / c.tpw;
+    if (any)
+        return g.x_bf16 ? go_any<true>(sg, g.x, g.k, grid, sub, c.wg, bpl, c.r, c.tpw, g.stream)
+                        : go_any<false>(sg, g.x, g.k, grid, sub, c.wg, bpl, c.r, c.tpw, g.stream);
     return g.x_bf16 ? go_cfg<true>(sg, g.x, g.k, grid, c.wg, bpl, c.r, c.tpw, g.stream)
                     : go_cfg<false>(sg, g.x, g.k, grid, c.wg, bpl, c.r, c.tpw, g.stream);
 }
@@ -959,10 +1083,10 @@ hipError_t launch_gemv_m1_group(const GemvGroup& g, int cus, const M1Config* for
 // for bit; other shapes fall back to the one-wave vocabulary configuration,
 // and where that does not fit either the caller gets hipErrorNotSupported and
 // runs the projection and argmax_rows.
-template <bool XBF16, int WG, int BPL, int R>
+template <bool XBF16, int WG, int BPL, int R, int SUB = 0>
 static hipError_t go_am(const Segs& sg, const void* x, uint32_t k, uint32_t grid, int tpw, uint32_t* idx, hipStream_t st) {
-    const size_t lds = (tpw > 1 ? (size_t)k * (XBF16 ? 2 : 4) : 0) + (size_t)tpw * 2 * WG * R * sizeof(float);
-    hipLaunchKernelGGL((gemv_m1_one_kernel<XBF16, WG, BPL, R, true>), dim3(grid), dim3(64 * WG * tpw), lds, st,
+    const size_t lds = (tpw > 1 ? x_copy_bytes<XBF16, WG, BPL, SUB>(k) : 0) + (size_t)tpw * 2 * WG * R * sizeof(float);
+    hipLaunchKernelGGL((gemv_m1_one_kernel<XBF16, WG, BPL, R, true, SUB>), dim3(grid), dim3(64 * WG * tpw), lds, st,
                        sg.packed[0], sg.scales[0], x, sg.n[0], k, sg.rowsets, (uint32_t)tpw, grid, sg.y[0],
                        sg.am_partial);
     hipError_t e = hipGetLastError();
@@ -981,18 +1105,36 @@ static hipError_t go_am_cfg(const Segs& sg, const void* x, uint32_t k, uint32_t 
     return hipErrorNotSupported;
 }
 
+// Widths of no whole lanes: the rows side by side and rows per team that the
+// rule picks for a vocabulary-sized weight.
+template <bool XBF16>
+static hipError_t go_am_any(const Segs& sg, const void* x, uint32_t k, uint32_t grid, int sub, int bpl, int r, int tpw,
+                            uint32_t* idx, hipStream_t st) {
+#define MX4_AM_CASE(S, B, R_) \
+    if (sub == S && bpl == B && r == R_) return go_am<XBF16, 1, B, R_, S>(sg, x, k, grid, tpw, idx, st);
+    MX4_AM_CASE(4, 1, 2) MX4_AM_CASE(2, 1, 2) MX4_AM_CASE(1, 1, 2) MX4_AM_CASE(1, 2, 2) MX4_AM_CASE(1, 3, 1)
+#undef MX4_AM_CASE
+    return hipErrorNotSupported;
+}
+
 static bool am_compiled(int wg, int bpl, int r) {
     return (wg == 1 && (bpl == 1 || bpl == 2) && (r == 2 || r == 4)) || (wg == 2 && bpl == 1 && (r == 2 || r == 4));
 }
 
 hipError_t launch_gemv_m1_argmax(const GemvArgs& a, uint64_t* partial, uint32_t max_partials, uint32_t* idx,
                                  int cus) {
-    if (!gemv_m1_supported(a.k) || a.n == 0) return hipErrorNotSupported;
+    const bool any = !gemv_m1_supported(a.k);
+    if ((any && !gemv_any_supported(a.k)) || a.n == 0) return hipErrorNotSupported;
     M1Config c;
-    default_m1_config(a.k, a.n, cus, c);
+    if (any) default_any_config(a.k, a.n, a.x_bf16, cus, c);
+    else default_m1_config(a.k, a.n, cus, c);
     const uint32_t nblk = a.k / 32;
-    int bpl = (int)(nblk / (64u * c.wg));
-    if (!am_compiled(c.wg, bpl, c.r) || c.tpw * c.wg > 8) {
+    const int sub = any ? any_sub(nblk) : 1;
+    const uint32_t set = (uint32_t)(c.r * sub);
+    int bpl = (int)((nblk + 64u * c.wg - 1) / (64u * c.wg));
+    if (any) {
+        if (c.wg != 1) return hipErrorNotSupported;
+    } else if (!am_compiled(c.wg, bpl, c.r) || c.tpw * c.wg > 8) {
         // the one-wave vocabulary-sized configuration (4 rows, 4 teams per CU, 4 per workgroup)
         c.wg = 1; c.r = 4; c.grid = 4 * (uint32_t)(cus > 0 ? cus : 256); c.tpw = 4;
         bpl = (int)(nblk / 64);
@@ -1004,18 +1146,21 @@ hipError_t launch_gemv_m1_argmax(const GemvArgs& a, uint64_t* partial, uint32_t 
     sg.scales[0] = a.scales;
     sg.y[0] = a.y;
     sg.n[0] = a.n;
-    const uint32_t rowsets = (a.n + c.r - 1) / c.r;
+    const uint32_t rowsets = (a.n + (any ? set : (uint32_t)c.r) - 1) / (any ? set : (uint32_t)c.r);
     for (int q = 1; q <= kMaxSegs; ++q) sg.first[q] = rowsets;
     sg.rowsets = rowsets;
     sg.am_partial = partial;
     const int tpw = c.tpw < 1 ? 1 : c.tpw;
-    if (tpw > 1 && (uint64_t)a.k * (a.x_bf16 ? 2 : 4) + (uint64_t)tpw * 2 * c.wg * c.r * 4 > 65536)
+    if (!any && tpw > 1 && (uint64_t)a.k * (a.x_bf16 ? 2 : 4) + (uint64_t)tpw * 2 * c.wg * c.r * 4 > 65536)
         return hipErrorNotSupported;
     uint32_t teams = c.grid == 0 || c.grid > rowsets ? rowsets : c.grid;
     const uint32_t per = (rowsets + teams - 1) / teams;
     teams = (rowsets + per - 1) / per;
     const uint32_t grid = (teams + tpw - 1) / tpw;
     if (grid > max_partials) return hipErrorNotSupported;
+    if (any)
+        return a.x_bf16 ? go_am_any<true>(sg, a.x, a.k, grid, sub, bpl, c.r, tpw, idx, a.stream)
+                        : go_am_any<false>(sg, a.x, a.k, grid, sub, bpl, c.r, tpw, idx, a.stream);
     return a.x_bf16 ? go_am_cfg<true>(sg, a.x, a.k, grid, c.wg, bpl, c.r, tpw, idx, a.stream)
                     : go_am_cfg<false>(sg, a.x, a.k, grid, c.wg, bpl, c.r, tpw, idx, a.stream);
 }

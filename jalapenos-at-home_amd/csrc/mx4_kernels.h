@@ -24,6 +24,8 @@ struct GemvArgs {
 };
 
 bool gemv_m1_supported(uint32_t k);
+// The same kernels for any other K % 32 == 0 up to 24576 (default launch shape only).
+bool gemv_any_supported(uint32_t k);
 hipError_t launch_gemv_m1(const GemvArgs& a, int cus);
 
 // M == 1 over up to 4 weights of width k sharing one x (q|k|v, gate|up).

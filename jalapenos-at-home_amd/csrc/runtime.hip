@@ -352,7 +352,9 @@ mx4_status run_matmul(mx4_context* ctx, const void* x, mx4_dtype xt, uint32_t m,
         // K >= 4096 (8B k/v)
         const bool tokens = mx4::gemv_mt_supported(m, w->cols, xt == MX4_BF16) &&
                             ((m == 2 && w->rows < 65536) || (w->rows <= 1024 && w->cols >= 4096));
-        if (((m == 1 && mx4::gemv_m1_supported(w->cols)) || tokens) && scales_foldable(w))
+        // (asked for by name, the GEMV path takes its tuned widths only)
+        const bool one = m == 1 && (mx4::gemv_m1_supported(w->cols) || mx4::gemv_any_supported(w->cols));
+        if ((one || tokens) && scales_foldable(w))
             path = MX4_PATH_GEMV;
         else if (m >= 2 && mx4::skinny_supported(m, w->cols) && scales_foldable(w))
             path = MX4_PATH_SKINNY;
@@ -364,7 +366,7 @@ mx4_status run_matmul(mx4_context* ctx, const void* x, mx4_dtype xt, uint32_t m,
     hipError_t e;
     switch (path) {
         case MX4_PATH_GEMV:
-            if (!(m == 1 && mx4::gemv_m1_supported(w->cols)) && !mx4::gemv_mt_supported(m, w->cols, xt == MX4_BF16))
+            if (!chosen && !(m == 1 && mx4::gemv_m1_supported(w->cols)) && !mx4::gemv_mt_supported(m, w->cols, xt == MX4_BF16))
                 return fail(MX4_ERR_UNSUPPORTED,
                             "GEMV path needs m == 1 and K/32 in {64,128,192,256,384}, or 2 <= m <= 4 with bf16 x "
                             "and K in {2048, 4096, 6144, 8192, 12288}");
@@ -797,7 +799,7 @@ mx4_status mx4_matmul_group(mx4_context* ctx, const void* x, mx4_dtype xt, uint3
     DeviceGuard g(ctx->device);
     bool foldable = true;
     for (uint32_t i = 0; i < count; ++i) foldable &= scales_foldable(w[i]);
-    if (m == 1 && mx4::gemv_m1_supported(w[0]->cols) && foldable) {
+    if (m == 1 && (mx4::gemv_m1_supported(w[0]->cols) || mx4::gemv_any_supported(w[0]->cols)) && foldable) {
         mx4::GemvGroup gg{};
         gg.count = count;
         gg.k = w[0]->cols;
@@ -1261,7 +1263,7 @@ mx4_status mx4_matmul_argmax(mx4_context* ctx, const void* x, mx4_dtype xt, cons
     if (y && ((uintptr_t)y & 3) != 0) return fail(MX4_ERR_ARGUMENT, "y must be 4-byte aligned");
     if (need_stored(w) != MX4_OK) return MX4_ERR_UNSUPPORTED;
     DeviceGuard g(ctx->device);
-    if (!w->bf16 && mx4::gemv_m1_supported(w->cols) && scales_foldable(w)) {
+    if (!w->bf16 && (mx4::gemv_m1_supported(w->cols) || mx4::gemv_any_supported(w->cols)) && scales_foldable(w)) {
         mx4::GemvArgs a{w->packed, w->scales, x, y, 1, w->rows, w->cols, xt == MX4_BF16, ctx->stream};
         hipError_t e = mx4::launch_gemv_m1_argmax(a, ctx->am_partial, kArgmaxPartials, idx, ctx->cus);
         if (e == hipSuccess) return MX4_OK;

@@ -104,3 +104,38 @@ def check_any_width(mx4, ctx, oracle, seed, m, ns, k, shift):
     (129, (50, 257), 352, 0), (40, (193, 33, 7, 64), 1600, 1), (200, (640, 96), 544, 2), (260, (2100,), 288, 3)])
 def test_prompt_any_width(mx4, ctx, oracle, m, ns, k, shift):
     check_any_width(mx4, ctx, oracle, m + k, m, ns, k, shift)
+
+
+# one token row: every number of rows side by side (up to 16, 32, more blocks),
+# blocks a lane, waves a team and rows a team, each with its lanes full, one
+# short and one over, K past the shared copy of x, and row counts that leave
+# row-sets ragged
+@pytest.mark.parametrize("ns,k,shift", [
+    ((1, 2, 5), 32, 0), ((70, 33), 512, 1), ((67, 4), 544, 2), ((1030, 6), 1024, 3), ((515, 1), 1056, 0),
+    ((9000, 130), 1600, 1), ((18000, 7), 480, 2), ((70000,), 992, 0), ((40001,), 288, 1), ((300, 20, 20), 2080, 3),
+    ((8200, 9), 3264, 0), ((33, 5), 4064, 0), ((300, 31), 5184, 1), ((65, 3), 6176, 2), ((513, 2), 8960, 0),
+    ((40, 41), 11008, 3), ((21, 8), 13824, 0), ((5, 9), 24576, 1), ((3, 2), 24608, 0)])
+def test_decode_any_width(mx4, ctx, oracle, ns, k, shift):
+    check_any_width(mx4, ctx, oracle, ns[0] + k, 1, ns, k, shift)
+
+
+@pytest.mark.parametrize("n,k", [(20001, 480), (20001, 992), (40003, 1024), (40003, 1600), (20002, 3264), (5000, 5184),
+                                 (100, 96)])
+def test_argmax_any_width(mx4, ctx, oracle, n, k):
+    """The fused lm_head: the logits are the projection's bit for bit, the
+    index the first maximum of them (a tie planted across the vocabulary)."""
+    rng = np.random.default_rng(n + k)
+    packed, scales = planted(rng, n, k)
+    packed[n - 1], scales[n - 1] = packed[7], scales[7]
+    w = wrapped(ctx, packed, scales, 1)
+    for xt in (mx4.BF16, mx4.F32):
+        xb, x = activations(mx4, ctx, rng, 1, k, xt)
+        y, z, idx = ctx.buffer(n * 4), ctx.buffer(n * 4), ctx.buffer(4)
+        ctx.matmul(xb, xt, 1, w, y)
+        ctx.matmul_argmax(xb, xt, w, z, idx)
+        logits = z.download(np.float32)
+        assert np.array_equal(y.download(np.uint32), logits.view(np.uint32)), (n, k, xt)
+        assert idx.download(np.uint32)[0] == int(np.argmax(logits)), (n, k, xt)
+        ctx.matmul_argmax(xb, xt, w, None, idx)
+        assert idx.download(np.uint32)[0] == int(np.argmax(logits)), (n, k, xt)
+    w.release()
