@@ -64,6 +64,37 @@ __device__ __forceinline__ void split3_bf16(float v, __bf16& hi, __bf16& mid, __
     lo = (__bf16)r2;
 }
 
+// The three terms of eight finite values, packed as MFMA operands: 5.5
+// operations a value where split3_bf16 takes twice that (its care for inf and
+// NaN). Those show in `bad`, which becomes NaN (or stays NaN); the caller then
+// splits again with split3_bf16. (A term of a tiny value may be cut at
+// bf16's least subnormal, 2^-133.)
+__device__ __forceinline__ void split3_finite(const u32x4 lo4, const u32x4 hi4, bf16x8& hi, bf16x8& mid, bf16x8& lo,
+                                              float& bad) {
+    uint32_t h[4], m[4], l[4];
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+        uint32_t r[2], d[2];
+        float rest[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            const uint32_t u = p < 2 ? lo4[2 * p + e] : hi4[2 * p + e - 4];
+            const float r1 = __uint_as_float(u) - __uint_as_float(u & 0xFFFF0000u);  // NaN if u is not finite
+            r[e] = __float_as_uint(r1);
+            rest[e] = r1 - __uint_as_float(r[e] & 0xFFFF0000u);
+            d[e] = u;
+        }
+        bad = __builtin_fmaf(rest[0], rest[1], bad);
+        // the upper halves of a pair: element 2 p below element 2 p + 1
+        h[p] = __builtin_amdgcn_perm(d[1], d[0], 0x07060302u);
+        m[p] = __builtin_amdgcn_perm(r[1], r[0], 0x07060302u);
+        l[p] = __builtin_amdgcn_perm(__float_as_uint(rest[1]), __float_as_uint(rest[0]), 0x07060302u);
+    }
+    hi = __builtin_bit_cast(bf16x8, u32x4{h[0], h[1], h[2], h[3]});
+    mid = __builtin_bit_cast(bf16x8, u32x4{m[0], m[1], m[2], m[3]});
+    lo = __builtin_bit_cast(bf16x8, u32x4{l[0], l[1], l[2], l[3]});
+}
+
 __device__ __forceinline__ uint64_t wave_max_u64(uint64_t m) {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {

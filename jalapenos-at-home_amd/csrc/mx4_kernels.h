@@ -79,6 +79,12 @@ struct SkinnyScratch {
 };
 hipError_t launch_skinny(const GemvArgs& a, int cus, const SkinnyScratch& sc);
 
+// The same for any width (MXFP4: K % 32 == 0, scale bytes 2..252; bf16 weights:
+// K % 8 == 0) and 2 <= m <= 32 (skinny_any.hip). bf16: null, or the weights'
+// values (one for each weight of the group; packed and scales are unused).
+bool skinny_any_supported(uint32_t m, uint32_t k, bool fp4);
+hipError_t launch_skinny_any(const GemvArgs& a, const uint16_t* const* bf16, int cus);
+
 // Exact GEMM on bf16 MFMA for more than 32 token rows (gemm.hip): K % 128 == 0,
 // scale bytes 2..252. GemmConfig picks an instance: waves along M x N and 32x32
 // MFMA tiles per wave along M x N (all zero: the default for the shape), and

@@ -345,6 +345,7 @@ mx4_status run_matmul(mx4_context* ctx, const void* x, mx4_dtype xt, uint32_t m,
     }
     mx4::GemvArgs a{w->packed, w->scales, x, y, m, w->rows, w->cols, xt == MX4_BF16, ctx->stream};
     const bool chosen = path == MX4_PATH_AUTO;
+    bool any_skinny = false;
     if (chosen) {
         // 2..4 bf16 token rows: the few-token GEMV where it measured faster
         // than the skinny kernel on the Qwen3 1.7B/8B shapes: 2 tokens below
@@ -358,6 +359,10 @@ mx4_status run_matmul(mx4_context* ctx, const void* x, mx4_dtype xt, uint32_t m,
             path = MX4_PATH_GEMV;
         else if (m >= 2 && mx4::skinny_supported(m, w->cols) && scales_foldable(w))
             path = MX4_PATH_SKINNY;
+        else if (mx4::skinny_any_supported(m, w->cols, true) && scales_foldable(w)) {
+            path = MX4_PATH_SKINNY;  // (asked for by name, the path takes its tuned widths only)
+            any_skinny = true;
+        }
         else if (m > 32 && mx4::gemm_any_supported(m, w->rows, w->cols, xt == MX4_BF16) && scales_foldable(w))
             path = MX4_PATH_GEMM;  // (asked for by name, the path takes K % 128 == 0 only)
         else
@@ -375,6 +380,10 @@ mx4_status run_matmul(mx4_context* ctx, const void* x, mx4_dtype xt, uint32_t m,
             e = m == 1 ? mx4::launch_gemv_m1(a, ctx->cus) : mx4::launch_gemv_mt(a, ctx->cus);
             break;
         case MX4_PATH_SKINNY:
+            if (any_skinny) {
+                e = mx4::launch_skinny_any(a, nullptr, ctx->cus);
+                break;
+            }
             if (!mx4::skinny_supported(m, w->cols))
                 return fail(MX4_ERR_UNSUPPORTED, "skinny path needs 1 <= m <= 32 and K in {2048, 4096, 6144, 8192, 12288}");
             if (!scales_foldable(w))
@@ -829,7 +838,8 @@ mx4_status mx4_matmul_group(mx4_context* ctx, const void* x, mx4_dtype xt, uint3
     const bool tokens = mx4::gemv_mt_supported(m, k, xt == MX4_BF16) &&
                         ((m == 2 && total < 65536) || (total <= 1024 && k >= 4096));
     const bool skinny = !tokens && m >= 2 && mx4::skinny_supported(m, k);
-    if (count > 1 && stored && foldable && (tokens || skinny)) {
+    const bool any_skinny = !tokens && !skinny && mx4::skinny_any_supported(m, k, true);
+    if (count > 1 && stored && foldable && (tokens || skinny || any_skinny)) {
         mx4::GemvGroup gg{};
         gg.count = count;
         gg.k = k;
@@ -845,8 +855,9 @@ mx4_status mx4_matmul_group(mx4_context* ctx, const void* x, mx4_dtype xt, uint3
         mx4::GemvArgs a{w[0]->packed, w[0]->scales, x, y[0], m, w[0]->rows, k, xt == MX4_BF16, ctx->stream};
         a.group = &gg;
         const hipError_t e =
-            tokens ? mx4::launch_gemv_mt(a, ctx->cus)
-                   : mx4::launch_skinny(a, ctx->cus, {ctx->split_part, ctx->split_count, kSplitPartTiles, kSplitCounts});
+            tokens       ? mx4::launch_gemv_mt(a, ctx->cus)
+            : any_skinny ? mx4::launch_skinny_any(a, nullptr, ctx->cus)
+                         : mx4::launch_skinny(a, ctx->cus, {ctx->split_part, ctx->split_count, kSplitPartTiles, kSplitCounts});
         if (e != hipSuccess) return fail(MX4_ERR_DEVICE, "kernel launch failed: %s", hipGetErrorString(e));
         return MX4_OK;
     }

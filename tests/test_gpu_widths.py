@@ -139,3 +139,49 @@ def test_argmax_any_width(mx4, ctx, oracle, n, k):
         ctx.matmul_argmax(xb, xt, w, None, idx)
         assert idx.download(np.uint32)[0] == int(np.argmax(logits)), (n, k, xt)
     w.release()
+
+
+# 2 to 32 token rows: one and two token tiles, chunks of 128 that leave 1 to 3
+# blocks, fewer chunks than waves, one to four chunks a wave, several slices of
+# K, and one, two and four row tiles a workgroup with several sets of them
+@pytest.mark.parametrize("m,ns,k,shift", [
+    (2, (1, 17, 33), 32, 0), (7, (100, 16), 96, 1), (16, (50, 7, 65, 16), 416, 2), (17, (130, 31), 1024, 3),
+    (3, (320, 64), 1600, 0), (32, (65, 40), 1632, 1), (9, (200, 3), 3264, 2), (29, (48, 70), 3104, 3),
+    (5, (33, 50), 4160, 0), (31, (90, 20), 4288, 1), (12, (35, 64), 9216 + 32, 2), (2, (8300, 9), 160, 0),
+    (16, (16500, 40), 224, 1), (20, (33000, 5), 96, 0), (4, (17000,), 1312, 3), (32, (9000, 700), 2304, 2)])
+def test_verify_any_width(mx4, ctx, oracle, m, ns, k, shift):
+    check_any_width(mx4, ctx, oracle, m + ns[0] + k, m, ns, k, shift)
+
+
+@pytest.mark.parametrize("m,k", [(1, 416), (5, 416), (13, 1600), (29, 544), (40, 352)])
+def test_nonfinite_activations_any_width(mx4, ctx, oracle, m, k):
+    """An inf, a NaN or the largest finite value in one token row shows in that
+    row as the reference's loop has it, and nowhere else; f32 and bf16."""
+    rng = np.random.default_rng(m * k)
+    n = 70
+    packed, scales = planted(rng, n, k)
+    scales[:] = np.minimum(scales, 123)  # the largest product stays below 2^128
+    w = wrapped(ctx, packed, scales, 1)
+    for xt in (mx4.BF16, mx4.F32):
+        for value in (np.inf, -np.inf, np.nan, np.float32(3.0e38)):
+            for at in (0, 33, k - 1):
+                x = rng.standard_normal((m, k)).astype(np.float32)
+                x[m // 2, at] = value
+                if xt == mx4.BF16:
+                    bits = (x.view(np.uint32) >> 16).astype(np.uint16)
+                    x = (bits.astype(np.uint32) << 16).view(np.float32)
+                xb = ctx.to_device(bits if xt == mx4.BF16 else x)
+                y = ctx.buffer(m * n * 4)
+                ctx.matmul(xb, xt, m, w, y)
+                out = y.download(np.float32).reshape(m, n)
+                with np.errstate(all="ignore"):
+                    ref = oracle.matmul(x, packed.reshape(-1), scales.reshape(-1))
+                what = f"m={m} k={k} xt={xt} value={value} at={at}"
+                assert np.array_equal(np.isnan(out), np.isnan(ref)), what
+                assert np.array_equal(np.isinf(out), np.isinf(ref)), what
+                ok = np.isfinite(ref)
+                assert np.array_equal(np.sign(out[np.isinf(ref)]), np.sign(ref[np.isinf(ref)])), what
+                for row in range(m):
+                    if ok[row].all():
+                        assert_close(out[row:row + 1], ref[row:row + 1], what, scaled=True)
+    w.release()
