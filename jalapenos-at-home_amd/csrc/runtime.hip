@@ -323,6 +323,10 @@ mx4_status check_matmul_args(mx4_context* ctx, const void* x, mx4_dtype xt, uint
 // never produces more than 252). Other bytes go to the exact generic kernel.
 bool scales_foldable(const mx4_weight* w) { return w->min_scale >= 2 && w->max_scale <= 252; }
 
+// Does the matrix-core form for bf16 weights and a few token rows take this
+// call (rows of whole 16-byte pieces)?
+bool bf16_skinny(const mx4_weight* w, uint32_t m) { return w->bf16 && mx4::skinny_any_supported(m, w->cols, false); }
+
 // Entry points that read the weight's stored row-major layout refuse a weight
 // whose layout was dropped (mx4_weight_drop_stored).
 mx4_status need_stored(const mx4_weight* w) {
@@ -336,10 +340,16 @@ mx4_status run_matmul(mx4_context* ctx, const void* x, mx4_dtype xt, uint32_t m,
                       float* y, mx4_path path) {
     if (need_stored(w) != MX4_OK) return MX4_ERR_UNSUPPORTED;
     if (w->bf16) {
-        // engine/src/lib.rs:255 `None` arm: one exact kernel for every M
+        // engine/src/lib.rs:255 `None` arm
         if (path != MX4_PATH_AUTO && path != MX4_PATH_GENERIC)
             return fail(MX4_ERR_UNSUPPORTED, "bf16 weights run on the generic path only");
-        hipError_t e = mx4::launch_bf16_matmul(w->bf16, x, xt == MX4_BF16, y, m, w->rows, w->cols, ctx->stream);
+        hipError_t e;
+        if (path == MX4_PATH_AUTO && bf16_skinny(w, m)) {
+            mx4::GemvArgs a{nullptr, nullptr, x, y, m, w->rows, w->cols, xt == MX4_BF16, ctx->stream};
+            e = mx4::launch_skinny_any(a, &w->bf16, ctx->cus);
+        } else {
+            e = mx4::launch_bf16_matmul(w->bf16, x, xt == MX4_BF16, y, m, w->rows, w->cols, ctx->stream);
+        }
         if (e != hipSuccess) return fail(MX4_ERR_DEVICE, "kernel launch failed: %s", hipGetErrorString(e));
         return MX4_OK;
     }
@@ -858,6 +868,24 @@ mx4_status mx4_matmul_group(mx4_context* ctx, const void* x, mx4_dtype xt, uint3
             tokens       ? mx4::launch_gemv_mt(a, ctx->cus)
             : any_skinny ? mx4::launch_skinny_any(a, nullptr, ctx->cus)
                          : mx4::launch_skinny(a, ctx->cus, {ctx->split_part, ctx->split_count, kSplitPartTiles, kSplitCounts});
+        if (e != hipSuccess) return fail(MX4_ERR_DEVICE, "kernel launch failed: %s", hipGetErrorString(e));
+        return MX4_OK;
+    }
+    // bf16 weights, 2..32 token rows: one launch over all of them
+    bool bf16_group = count > 1;
+    for (uint32_t i = 0; i < count; ++i) bf16_group &= bf16_skinny(w[i], m);
+    if (bf16_group) {
+        mx4::GemvGroup gg{};
+        const uint16_t* values[4] = {};
+        gg.count = count;
+        for (uint32_t i = 0; i < count; ++i) {
+            values[i] = w[i]->bf16;
+            gg.y[i] = y[i];
+            gg.n[i] = w[i]->rows;
+        }
+        mx4::GemvArgs a{nullptr, nullptr, x, nullptr, m, 0, k, xt == MX4_BF16, ctx->stream};
+        a.group = &gg;
+        const hipError_t e = mx4::launch_skinny_any(a, values, ctx->cus);
         if (e != hipSuccess) return fail(MX4_ERR_DEVICE, "kernel launch failed: %s", hipGetErrorString(e));
         return MX4_OK;
     }

@@ -362,6 +362,28 @@ __global__ __launch_bounds__(64 * TW) void skinny_any_kernel(const void* __restr
             if (at < tiles) {
                 const Pick p = pick(g, at);
                 const uint32_t row = (at - p.first) * 16 + col;
+                if constexpr (!FP4 && !XBF16) {
+                    // An inf weight times a zero mid or lo term is a NaN that
+                    // the reference's product of the whole value is not: what
+                    // came out as NaN is summed again from whole values, by
+                    // the wave, one output after the other.
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        uint64_t todo = __ballot(sum[r] != sum[r] && row < p.n && 16 * j + 4 * gq + r < m);
+                        while (todo) {
+                            const uint32_t l = (uint32_t)__builtin_ctzll(todo);
+                            todo &= todo - 1;
+                            const uint32_t rr = (at - p.first) * 16 + l % 16, tok = tok0 + 16 * j + 4 * (l / 16) + r;
+                            const uint16_t* wr = reinterpret_cast<const uint16_t*>(p.data) + (size_t)rr * k;
+                            const float* xrow = static_cast<const float*>(x) + (size_t)tok * k;
+                            float part = 0.0f;
+                            for (uint32_t e = lane; e < k; e += 64)
+                                part = __builtin_fmaf(xrow[e], bf16_bits_to_f32(wr[e]), part);
+                            part = wave_sum(part);
+                            if (lane == l) sum[r] = (double)part;
+                        }
+                    }
+                }
                 if (row < p.n) {
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
@@ -395,6 +417,9 @@ hipError_t go(const Weights& g, const void* x, uint32_t m, uint32_t k, uint32_t 
 //    token tiles, or with one tile a workgroup): 18432 x 3264 at 7 rows 13.7
 //    with four, 16.2 with two, 18.8 with one; 1600 x 1600 at 7 rows 4.1 (before
 //    20), 8576 x 1600 at 29 rows 9.7;
+//  * bf16 weights (four times the loads): one chunk, and one tile a workgroup
+//    up to four workgroups per CU: 12288 x 2048 at 7 rows 16.0 against 20.9
+//    with two of each; two of each with two token tiles;
 //  * f32 x: one (two spill), the second token tile counted as tiles of their
 //    own: 1600 x 1600 at 7 rows 6.1, 18432 x 3264 at 7 / 29 rows 29 / 59.
 template <bool FP4, bool XBF16, int MT>
@@ -407,15 +432,20 @@ hipError_t go_shape(const Weights& g, const void* x, uint32_t m, uint32_t k, uin
     uint32_t t = tiles * halves <= nc ? 1 : tiles * halves <= 2 * nc ? 2 : 4;
     uint32_t chunks = per_wave >= 3 ? 4u : per_wave;
     if (chunks > (uint32_t)kMost) chunks = (uint32_t)kMost;
-    if (chunks > 2 && (t == 1 || !FP4)) chunks = 2;
-    if (chunks == 4 || (chunks == 2 && (MT == 1 || !FP4))) t = t > 2 ? 2 : t;
+    if (chunks > 2 && t == 1) chunks = 2;
+    if (!FP4 && XBF16) {
+        chunks = MT == 2 && t > 1 ? chunks : 1;
+        t = MT == 1 && tiles <= 4 * nc ? 1 : t > 2 ? 2 : t;
+    }
+    if (chunks == 4 || (chunks == 2 && MT == 1)) t = t > 2 ? 2 : t;
     uint32_t grid = (tiles + t - 1) / t;
     if (t > 1 && grid > (XBF16 ? nc : 2 * nc)) grid = XBF16 ? nc : 2 * nc;
     // the same number of sets for every workgroup
     const uint32_t sets = (tiles + grid * t - 1) / (grid * t);
     grid = (tiles + sets * t - 1) / (sets * t);
 #define MX4_SKINNY_ANY(C, T_)                                            \
-    if constexpr (C <= kMost && (FP4 || C * T_ <= 4) && (C == 1 || T_ <= 2 || MT == 2)) \
+    if constexpr (C <= kMost && (FP4 || !XBF16 || (T_ <= 2 && C == 1) || (T_ == 2 && MT == 2)) && \
+                  (C == 1 || T_ <= 2 || MT == 2))                         \
         if (chunks == C && t == T_) return go<FP4, XBF16, MT, C, T_>(g, x, m, k, tiles, grid, s);
     MX4_SKINNY_ANY(1, 1) MX4_SKINNY_ANY(1, 2) MX4_SKINNY_ANY(1, 4) MX4_SKINNY_ANY(2, 1) MX4_SKINNY_ANY(2, 2)
     MX4_SKINNY_ANY(2, 4) MX4_SKINNY_ANY(4, 2)

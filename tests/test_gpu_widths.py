@@ -4,7 +4,7 @@ their ranges. Bars as in test_gpu_parity (assert_close)."""
 import numpy as np
 import pytest
 
-from test_gpu_parity import assert_close, ctx, mx4  # noqa: F401  (ctx, mx4: fixtures)
+from test_gpu_parity import assert_close, ctx, f32_bits, mx4  # noqa: F401  (ctx, mx4: fixtures)
 
 pytestmark = pytest.mark.gpu
 
@@ -185,3 +185,74 @@ def test_nonfinite_activations_any_width(mx4, ctx, oracle, m, k):
                     if ok[row].all():
                         assert_close(out[row:row + 1], ref[row:row + 1], what, scaled=True)
     w.release()
+
+
+def check_bf16_weights(mx4, ctx, oracle, seed, m, ns, k):
+    """bf16 weights (one, and the group of all of ns) through the default path
+    against the oracle, bf16 and f32 activations."""
+    rng = np.random.default_rng(seed)
+    ws, vals = [], []
+    for n in ns:
+        bits = (rng.standard_normal((n, k)).astype(np.float32).view(np.uint32) >> 16).astype(np.uint16)
+        vals.append(bits)
+        ws.append(ctx.upload_weight_bf16(bits, n, k))
+    for xt in (mx4.BF16, mx4.F32):
+        xb, x = activations(mx4, ctx, rng, m, k, xt)
+        refs = [oracle.matmul_bf16(x, b) for b in vals]
+        what = f"bf16 weights m={m} ns={ns} k={k} xt={xt}"
+        y = ctx.to_device(np.full(m * ns[0] + 64, 7.0, np.float32))
+        ctx.matmul(xb, xt, m, ws[0], y)
+        out = y.download(np.float32)
+        assert np.all(out[m * ns[0]:] == 7.0), f"{what}: written past the output"
+        assert_close(out[:m * ns[0]].reshape(m, ns[0]), refs[0], what, scaled=True)
+        ys = [ctx.to_device(np.full(m * n + 64, 7.0, np.float32)) for n in ns]
+        ctx.matmul_group(xb.ptr, xt, m, ws, [b.ptr for b in ys])
+        for n, b, ref in zip(ns, ys, refs):
+            out = b.download(np.float32)
+            assert np.all(out[m * n:] == 7.0), f"{what}: written past a group's output"
+            assert_close(out[:m * n].reshape(m, n), ref, f"{what} group", scaled=True)
+    for w in ws:
+        w.release()
+
+
+# K of whole 16-byte pieces and not (9, 1604: the element-wise kernel)
+@pytest.mark.parametrize("m,ns,k", [
+    (2, (1, 17), 8), (5, (33, 16), 9), (7, (100, 3), 120), (16, (50, 64, 7), 136), (17, (70, 40), 1024),
+    (32, (65, 2), 1608), (3, (40, 20), 1604), (12, (8200, 5), 264), (29, (17000,), 136), (9, (70, 300), 4104)])
+def test_bf16_verify(mx4, ctx, oracle, m, ns, k):
+    check_bf16_weights(mx4, ctx, oracle, m + k, m, ns, k)
+
+
+@pytest.mark.parametrize("m,k", [(1, 264), (5, 264), (29, 136), (40, 264), (70, 72)])
+def test_bf16_nonfinite(mx4, ctx, oracle, m, k):
+    """inf and NaN weights, and inf, NaN and 3e38 activations, give what the
+    reference's loop gives, f32 and bf16 activations."""
+    rng = np.random.default_rng(m * k)
+    n = 40
+    for value in (np.inf, np.nan, np.float32(3.0e38)):
+        for where in ("weight", "x"):
+            wf = rng.standard_normal((n, k)).astype(np.float32) * 0.1
+            x = rng.standard_normal((m, k)).astype(np.float32)
+            x[:, 8] = 1.0  # a value whose lower bf16 terms are zero
+            if where == "weight":
+                wf[3, 8] = wf[20, k - 1] = value
+            else:
+                x[m // 2, 8] = value
+            wbits = (f32_bits(wf) >> 16).astype(np.uint16) | (np.isnan(wf) * 0x40).astype(np.uint16)
+            xbits = (f32_bits(x) >> 16).astype(np.uint16) | (np.isnan(x) * 0x40).astype(np.uint16)
+            w = ctx.upload_weight_bf16(wbits, n, k)
+            for xt, host, dev in ((mx4.F32, x, ctx.to_device(x)),
+                                  (mx4.BF16, (xbits.astype(np.uint32) << 16).view(np.float32), ctx.to_device(xbits))):
+                y = ctx.buffer(m * n * 4)
+                ctx.matmul(dev, xt, m, w, y)
+                out = y.download(np.float32).reshape(m, n)
+                with np.errstate(all="ignore"):
+                    ref = oracle.matmul_bf16(host, wbits)
+                what = f"m={m} k={k} xt={xt} {where}={value}"
+                assert np.array_equal(np.isnan(out), np.isnan(ref)), what
+                assert np.array_equal(np.isinf(out), np.isinf(ref)), what
+                inf = np.isinf(ref)
+                assert np.array_equal(np.sign(out[inf]), np.sign(ref[inf])), what
+                ok = np.isfinite(ref)
+                assert np.all(np.abs(out[ok].astype(np.float64) - ref[ok]) <= 1e-3 + 1e-5 * np.abs(ref[ok].astype(np.float64))), what
+            w.release()
