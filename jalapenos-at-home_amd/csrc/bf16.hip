@@ -7,6 +7,10 @@
 // is exact (the top half of an f32), so the only difference from the
 // reference's sequential loop is the summation order.
 //
+// One token row (decode): bf16_gemv_kernel streams the weights, up to four
+// matrices that share x in a launch. Two to 32 rows run skinny_any.hip. The
+// rest, and rows that are not whole 16-byte pieces:
+//
 // One wave per weight row, MT tokens per wave: each lane streams 16-byte
 // pieces (8 weights) of the row, fully coalesced, and reuses each piece for the
 // MT activation rows; the wave then reduces with lane shuffles. Rows whose
@@ -93,6 +97,146 @@ __global__ __launch_bounds__(256) void bf16_matmul_kernel(const uint16_t* __rest
     }
 }
 
+// One token row. A wave takes a row at a time, U x 512 elements of it per turn
+// (U loads of 1 KiB), the next turn's loads (of this row or its next one) issued
+// before this turn's products; x lies in LDS once per workgroup, filled by
+// direct-to-LDS loads that are issued first. Bound by HBM: 24576 x 4096 (201 MB)
+// 35.4 us, 5.7 TB/s; 4096 x 12288 20.1 us, 5.0 TB/s. A layer of hidden size 2048
+// ran at 2.4 TB/s with a load waited for at a time and q, k, v and gate, up
+// launched one by one. Two rows a wave measured the same or slower (12288 x 2048
+// 11.1 against 10.5 us), two turns' worth of loads (U = 2) slower past K = 1024.
+struct Bf16Group {
+    const uint16_t* w[4];
+    float* y[4];
+    uint32_t n[4];
+    uint32_t first[5];  // row-sets of each weight; first[count] .. first[4] are all of them
+    uint32_t count;
+};
+
+template <bool XBF16, int U>
+__global__ __launch_bounds__(512) void bf16_gemv_kernel(const void* __restrict__ x, uint32_t k, uint32_t turns,
+                                                        uint32_t rowsets, uint32_t stride, const Bf16Group g) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t xl[];
+    constexpr int R = 1;  // rows a wave
+    constexpr uint32_t XB = XBF16 ? 2 : 4;
+    const uint32_t lane = threadIdx.x % 64;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    {
+        // turns x U x 512 elements, zeros past K
+        const __amdgpu_buffer_rsrc_t xr = rsrc(x, k * XB);
+        const uint32_t bytes = turns * U * 512 * XB;
+        for (uint32_t c = wave * 1024; c < bytes; c += 8 * 1024) load_lds16(xr, (lds_ptr)(xl + c), c + 16 * lane);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    struct Turn {
+        u32x4 w[R][U];
+    };
+    auto pick = [&](uint32_t set, const uint16_t*& w, float*& y, uint32_t& n, uint32_t& row0) {
+        w = g.w[0];
+        y = g.y[0];
+        n = g.n[0];
+        uint32_t first = 0;
+#pragma unroll
+        for (int q = 1; q < 4; ++q) {
+            const bool in = q < (int)g.count && set >= g.first[q];
+            w = in ? g.w[q] : w;
+            y = in ? g.y[q] : y;
+            n = in ? g.n[q] : n;
+            first = in ? g.first[q] : first;
+        }
+        row0 = (set - first) * R;
+    };
+    // a row-set past the end loads zeros without touching memory
+    auto load = [&](uint32_t set, uint32_t turn, Turn& t) {
+        const uint16_t* w;
+        float* y;
+        uint32_t n, row0;
+        pick(set, w, y, n, row0);
+        const bool valid = set < rowsets;
+        row0 = valid ? row0 : 0;
+        const uint32_t rows = valid ? (n - row0 < (uint32_t)R ? n - row0 : (uint32_t)R) : 0;
+        const __amdgpu_buffer_rsrc_t r = rsrc(w + (size_t)row0 * k, rows * k * 2);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t e = (turn * U + u) * 512 + 8 * lane;
+#pragma unroll
+            for (int i = 0; i < R; ++i)
+                t.w[i][u] = __builtin_amdgcn_raw_buffer_load_b128(r, e < k ? 2 * (i * k + e) : 0x80000000u, 0, 2);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    float acc[R];
+    auto consume = [&](uint32_t turn, const Turn& t) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint8_t* xp = xl + ((turn * U + u) * 512 + 8 * lane) * XB;
+            if constexpr (XBF16) {
+                const u32x4 v = *reinterpret_cast<const u32x4*>(xp);
+#pragma unroll
+                for (int i = 0; i < R; ++i)
+#pragma unroll
+                    for (int d = 0; d < 4; ++d)
+                        acc[i] = __builtin_amdgcn_fdot2_f32_bf16(as_bf16x2(t.w[i][u][d]), as_bf16x2(v[d]), acc[i], false);
+            } else {
+                const f32x4 a = *reinterpret_cast<const f32x4*>(xp), b = *reinterpret_cast<const f32x4*>(xp + 16);
+                const float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+#pragma unroll
+                for (int i = 0; i < R; ++i)
+#pragma unroll
+                    for (int d = 0; d < 4; ++d) {
+                        const uint32_t p = t.w[i][u][d];
+                        acc[i] = __builtin_fmaf(v[2 * d], __uint_as_float(p << 16), acc[i]);
+                        acc[i] = __builtin_fmaf(v[2 * d + 1], __uint_as_float(p & 0xffff0000u), acc[i]);
+                    }
+            }
+        }
+    };
+    auto finish = [&](uint32_t set) {
+        const uint16_t* w;
+        float* y;
+        uint32_t n, row0;
+        pick(set, w, y, n, row0);
+        const float total = wave_reduce_rows<R>(acc, lane);
+        const uint32_t row = row0 + reduced_row_of_lane<R>(lane);
+        if (row_writer<R>(lane) && row < n) y[row] = total;
+    };
+    uint32_t set = blockIdx.x * 8 + wave, turn = 0;
+    Turn a, b;
+    load(set, 0, a);
+    wait_vm<R * U>();  // x is in, the weights need not be
+    __syncthreads();
+    if (set >= rowsets) return;
+#pragma unroll
+    for (int i = 0; i < R; ++i) acc[i] = 0.0f;
+    auto step = [&](const Turn& cur, Turn& nxt) -> bool {
+        const bool last = turn + 1 == turns;
+        const uint32_t nset = last ? set + stride : set, nturn = last ? 0 : turn + 1;
+        load(nset, nturn, nxt);
+        consume(turn, cur);
+        if (last) {
+            finish(set);
+#pragma unroll
+            for (int i = 0; i < R; ++i) acc[i] = 0.0f;
+            if (nset >= rowsets) return true;
+        }
+        set = nset;
+        turn = nturn;
+        return false;
+    };
+    for (;;) {
+        if (step(a, b)) break;
+        if (step(b, a)) break;
+    }
+}
+
+template <bool XBF16, int U>
+hipError_t go_gemv(const Bf16Group& g, const void* x, uint32_t k, uint32_t rowsets, uint32_t grid, hipStream_t s) {
+    const uint32_t turns = (k + 512 * U - 1) / (512 * U);
+    hipLaunchKernelGGL((bf16_gemv_kernel<XBF16, U>), dim3(grid), dim3(512), turns * U * 512 * (XBF16 ? 2 : 4), s, x, k,
+                       turns, rowsets, grid * 8, g);
+    return hipGetLastError();
+}
+
 template <bool XBF16, int MT>
 hipError_t go(const uint16_t* w, const void* x, float* y, uint32_t m, uint32_t n, uint32_t k, bool vec,
               hipStream_t s) {
@@ -105,6 +249,38 @@ hipError_t go(const uint16_t* w, const void* x, float* y, uint32_t m, uint32_t n
 }
 
 }  // namespace
+
+bool bf16_gemv_supported(uint32_t k, bool x_bf16) {
+    // rows of whole 16-byte pieces; x (rounded up to whole turns) in 64 KiB of LDS
+    return k >= 8 && k % 8 == 0 && (k + 2047) / 2048 * 2048 * (x_bf16 ? 2 : 4) <= 65536;
+}
+
+hipError_t launch_bf16_gemv(const uint16_t* const* w, float* const* y, const uint32_t* n, uint32_t count, const void* x,
+                            bool x_bf16, uint32_t k, int cus, hipStream_t s) {
+    if (count < 1 || count > 4 || !bf16_gemv_supported(k, x_bf16)) return hipErrorNotSupported;
+    uint32_t rows = 0;
+    for (uint32_t i = 0; i < count; ++i) {
+        if (n[i] == 0) return hipErrorNotSupported;
+        rows += n[i];
+    }
+    const uint32_t nc = (uint32_t)(cus > 0 ? cus : 256);
+    Bf16Group g{};
+    g.count = count;
+    for (uint32_t i = 0; i < count; ++i) {
+        g.w[i] = w[i];
+        g.y[i] = y[i];
+        g.n[i] = n[i];
+        g.first[i + 1] = g.first[i] + n[i];
+    }
+    for (uint32_t i = count; i < 4; ++i) g.first[i + 1] = g.first[count];
+    // four workgroups of eight waves per CU, the same number of rows for every wave
+    uint32_t grid = (rows + 7) / 8;
+    if (grid > 4 * nc) grid = 4 * nc;
+    const uint32_t each = (rows + grid * 8 - 1) / (grid * 8);
+    grid = (rows + each * 8 - 1) / (each * 8);
+    if (k <= 1024) return x_bf16 ? go_gemv<true, 2>(g, x, k, rows, grid, s) : go_gemv<false, 2>(g, x, k, rows, grid, s);
+    return x_bf16 ? go_gemv<true, 4>(g, x, k, rows, grid, s) : go_gemv<false, 4>(g, x, k, rows, grid, s);
+}
 
 hipError_t launch_bf16_matmul(const uint16_t* w, const void* x, bool x_bf16, float* y, uint32_t m, uint32_t n,
                               uint32_t k, hipStream_t s) {

@@ -137,101 +137,6 @@ struct Segs {
     uint64_t* am_partial;  // greedy-argmax epilogue: one key per workgroup (unused otherwise)
 };
 
-// Sum R per-lane values over the 64 lanes of a wave in log2(64) exchange
-// stages. In the first log2(R) stages each lane keeps half of its values and
-// sends the other half to its partner, so the R totals cost 63 + R - 1
-// additions instead of R * 63. The exchanges stay in the VALU: DPP
-// row_half_mirror (partner l ^ 7), quad permutations (l ^ 1, l ^ 2) and
-// row_ror:8 (l ^ 8) within rows of 16 lanes, then v_permlane16_swap (l ^ 16)
-// and v_permlane32_swap (l ^ 32). The half-mirror stage goes first: it flips
-// lane bits 0-2 together, which is a valid butterfly partner only while no
-// earlier stage has made lanes differ in bits 0-1. The halving stages select
-// by lane bits 2, 0, 1 in that order, so lane l ends with the total of row
-// reduced_row_of_lane<R>(l).
-template <int CTRL>
-__device__ __forceinline__ float dpp_partner(float v) {
-    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
-}
-
-template <int CTRL, int R>
-__device__ __forceinline__ void dpp_stage(float (&v)[R], int& n, bool upper) {
-    if (n > 1) {
-        const int half = n / 2;
-#pragma unroll
-        for (int i = 0; i < R / 2; ++i) {
-            if (i < half) {
-                const float send = upper ? v[i] : v[i + half];
-                const float keep = upper ? v[i + half] : v[i];
-                v[i] = keep + dpp_partner<CTRL>(send);
-            }
-        }
-        n = half;
-    } else {
-        v[0] += dpp_partner<CTRL>(v[0]);
-    }
-}
-
-// Exchange across rows (SWAP = 16) or half-waves (SWAP = 32). After
-// permlane*_swap(a, b) lane l holds {own a, partner's a} if it is the lower
-// partner and {partner's b, own b} if it is the upper one, so the sum of the
-// pair is keep + partner's send in both cases.
-template <int SWAP>
-__device__ __forceinline__ float swap_sum(float lower_keeps, float upper_keeps) {
-    const auto p = SWAP == 16
-                       ? __builtin_amdgcn_permlane16_swap(__float_as_uint(lower_keeps), __float_as_uint(upper_keeps), false, false)
-                       : __builtin_amdgcn_permlane32_swap(__float_as_uint(lower_keeps), __float_as_uint(upper_keeps), false, false);
-    return __uint_as_float(p[0]) + __uint_as_float(p[1]);
-}
-
-template <int SWAP, int R>
-__device__ __forceinline__ void swap_stage(float (&v)[R], int& n) {
-    if (n > 1) {
-        const int half = n / 2;
-#pragma unroll
-        for (int i = 0; i < R / 2; ++i)
-            if (i < half) v[i] = swap_sum<SWAP>(v[i], v[i + half]);
-        n = half;
-    } else {
-        v[0] = swap_sum<SWAP>(v[0], v[0]);
-    }
-}
-
-constexpr int kDppHalfMirror = 0x141, kDppQuadXor1 = 0xB1, kDppQuadXor2 = 0x4E, kDppRowRor8 = 0x128;
-
-// SUB rows side by side: the sum over each 64 / SUB lanes only (SUB 2 or 4;
-// lane l's row is then reduced_row_of_lane<R>(l) of its part of the wave).
-template <int R, int SUB = 1>
-__device__ __forceinline__ float wave_reduce_rows(float (&v)[R], uint32_t lane) {
-    int n = R;
-    dpp_stage<kDppHalfMirror, R>(v, n, (lane & 4) != 0);
-    dpp_stage<kDppQuadXor1, R>(v, n, (lane & 1) != 0);
-    dpp_stage<kDppQuadXor2, R>(v, n, (lane & 2) != 0);
-    dpp_stage<kDppRowRor8, R>(v, n, (lane & 8) != 0);
-    if constexpr (SUB < 4) swap_stage<16, R>(v, n);
-    if constexpr (SUB < 2) swap_stage<32, R>(v, n);
-    return v[0];
-}
-
-// Row whose total lane `lane` holds after wave_reduce_rows<R> (R <= 8): the
-// halving stages take the upper half when lane bit 2, then 0, then 1 is set.
-template <int R>
-__device__ __forceinline__ uint32_t reduced_row_of_lane(uint32_t lane) {
-    static_assert(R == 1 || R == 2 || R == 4 || R == 8, "rows per team");
-    uint32_t row = 0;
-    if constexpr (R >= 2) row += (lane & 4) ? R / 2 : 0;
-    if constexpr (R >= 4) row += (lane & 1) ? R / 4 : 0;
-    if constexpr (R >= 8) row += (lane & 2) ? 1 : 0;
-    return row;
-}
-
-// One lane per row writes its total: lane bits outside the row-select bits are zero.
-template <int R>
-__device__ __forceinline__ bool row_writer(uint32_t lane) {
-    constexpr uint32_t row_bits = R >= 8 ? 7u : R == 4 ? 5u : R == 2 ? 4u : 0u;
-    return (lane & ~row_bits) == 0;
-}
-
-
 constexpr int kNonTemporal = 2;  // streamed once per pass: do not keep in the caches
 
 template <bool XBF16, int BPL, int R>

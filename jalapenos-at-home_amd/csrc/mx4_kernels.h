@@ -104,6 +104,12 @@ hipError_t launch_gemm_exact(const GemvArgs& a, int cus, const GemmConfig* force
 hipError_t launch_bf16_matmul(const uint16_t* w, const void* x, bool x_bf16, float* y, uint32_t m, uint32_t n,
                               uint32_t k, hipStream_t s);
 
+// One token row over up to four bf16 weights of width k sharing x (16-byte
+// aligned): k % 8 == 0 and x within the LDS.
+bool bf16_gemv_supported(uint32_t k, bool x_bf16);
+hipError_t launch_bf16_gemv(const uint16_t* const* w, float* const* y, const uint32_t* n, uint32_t count, const void* x,
+                            bool x_bf16, uint32_t k, int cus, hipStream_t s);
+
 // Block-scaled MFMA prefill on requantized activations. Both operands are in
 // the fragment-native layout of prefill.hip (launch_to_fragments, or the
 // quantizers' fragment output).

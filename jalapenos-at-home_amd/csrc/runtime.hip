@@ -344,7 +344,9 @@ mx4_status run_matmul(mx4_context* ctx, const void* x, mx4_dtype xt, uint32_t m,
         if (path != MX4_PATH_AUTO && path != MX4_PATH_GENERIC)
             return fail(MX4_ERR_UNSUPPORTED, "bf16 weights run on the generic path only");
         hipError_t e;
-        if (path == MX4_PATH_AUTO && bf16_skinny(w, m)) {
+        if (path == MX4_PATH_AUTO && m == 1 && mx4::bf16_gemv_supported(w->cols, xt == MX4_BF16)) {
+            e = mx4::launch_bf16_gemv(&w->bf16, &y, &w->rows, 1, x, xt == MX4_BF16, w->cols, ctx->cus, ctx->stream);
+        } else if (path == MX4_PATH_AUTO && bf16_skinny(w, m)) {
             mx4::GemvArgs a{nullptr, nullptr, x, y, m, w->rows, w->cols, xt == MX4_BF16, ctx->stream};
             e = mx4::launch_skinny_any(a, &w->bf16, ctx->cus);
         } else {
@@ -871,9 +873,24 @@ mx4_status mx4_matmul_group(mx4_context* ctx, const void* x, mx4_dtype xt, uint3
         if (e != hipSuccess) return fail(MX4_ERR_DEVICE, "kernel launch failed: %s", hipGetErrorString(e));
         return MX4_OK;
     }
-    // bf16 weights, 2..32 token rows: one launch over all of them
-    bool bf16_group = count > 1;
-    for (uint32_t i = 0; i < count; ++i) bf16_group &= bf16_skinny(w[i], m);
+    // bf16 weights: one launch over all of them
+    bool bf16_group = count > 1, bf16_one = m == 1 && mx4::bf16_gemv_supported(k, xt == MX4_BF16);
+    for (uint32_t i = 0; i < count; ++i) {
+        bf16_one &= w[i]->bf16 != nullptr;
+        bf16_group &= bf16_skinny(w[i], m);
+    }
+    if (bf16_one) {
+        const uint16_t* values[4] = {};
+        uint32_t rows[4] = {};
+        for (uint32_t i = 0; i < count; ++i) {
+            values[i] = w[i]->bf16;
+            rows[i] = w[i]->rows;
+        }
+        const hipError_t e =
+            mx4::launch_bf16_gemv(values, y, rows, count, x, xt == MX4_BF16, k, ctx->cus, ctx->stream);
+        if (e != hipSuccess) return fail(MX4_ERR_DEVICE, "kernel launch failed: %s", hipGetErrorString(e));
+        return MX4_OK;
+    }
     if (bf16_group) {
         mx4::GemvGroup gg{};
         const uint16_t* values[4] = {};

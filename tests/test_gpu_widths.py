@@ -256,3 +256,13 @@ def test_bf16_nonfinite(mx4, ctx, oracle, m, k):
                 ok = np.isfinite(ref)
                 assert np.all(np.abs(out[ok].astype(np.float64) - ref[ok]) <= 1e-3 + 1e-5 * np.abs(ref[ok].astype(np.float64))), what
             w.release()
+
+
+# rows of one and two a wave, K of one turn and several with lanes past its end,
+# K past the LDS copy of x (24576 f32: the row-per-wave kernel) and K of no
+# whole pieces
+@pytest.mark.parametrize("ns,k", [
+    ((1, 3), 8), ((33, 5), 520), ((50, 64, 7), 1024), ((130, 2), 1608), ((70, 9), 2056), ((5000, 1), 264),
+    ((9000, 4000, 3), 136), ((40, 41), 12296), ((20, 3), 20480), ((17, 5), 24576), ((40, 20), 1604)])
+def test_bf16_decode(mx4, ctx, oracle, ns, k):
+    check_bf16_weights(mx4, ctx, oracle, ns[0] + k, 1, ns, k)
