@@ -41,7 +41,7 @@ namespace {
 
 // Three bf16 terms of eight f32 values, hi + mid + lo = x exactly
 // (split3_bf16: non-finite values stay in hi).
-__device__ __forceinline__ void split3x8(const f32x4 a, const f32x4 b, bf16x8& hi, bf16x8& mid, bf16x8& lo) {
+__device__ __forceinline__ void split3_each(const f32x4 a, const f32x4 b, bf16x8& hi, bf16x8& mid, bf16x8& lo) {
     const float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -295,7 +295,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_exact_kernel(const uint8_t*
                     const f32x4 v0 = __builtin_bit_cast(f32x4, *reinterpret_cast<const u32x4*>(ap + c0 * 16));
                     const f32x4 v1 = __builtin_bit_cast(f32x4, *reinterpret_cast<const u32x4*>(ap + c1 * 16));
                     bf16x8 hi, mid, lo;
-                    split3x8(v0, v1, hi, mid, lo);
+                    split3_each(v0, v1, hi, mid, lo);
 #pragma unroll
                     for (int j = 0; j < TN; ++j) {
                         mac(s, i, j, hi, b[j], true);
@@ -414,9 +414,7 @@ hipError_t go(const GemvArgs& a, uint32_t ks, float* part) {
                        ks > 1 ? part : nullptr, NoGemmSegs{});
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || ks == 1) return e;
-    const uint32_t count = a.m * a.n, threads = count % 4 == 0 ? count / 4 : count;
-    hipLaunchKernelGGL(split_sum_kernel, dim3((threads + 255) / 256), dim3(256), 0, a.stream, part, ks, count, a.y);
-    return hipGetLastError();
+    return launch_split_sum(part, ks, a.m * a.n, a.y, a.stream);
 }
 
 // the instances that the shape rule picks from, for widths of whole stages and for any
@@ -449,6 +447,12 @@ hipError_t dispatch(const GemvArgs& a, const GemmConfig& c, float* part) {
 }
 
 }  // namespace
+
+hipError_t launch_split_sum(const float* part, uint32_t ks, uint32_t count, float* y, hipStream_t s) {
+    const uint32_t threads = count % 4 == 0 ? count / 4 : count;
+    hipLaunchKernelGGL(split_sum_kernel, dim3((threads + 255) / 256), dim3(256), 0, s, part, ks, count, y);
+    return hipGetLastError();
+}
 
 bool gemm_exact_supported(uint32_t m, uint32_t n, uint32_t k, bool x_bf16) {
     // 32-bit buffer offsets over x and the packed weights

@@ -95,6 +95,23 @@ __device__ __forceinline__ void split3_finite(const u32x4 lo4, const u32x4 hi4, 
     lo = __builtin_bit_cast(bf16x8, u32x4{l[0], l[1], l[2], l[3]});
 }
 
+// The terms of eight values, finite or not: the wave takes the short form and,
+// where some lane has an inf or a NaN (or the check overflows), the careful one.
+__device__ __forceinline__ void split3x8(const u32x4 a, const u32x4 b, bf16x8& hi, bf16x8& mid, bf16x8& lo) {
+    float bad = 0.0f;
+    split3_finite(a, b, hi, mid, lo, bad);
+    if (__any(bad != bad)) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            __bf16 h, m, l;
+            split3_bf16(__uint_as_float(e < 4 ? a[e] : b[e - 4]), h, m, l);
+            hi[e] = h;
+            mid[e] = m;
+            lo[e] = l;
+        }
+    }
+}
+
 __device__ __forceinline__ uint64_t wave_max_u64(uint64_t m) {
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) {

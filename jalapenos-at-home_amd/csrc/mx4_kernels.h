@@ -110,6 +110,16 @@ bool bf16_gemv_supported(uint32_t k, bool x_bf16);
 hipError_t launch_bf16_gemv(const uint16_t* const* w, float* const* y, const uint32_t* n, uint32_t count, const void* x,
                             bool x_bf16, uint32_t k, int cus, hipStream_t s);
 
+// More than 32 token rows over up to four bf16 weights of width k sharing x
+// (k % 8 == 0, gemm_bf16.hip). A K split (one weight) writes its partials to
+// `part`, scratch shared with the other split launches of the stream.
+bool gemm_bf16_supported(uint32_t m, uint32_t n, uint32_t k, bool x_bf16);
+hipError_t launch_gemm_bf16(const uint16_t* const* w, float* const* y, const uint32_t* n, uint32_t count, const void* x,
+                            bool x_bf16, uint32_t m, uint32_t k, int cus, float* part, uint64_t part_bytes,
+                            hipStream_t s);
+// y = sum over ks slices of part[s] (count floats each), in slice order.
+hipError_t launch_split_sum(const float* part, uint32_t ks, uint32_t count, float* y, hipStream_t s);
+
 // Block-scaled MFMA prefill on requantized activations. Both operands are in
 // the fragment-native layout of prefill.hip (launch_to_fragments, or the
 // quantizers' fragment output).

@@ -346,6 +346,9 @@ mx4_status run_matmul(mx4_context* ctx, const void* x, mx4_dtype xt, uint32_t m,
         hipError_t e;
         if (path == MX4_PATH_AUTO && m == 1 && mx4::bf16_gemv_supported(w->cols, xt == MX4_BF16)) {
             e = mx4::launch_bf16_gemv(&w->bf16, &y, &w->rows, 1, x, xt == MX4_BF16, w->cols, ctx->cus, ctx->stream);
+        } else if (path == MX4_PATH_AUTO && m > 32 && mx4::gemm_bf16_supported(m, w->rows, w->cols, xt == MX4_BF16)) {
+            e = mx4::launch_gemm_bf16(&w->bf16, &y, &w->rows, 1, x, xt == MX4_BF16, m, w->cols, ctx->cus, ctx->split_part,
+                                      kSplitPartBytes, ctx->stream);
         } else if (path == MX4_PATH_AUTO && bf16_skinny(w, m)) {
             mx4::GemvArgs a{nullptr, nullptr, x, y, m, w->rows, w->cols, xt == MX4_BF16, ctx->stream};
             e = mx4::launch_skinny_any(a, &w->bf16, ctx->cus);
@@ -875,11 +878,13 @@ mx4_status mx4_matmul_group(mx4_context* ctx, const void* x, mx4_dtype xt, uint3
     }
     // bf16 weights: one launch over all of them
     bool bf16_group = count > 1, bf16_one = m == 1 && mx4::bf16_gemv_supported(k, xt == MX4_BF16);
+    bool bf16_many = m > 32;
     for (uint32_t i = 0; i < count; ++i) {
         bf16_one &= w[i]->bf16 != nullptr;
+        bf16_many &= w[i]->bf16 != nullptr && mx4::gemm_bf16_supported(m, w[i]->rows, k, xt == MX4_BF16);
         bf16_group &= bf16_skinny(w[i], m);
     }
-    if (bf16_one) {
+    if (bf16_one || bf16_many) {
         const uint16_t* values[4] = {};
         uint32_t rows[4] = {};
         for (uint32_t i = 0; i < count; ++i) {
@@ -887,7 +892,9 @@ mx4_status mx4_matmul_group(mx4_context* ctx, const void* x, mx4_dtype xt, uint3
             rows[i] = w[i]->rows;
         }
         const hipError_t e =
-            mx4::launch_bf16_gemv(values, y, rows, count, x, xt == MX4_BF16, k, ctx->cus, ctx->stream);
+            bf16_one ? mx4::launch_bf16_gemv(values, y, rows, count, x, xt == MX4_BF16, k, ctx->cus, ctx->stream)
+                     : mx4::launch_gemm_bf16(values, y, rows, count, x, xt == MX4_BF16, m, k, ctx->cus, ctx->split_part,
+                                             kSplitPartBytes, ctx->stream);
         if (e != hipSuccess) return fail(MX4_ERR_DEVICE, "kernel launch failed: %s", hipGetErrorString(e));
         return MX4_OK;
     }

@@ -266,3 +266,13 @@ def test_bf16_nonfinite(mx4, ctx, oracle, m, k):
     ((9000, 4000, 3), 136), ((40, 41), 12296), ((20, 3), 20480), ((17, 5), 24576), ((40, 20), 1604)])
 def test_bf16_decode(mx4, ctx, oracle, ns, k):
     check_bf16_weights(mx4, ctx, oracle, ns[0] + k, 1, ns, k)
+
+
+# tiles of 64 and 128 rows and columns, each full, one short and one over; K below,
+# at and past a 64-element stage, odd and even stage counts, K splits with a
+# short last slice, and K of no whole pieces
+@pytest.mark.parametrize("m,ns,k", [
+    (33, (1, 65), 8), (64, (64, 128, 2), 64), (65, (127, 33), 72), (129, (130, 5), 200), (40, (300, 7, 64, 1), 1032),
+    (200, (257, 64), 2056), (500, (1100, 40), 328), (70, (60, 9), 4100), (1000, (520,), 136)])
+def test_bf16_prompt(mx4, ctx, oracle, m, ns, k):
+    check_bf16_weights(mx4, ctx, oracle, m + k, m, ns, k)
