@@ -39,20 +39,6 @@ namespace mx4 {
 
 namespace {
 
-// Three bf16 terms of eight f32 values, hi + mid + lo = x exactly
-// (split3_bf16: non-finite values stay in hi).
-__device__ __forceinline__ void split3_each(const f32x4 a, const f32x4 b, bf16x8& hi, bf16x8& mid, bf16x8& lo) {
-    const float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        __bf16 h, md, l;
-        split3_bf16(v[e], h, md, l);
-        hi[e] = h;
-        mid[e] = md;
-        lo[e] = l;
-    }
-}
-
 // Eight weights of one lane at one k-step: packed word `word` (elements
 // [8s, 8s + 8) of the lane's 64), block scale 2^(s - 127) folded in.
 __device__ __forceinline__ bf16x8 decode8(uint32_t word, float sc) {
@@ -110,7 +96,9 @@ struct Geometry {
 // token rows) in one launch: weight s owns the column tiles [tile0[s],
 // tile0[s + 1]) of the grid; a workgroup picks its weight with uniform
 // selects. Passed as the trailing argument, so the leading scalars keep
-// arriving preloaded; NoGemmSegs stands there for one weight. No K split.
+// arriving preloaded; NoGemmSegs stands there for one weight. A K split's
+// partials of weight s are m x n[s] floats from m x row0[s] on in each slice's
+// m x rows.
 struct NoGemmSegs {};
 struct GemmSegs {
     const uint8_t* packed[4];
@@ -118,6 +106,8 @@ struct GemmSegs {
     float* y[4];
     uint32_t n[4];
     uint32_t tile0[4];
+    uint32_t row0[4];
+    uint32_t rows;
     uint32_t count;
 };
 
@@ -141,6 +131,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_exact_kernel(const uint8_t*
     const uint32_t slice = blockIdx.x / tiles, tile = blockIdx.x % tiles;
     uint32_t tn = tile % tiles_n;
     const uint32_t tm = tile / tiles_n;
+    uint32_t prow0 = 0, prows = n;  // a K split's partials
     if constexpr (std::is_same_v<SG, GemmSegs>) {
         // the column tile's weight, and the tile within it
         uint32_t t0 = 0;
@@ -148,6 +139,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_exact_kernel(const uint8_t*
         scales = group.scales[0];
         y = group.y[0];
         n = group.n[0];
+        prows = group.rows;
 #pragma unroll
         for (int q = 1; q < 4; ++q) {
             const bool in = q < (int)group.count && tn >= group.tile0[q];
@@ -156,6 +148,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_exact_kernel(const uint8_t*
             y = in ? group.y[q] : y;
             n = in ? group.n[q] : n;
             t0 = in ? group.tile0[q] : t0;
+            prow0 = in ? group.row0[q] : prow0;
         }
         tn -= t0;
     }
@@ -164,7 +157,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_exact_kernel(const uint8_t*
     const uint32_t k0 = slice * kslice;
     const uint32_t klen = ANY ? (k - k0 < kslice ? k - k0 : kslice) : kslice;
     const uint32_t stages = ANY ? (klen + kBK - 1) / kBK : klen / kBK;
-    if (part) y = part + (size_t)slice * m * n;
+    if (part) y = part + (size_t)slice * m * prows + (size_t)m * prow0;
 
     const __amdgpu_buffer_rsrc_t xr = rsrc(x, m * k * G::XB);
     const __amdgpu_buffer_rsrc_t pr = rsrc(packed, n * (k / 2));
@@ -292,10 +285,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_exact_kernel(const uint8_t*
                     for (int j = 0; j < TN; ++j) mac(s, i, j, a, b[j], true);
                 } else {
                     const uint32_t c0 = (16 * h + 2 * s) ^ sw16, c1 = (16 * h + 2 * s + 1) ^ sw16;
-                    const f32x4 v0 = __builtin_bit_cast(f32x4, *reinterpret_cast<const u32x4*>(ap + c0 * 16));
-                    const f32x4 v1 = __builtin_bit_cast(f32x4, *reinterpret_cast<const u32x4*>(ap + c1 * 16));
+                    const u32x4 v0 = *reinterpret_cast<const u32x4*>(ap + c0 * 16);
+                    const u32x4 v1 = *reinterpret_cast<const u32x4*>(ap + c1 * 16);
                     bf16x8 hi, mid, lo;
-                    split3_each(v0, v1, hi, mid, lo);
+                    split3x8(v0, v1, hi, mid, lo);
 #pragma unroll
                     for (int j = 0; j < TN; ++j) {
                         mac(s, i, j, hi, b[j], true);
@@ -379,6 +372,24 @@ __global__ __launch_bounds__(256) void split_sum_kernel(const float* __restrict_
     }
 }
 
+// The same for a group: the slices of all its weights in one pass.
+__global__ __launch_bounds__(256) void split_sum_group_kernel(const float* __restrict__ part, uint32_t ks, uint32_t m,
+                                                              const GemmSegs g) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x, count = m * g.rows;
+    if (i >= count) return;
+    float a = part[i];
+    for (uint32_t s = 1; s < ks; ++s) a += part[(size_t)s * count + i];
+    float* y = g.y[0];
+    uint32_t at = i;
+#pragma unroll
+    for (int q = 1; q < 4; ++q)
+        if (q < (int)g.count && i >= m * g.row0[q]) {
+            y = g.y[q];
+            at = i - m * g.row0[q];
+        }
+    y[at] = a;
+}
+
 template <bool XBF16, int WM, int WN, int TM, int TN, bool ANY>
 hipError_t go(const GemvArgs& a, uint32_t ks, float* part) {
     // deepest ring that fits: 3 stages of a 128 x 128 bf16 tile (121.5 KiB)
@@ -388,8 +399,7 @@ hipError_t go(const GemvArgs& a, uint32_t ks, float* part) {
     using G = Geometry<XBF16, WM, WN, TM, TN, D, ANY>;
     const uint32_t tiles_m = (a.m + G::BM - 1) / G::BM;
     if (a.group) {
-        // each weight of the group a run of column tiles; no K split
-        if (ks > 1) return hipErrorNotSupported;
+        // each weight of the group a run of column tiles
         GemmSegs sg{};
         uint32_t tiles_n = 0;
         sg.count = a.group->count;
@@ -399,11 +409,19 @@ hipError_t go(const GemvArgs& a, uint32_t ks, float* part) {
             sg.y[s] = a.group->y[s];
             sg.n[s] = a.group->n[s];
             sg.tile0[s] = tiles_n;
+            sg.row0[s] = sg.rows;
             tiles_n += (sg.n[s] + G::BN - 1) / G::BN;
+            sg.rows += sg.n[s];
         }
+        if (ks < 1) ks = 1;
         const uint32_t tiles = tiles_n * tiles_m;
-        hipLaunchKernelGGL((gemm_exact_kernel<XBF16, WM, WN, TM, TN, D, ANY, GemmSegs>), dim3(tiles), dim3(G::NT), 0,
-                           a.stream, nullptr, nullptr, a.x, nullptr, a.m, 0u, a.k, tiles_n, tiles, a.k, nullptr, sg);
+        hipLaunchKernelGGL((gemm_exact_kernel<XBF16, WM, WN, TM, TN, D, ANY, GemmSegs>), dim3(tiles * ks), dim3(G::NT), 0,
+                           a.stream, nullptr, nullptr, a.x, nullptr, a.m, 0u, a.k, tiles_n, tiles, slice_k(a.k, ks),
+                           ks > 1 ? part : nullptr, sg);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess || ks == 1) return e;
+        hipLaunchKernelGGL(split_sum_group_kernel, dim3((a.m * sg.rows + 255) / 256), dim3(256), 0, a.stream, part, ks,
+                           a.m, sg);
         return hipGetLastError();
     }
     const uint32_t tiles_n = (a.n + G::BN - 1) / G::BN;
@@ -425,11 +443,29 @@ hipError_t dispatch_rule(const GemvArgs& a, const GemmConfig& c, uint32_t ks, fl
     if (c.wm == 2 && c.wn == 2 && c.tm == 1 && c.tn == 1) return go<XBF16, 2, 2, 1, 1, ANY>(a, ks, part);
     if (c.wm == 1 && c.wn == 4 && c.tm == 2 && c.tn == 2) return go<XBF16, 1, 4, 2, 2, ANY>(a, ks, part);
     if (c.wm == 1 && c.wn == 4 && c.tm == 2 && c.tn == 1) return go<XBF16, 1, 4, 2, 1, ANY>(a, ks, part);
-    // a 128 x 256 tile of f32 activations would leave room for one stage only,
-    // and 64-bit sums do not fit the registers of its eight waves
-    if constexpr (XBF16 && !ANY)
+    if (c.wm == 2 && c.wn == 4 && c.tm == 1 && c.tn == 2) return go<XBF16, 2, 4, 1, 2, ANY>(a, ks, part);
+    // (picked by eight_waves only)
+    if constexpr (XBF16 == ANY) {
+        if (c.wm == 4 && c.wn == 2 && c.tm == 1 && c.tn == 2) return go<XBF16, 4, 2, 1, 2, ANY>(a, ks, part);
+        if (c.wm == 2 && c.wn == 4 && c.tm == 1 && c.tn == 1) return go<XBF16, 2, 4, 1, 1, ANY>(a, ks, part);
+    }
+    // a 128 x 256 tile of f32 activations would leave room for one stage only
+    if constexpr (XBF16)
         if (c.wm == 2 && c.wn == 4 && c.tm == 2 && c.tn == 2) return go<XBF16, 2, 4, 2, 2, ANY>(a, ks, part);
     return hipErrorNotSupported;
+}
+
+// Eight waves, two a SIMD, for the same tile where one wave's conversions (f32
+// activations, whole stages: 24576 x 4096 at 64 rows 96 -> 75 us, 12288 x 2048
+// at 300 rows 58.6 -> 50.7) or 64-bit sums (bf16, any width: 8576 x 1600 at 200
+// rows 27.5 -> 24.4 us) hold up its MFMAs. f32 at any width has both, and four
+// waves measured faster (8576 x 1600 at 77 rows 47 against 63 us); bf16 of whole
+// stages has neither, and runs the same in both.
+GemmConfig eight_waves(GemmConfig c, bool x_bf16, bool any) {
+    if (x_bf16 != any) return c;
+    if (c.wm == 2 && c.wn == 2 && c.tm == 2 && c.tn == 2) c.wm = 4, c.tm = 1;
+    else if (c.wm == 1 && c.wn == 4 && c.tm == 2) c.wm = 2, c.tm = 1;
+    return c;
 }
 
 template <bool XBF16>
@@ -442,7 +478,6 @@ hipError_t dispatch(const GemvArgs& a, const GemmConfig& c, float* part) {
     if (c.wm == 4 && c.wn == 1 && c.tm == 1 && c.tn == 2) return go<XBF16, 4, 1, 1, 2, false>(a, ks, part);
     if (c.wm == 1 && c.wn == 4 && c.tm == 1 && c.tn == 2) return go<XBF16, 1, 4, 1, 2, false>(a, ks, part);
     if (c.wm == 1 && c.wn == 4 && c.tm == 1 && c.tn == 1) return go<XBF16, 1, 4, 1, 1, false>(a, ks, part);
-    if (c.wm == 2 && c.wn == 4 && c.tm == 1 && c.tn == 2) return go<XBF16, 2, 4, 1, 2, false>(a, ks, part);
     return dispatch_rule<XBF16, false>(a, c, ks, part);
 }
 
@@ -492,6 +527,8 @@ hipError_t launch_gemm_exact(const GemvArgs& a, int cus, const GemmConfig* force
     GemmConfig c;
     if (forced && forced->wm) {
         c = *forced;
+        // arrangements of the shape rule's own
+        if ((c.wm == 4 && c.wn == 2) || (c.wm == 2 && c.wn == 4 && c.tm == 1 && c.tn == 1)) return hipErrorNotSupported;
         // an explicit K split: whole stages per slice and partials within the scratch
         if (c.ks > 1 && (a.k % ((uint32_t)c.ks * kBK) != 0 || !part ||
                          (uint64_t)c.ks * a.m * a.n * 4 > part_bytes))
@@ -514,8 +551,13 @@ hipError_t launch_gemm_exact(const GemvArgs& a, int cus, const GemmConfig* force
                               {1, 4, 2, 1, 64, 128, 22.0},  {2, 2, 1, 1, 64, 64, 16.5}};
         const uint64_t nc = (uint64_t)(cus > 0 ? cus : 256);
         const uint64_t want = nc * 3 / 4;
-        // 128 x 256 has an instance for bf16 x and whole stages only
-        auto wide = [&](const Cand& cd) { return cd.bn == 256 && cd.bm == 128 && (!a.x_bf16 || a.k % kBK != 0); };
+        // 128 x 256 has an instance for bf16 x only
+        auto wide = [&](const Cand& cd) { return cd.bn == 256 && cd.bm == 128 && !a.x_bf16; };
+        uint32_t rows = a.n;  // weight rows, of all the group's weights
+        if (a.group) {
+            rows = 0;
+            for (uint32_t s = 0; s < a.group->count; ++s) rows += a.group->n[s];
+        }
         const Cand* best = nullptr;
         double best_t = 0.0;
         for (const Cand& cd : cands) {
@@ -545,7 +587,7 @@ hipError_t launch_gemm_exact(const GemvArgs& a, int cus, const GemmConfig* force
                 const uint64_t tiles = (uint64_t)((a.m + cd.bm - 1) / cd.bm) * col_tiles(cd.bn);
                 for (uint32_t ks = 1; ks <= 4; ++ks) {
                     if (!slices_fit(a.k, ks)) continue;
-                    if (ks > 1 && (a.group || !part || (uint64_t)ks * a.m * a.n * 4 > part_bytes)) continue;
+                    if (ks > 1 && (!part || (uint64_t)ks * a.m * rows * 4 > part_bytes)) continue;
                     const uint64_t wgs = tiles * ks, area = (uint64_t)cd.bm * cd.bn;
                     if (wgs > nc || wgs < want) continue;
                     if (!sel || area > sel_area || (area == sel_area && wgs > sel_wgs)) {
@@ -559,7 +601,7 @@ hipError_t launch_gemm_exact(const GemvArgs& a, int cus, const GemmConfig* force
             if (sel) {
                 c.wm = sel->wm; c.wn = sel->wn; c.tm = sel->tm; c.tn = sel->tn;
                 c.ks = (int)sel_ks;
-                if (a.group) return a.x_bf16 ? dispatch<true>(a, c, nullptr) : dispatch<false>(a, c, nullptr);
+                c = eight_waves(c, a.x_bf16, a.k % kBK != 0);
                 return a.x_bf16 ? dispatch<true>(a, c, part) : dispatch<false>(a, c, part);
             }
         }
@@ -570,16 +612,13 @@ hipError_t launch_gemm_exact(const GemvArgs& a, int cus, const GemmConfig* force
         // fit the scratch; a second small kernel adds them in slice order.
         const uint64_t tiles = (uint64_t)((a.m + pick.bm - 1) / pick.bm) * col_tiles(pick.bn);
         c.ks = 1;
-        // a group runs unsplit even when its tiles leave CUs idle: one round
-        // of them beats its weights' separate launches, split or not (8B
-        // q|k|v at 64 token rows: 96 tiles)
-        if (a.group) return a.x_bf16 ? dispatch<true>(a, c, nullptr) : dispatch<false>(a, c, nullptr);
         for (uint32_t ks = 4; ks >= 2 && tiles < want; --ks) {
-            if (slices_fit(a.k, ks) && part && (uint64_t)ks * a.m * a.n * 4 <= kFewRowsSplitBytes) {
+            if (slices_fit(a.k, ks) && part && (uint64_t)ks * a.m * rows * 4 <= kFewRowsSplitBytes) {
                 c.ks = (int)ks;
                 break;
             }
         }
+        c = eight_waves(c, a.x_bf16, a.k % kBK != 0);
     }
     return a.x_bf16 ? dispatch<true>(a, c, part) : dispatch<false>(a, c, part);
 }
