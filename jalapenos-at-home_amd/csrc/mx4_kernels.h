@@ -84,6 +84,9 @@ hipError_t launch_skinny(const GemvArgs& a, int cus, const SkinnyScratch& sc);
 // values (one for each weight of the group; packed and scales are unused).
 bool skinny_any_supported(uint32_t m, uint32_t k, bool fp4);
 hipError_t launch_skinny_any(const GemvArgs& a, const uint16_t* const* bf16, int cus);
+// Does it beat the skinny kernel on a launch of `tiles` 16-row tiles of a width
+// that both take?
+bool skinny_any_faster(uint32_t m, uint32_t k, uint32_t tiles, bool x_bf16, int cus);
 
 // Exact GEMM on bf16 MFMA for more than 32 token rows (gemm.hip): K % 128 == 0,
 // scale bytes 2..252. GemmConfig picks an instance: waves along M x N and 32x32

@@ -372,7 +372,8 @@ mx4_status run_matmul(mx4_context* ctx, const void* x, mx4_dtype xt, uint32_t m,
         const bool one = m == 1 && (mx4::gemv_m1_supported(w->cols) || mx4::gemv_any_supported(w->cols));
         if ((one || tokens) && scales_foldable(w))
             path = MX4_PATH_GEMV;
-        else if (m >= 2 && mx4::skinny_supported(m, w->cols) && scales_foldable(w))
+        else if (m >= 2 && mx4::skinny_supported(m, w->cols) && scales_foldable(w) &&
+                 !mx4::skinny_any_faster(m, w->cols, (w->rows + 15) / 16, xt == MX4_BF16, ctx->cus))
             path = MX4_PATH_SKINNY;
         else if (mx4::skinny_any_supported(m, w->cols, true) && scales_foldable(w)) {
             path = MX4_PATH_SKINNY;  // (asked for by name, the path takes its tuned widths only)
@@ -844,15 +845,17 @@ mx4_status mx4_matmul_group(mx4_context* ctx, const void* x, mx4_dtype xt, uint3
     // few-token GEMV or the skinny kernel over all the weights' rows, chosen
     // as mx4_matmul chooses for one weight of the group's total rows
     bool stored = true;
-    uint32_t total = 0;
+    uint32_t total = 0, tiles = 0;
     for (uint32_t i = 0; i < count; ++i) {
         stored &= w[i]->bf16 == nullptr;
         total += w[i]->rows;
+        tiles += (w[i]->rows + 15) / 16;
     }
     const uint32_t k = w[0]->cols;
     const bool tokens = mx4::gemv_mt_supported(m, k, xt == MX4_BF16) &&
                         ((m == 2 && total < 65536) || (total <= 1024 && k >= 4096));
-    const bool skinny = !tokens && m >= 2 && mx4::skinny_supported(m, k);
+    const bool skinny = !tokens && m >= 2 && mx4::skinny_supported(m, k) &&
+                        !mx4::skinny_any_faster(m, k, tiles, xt == MX4_BF16, ctx->cus);
     const bool any_skinny = !tokens && !skinny && mx4::skinny_any_supported(m, k, true);
     if (count > 1 && stored && foldable && (tokens || skinny || any_skinny)) {
         mx4::GemvGroup gg{};

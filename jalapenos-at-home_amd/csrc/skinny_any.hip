@@ -460,6 +460,24 @@ bool skinny_any_supported(uint32_t m, uint32_t k, bool fp4) {
     return m >= 2 && m <= 32 && k >= 32 && k % (fp4 ? 32 : 8) == 0 && k <= (1u << 20);
 }
 
+// The tuned widths (skinny.hip). f32 activations: skinny.hip splits a token's
+// values again for every 16-row tile, here once for up to four of them (8B gate|up
+// at 7 / 29 rows 48 / 110 against 32 / 64 us, o 10.4 / 20.4 against 9.9 / 17.5,
+// down 25.9 / 63 against 22.4 / 45; 1.7B gate|up 17.1 / 37.3 against 11.1 / 24.8).
+// At K = 2048 with a tile or less a CU and one token tile it stays ahead (1.7B
+// q|k|v 6.3 against 6.7 us). bf16 ones: up to 16 rows it stays ahead everywhere
+// (its activations are resident too); beyond, where its weights are too long for
+// one tile a workgroup and too short for the tile ring, it loads them for every
+// tile (1.7B gate|up 20.8 against 10.5 us, 8B q|k|v 20.9 against 13.2; with fewer
+// tiles 11.2 against 11.4, with the ring 26.7 against 32).
+bool skinny_any_faster(uint32_t m, uint32_t k, uint32_t tiles, bool x_bf16, int cus) {
+    const uint32_t nc = (uint32_t)(cus > 0 ? cus : 256);
+    if (!x_bf16) return m > 16 || k != 2048 || tiles > nc;
+    // (the ring: two tiles for each of the workgroups of eight waves a CU)
+    const uint32_t ring = k == 2048 ? 4 * nc : 2 * nc;
+    return m > 16 && (k == 2048 || k == 4096) && tiles > nc && tiles < ring;
+}
+
 hipError_t launch_skinny_any(const GemvArgs& a, const uint16_t* const* bf16, int cus) {
     const bool fp4 = bf16 == nullptr;
     if (!skinny_any_supported(a.m, a.k, fp4)) return hipErrorNotSupported;
