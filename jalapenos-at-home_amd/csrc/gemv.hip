@@ -833,18 +833,22 @@ bool gemv_m1_supported(uint32_t k) {
 // because every workgroup loads the whole activation row (24 KiB at K =
 // 12288): at 12288 four 2-wave teams share one LDS copy of it. Grids are in
 // teams per CU.
-static void default_m1_config(uint32_t k, uint32_t rows, int cus, M1Config& c) {
+static void default_m1_config(uint32_t k, uint32_t rows, bool x_bf16, int cus, M1Config& c) {
     const uint32_t nblk = k / 32;
     const uint32_t scale = (uint32_t)(cus > 0 ? cus : 256);  // the table is for 256 CUs
     c.tpw = 1;
     switch (nblk) {
         case 64:  // K = 2048 (Qwen3-1.7B sweep: q|k|v 3.33 -> 3.14 us, gate|up 4.86 -> 4.71 us)
-            c.wg = 1; c.r = 2; c.grid = (rows > 2048 && rows <= 4096 ? 4 : 12) * scale;
-            // up to 2048 rows (o): eight one-row teams per workgroup sharing x,
-            // fetched ahead of the weights (2.42 -> 2.22 us)
-            if (rows <= 2048) { c.r = 1; c.grid = 8 * scale; c.tpw = 8; }
-            if (rows > 4096 && rows <= 8192) c.r = 4;
-            if (rows > 8192) c.grid = 16 * scale;
+            // up to 8192 rows: one-row teams, eight a workgroup (four with the
+            // twice as wide f32 x) sharing x, fetched ahead of the weights (o
+            // 2.42 -> 2.22 us; gate 3.57 -> 3.32 against four-row teams of their
+            // own, q|k|v 3.19 as with two-row ones; f32 x: k 3.06 -> 2.44, gate
+            // 4.37 -> 3.95 us)
+            c.wg = 1; c.r = 1; c.tpw = x_bf16 ? 8 : 4;
+            c.grid = (rows <= 4096 ? 8 : x_bf16 ? 32 : 16) * scale;
+            // gate|up: two rows, bf16 x not shared (4.7 against 5.0 us), f32 x by
+            // four teams (6.49 -> 5.56 us)
+            if (rows > 8192) { c.r = 2; c.tpw = x_bf16 && rows <= 12288 ? 1 : 4; c.grid = 16 * scale; }
             if (rows > 65536) { c.r = 4; c.tpw = 8; c.grid = 8 * scale; }  // vocabulary-sized
             break;
         case 128:  // K = 4096
@@ -853,14 +857,21 @@ static void default_m1_config(uint32_t k, uint32_t rows, int cus, M1Config& c) {
             // workgroup sharing x, fetched ahead of the weights
             if (rows <= 8192) { c.r = 1; c.grid = 8 * scale; c.tpw = 4; }
             if (rows > 8192) c.tpw = 8;
-            if (rows > 65536) { c.wg = 2; c.grid = 8 * scale; c.tpw = 4; }  // vocabulary-sized
+            // up to 16384 rows (gate alone 7.02 -> 6.52 us), and with f32 x (gate
+            // 8.91 -> 6.95, gate|up 12.1 -> 11.4 us), one-row teams too
+            if (rows > 8192 && (rows <= 16384 || !x_bf16)) { c.r = 1; c.grid = (x_bf16 ? 32 : 16) * scale; c.tpw = 4; }
+            if (rows > 65536) { c.r = 2; c.wg = 2; c.grid = 8 * scale; c.tpw = 4; }  // vocabulary-sized
             break;
         case 192:  // K = 6144: four one-wave teams per workgroup sharing x,
                    // fetched ahead of the weights (Qwen3-1.7B down 3.43 -> 3.09 us)
             c.wg = 1; c.r = 1; c.grid = 4 * scale; c.tpw = 4;
+            // more rows than that fills: eight (4096 / 16384 rows 4.61 / 11.5 -> 4.29 / 10.2 us)
+            if (rows > 2048 && x_bf16) { c.tpw = 8; c.grid = 8 * scale; }
             break;
-        case 256:  // K = 8192
-            c.wg = 2; c.r = 4; c.grid = 8 * scale;
+        case 256:  // K = 8192: four two-row teams of two waves sharing x (8192
+                   // rows, bf16 / f32 x: 9.8 / 14.9 -> 8.0 / 8.3 us against four
+                   // rows and x read by every team)
+            c.wg = 2; c.r = 2; c.grid = 4 * scale; c.tpw = 4;
             break;
         default:  // K = 12288
             c.wg = 2; c.r = 1; c.grid = 4 * scale; c.tpw = 4;
@@ -937,7 +948,7 @@ hipError_t launch_gemv_m1_group(const GemvGroup& g, int cus, const M1Config* for
     for (uint32_t s = 0; s < g.count; ++s) rows += g.n[s];
     M1Config c;
     if (any) default_any_config(g.k, rows, g.x_bf16, cus, c);
-    else default_m1_config(g.k, rows, cus, c);
+    else default_m1_config(g.k, rows, g.x_bf16, cus, c);
     if (forced) {
         if (forced->wg) c.wg = forced->wg;
         if (forced->r) c.r = forced->r;
@@ -1032,7 +1043,7 @@ hipError_t launch_gemv_m1_argmax(const GemvArgs& a, uint64_t* partial, uint32_t 
     if ((any && !gemv_any_supported(a.k)) || a.n == 0) return hipErrorNotSupported;
     M1Config c;
     if (any) default_any_config(a.k, a.n, a.x_bf16, cus, c);
-    else default_m1_config(a.k, a.n, cus, c);
+    else default_m1_config(a.k, a.n, a.x_bf16, cus, c);
     const uint32_t nblk = a.k / 32;
     const int sub = any ? any_sub(nblk) : 1;
     const uint32_t set = (uint32_t)(c.r * sub);
