@@ -187,6 +187,8 @@ hipError_t launch_synth_weight(uint64_t seed, double sigma, uint32_t rows, uint3
 constexpr uint32_t kMinMaxBlocks = 256;
 uint32_t min_max_scale_blocks(uint64_t count);
 hipError_t launch_min_max_scale(const uint8_t* scales, uint64_t count, uint32_t* out, hipStream_t s);
+// out[0 .. words) = in[0 .. words) on the stream; both 16-byte aligned.
+hipError_t launch_copy_words(const uint32_t* in, uint32_t* out, uint32_t words, hipStream_t s);
 // Hardware-converter table for the exhaustive decode check: out[s*16 + c]
 hipError_t launch_decode_table(int mode, float* out, hipStream_t s);
 // Matrix-core ceiling probe (probe.hip): back-to-back scaled FP4 MFMAs

@@ -717,6 +717,22 @@ __global__ void fill_u32_kernel(uint32_t* p, uint32_t count, uint32_t value) {
     if (i < count) p[i] = value;
 }
 
+// A copy within one queue, for the small operands of the per-call interface
+// (pinned host memory to HBM), which spend more on the waits between the
+// runtime's copy engine and the kernels' queue than on the transfer.
+__global__ __launch_bounds__(256) void copy_words_kernel(const uint32_t* __restrict__ in, uint32_t* __restrict__ out,
+                                                         uint32_t words) {
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x, quads = words / 4;
+    if (i < quads) reinterpret_cast<u32x4*>(out)[i] = reinterpret_cast<const u32x4*>(in)[i];
+    else if (i - quads < words % 4) out[4 * quads + i - quads] = in[4 * quads + i - quads];
+}
+
+hipError_t launch_copy_words(const uint32_t* in, uint32_t* out, uint32_t words, hipStream_t s) {
+    if (words == 0) return hipSuccess;
+    hipLaunchKernelGGL(copy_words_kernel, dim3((words / 4 + words % 4 + 255) / 256), dim3(256), 0, s, in, out, words);
+    return hipGetLastError();
+}
+
 hipError_t launch_fill_u32(uint32_t* p, uint32_t count, uint32_t value, hipStream_t s) {
     if (count == 0) return hipSuccess;
     hipLaunchKernelGGL(fill_u32_kernel, dim3((count + 255) / 256), dim3(256), 0, s, p, count, value);
