@@ -612,7 +612,11 @@ hipError_t launch_gemm_exact(const GemvArgs& a, int cus, const GemmConfig* force
         // fit the scratch; a second small kernel adds them in slice order.
         const uint64_t tiles = (uint64_t)((a.m + pick.bm - 1) / pick.bm) * col_tiles(pick.bn);
         c.ks = 1;
-        for (uint32_t ks = 4; ks >= 2 && tiles < want; --ks) {
+        // A bf16 group of whole stages splits below 2/7 of the CUs only: with 66
+        // tiles of 256 (q|k|v of width 2816 at 40 rows) the layer went 45.3 -> 43.8
+        // us, with 80 (4096 wide, 48 rows) 89.8 -> 90.3.
+        const bool few = a.group && a.x_bf16 && a.k % kBK == 0 ? 7 * tiles <= 2 * nc : tiles < want;
+        for (uint32_t ks = 4; ks >= 2 && few; --ks) {
             if (slices_fit(a.k, ks) && part && (uint64_t)ks * a.m * rows * 4 <= kFewRowsSplitBytes) {
                 c.ks = (int)ks;
                 break;
