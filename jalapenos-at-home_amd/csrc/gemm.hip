@@ -553,6 +553,11 @@ hipError_t launch_gemm_exact(const GemvArgs& a, int cus, const GemmConfig* force
         const uint64_t want = nc * 3 / 4;
         // 128 x 256 has an instance for bf16 x only
         auto wide = [&](const Cand& cd) { return cd.bn == 256 && cd.bm == 128 && !a.x_bf16; };
+        // A bf16 group of whole stages runs unsplit even when its tiles leave
+        // CUs idle: one short round of them beats a split and the pass that
+        // adds it (a small model's layer 28.0 against 30.3 us, 4096 wide at 48
+        // rows 89.8 against 90.3), and its weights' separate launches.
+        const bool may_split = !(a.group && a.x_bf16 && a.k % kBK == 0);
         uint32_t rows = a.n;  // weight rows, of all the group's weights
         if (a.group) {
             rows = 0;
@@ -587,7 +592,7 @@ hipError_t launch_gemm_exact(const GemvArgs& a, int cus, const GemmConfig* force
                 const uint64_t tiles = (uint64_t)((a.m + cd.bm - 1) / cd.bm) * col_tiles(cd.bn);
                 for (uint32_t ks = 1; ks <= 4; ++ks) {
                     if (!slices_fit(a.k, ks)) continue;
-                    if (ks > 1 && (!part || (uint64_t)ks * a.m * rows * 4 > part_bytes)) continue;
+                    if (ks > 1 && (!may_split || !part || (uint64_t)ks * a.m * rows * 4 > part_bytes)) continue;
                     const uint64_t wgs = tiles * ks, area = (uint64_t)cd.bm * cd.bn;
                     if (wgs > nc || wgs < want) continue;
                     if (!sel || area > sel_area || (area == sel_area && wgs > sel_wgs)) {
@@ -612,11 +617,7 @@ hipError_t launch_gemm_exact(const GemvArgs& a, int cus, const GemmConfig* force
         // fit the scratch; a second small kernel adds them in slice order.
         const uint64_t tiles = (uint64_t)((a.m + pick.bm - 1) / pick.bm) * col_tiles(pick.bn);
         c.ks = 1;
-        // A bf16 group of whole stages splits below 2/7 of the CUs only: with 66
-        // tiles of 256 (q|k|v of width 2816 at 40 rows) the layer went 45.3 -> 43.8
-        // us, with 80 (4096 wide, 48 rows) 89.8 -> 90.3.
-        const bool few = a.group && a.x_bf16 && a.k % kBK == 0 ? 7 * tiles <= 2 * nc : tiles < want;
-        for (uint32_t ks = 4; ks >= 2 && few; --ks) {
+        for (uint32_t ks = 4; ks >= 2 && tiles < want && may_split; --ks) {
             if (slices_fit(a.k, ks) && part && (uint64_t)ks * a.m * rows * 4 <= kFewRowsSplitBytes) {
                 c.ks = (int)ks;
                 break;

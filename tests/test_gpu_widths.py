@@ -102,7 +102,7 @@ def check_any_width(mx4, ctx, oracle, seed, m, ns, k, shift):
 @pytest.mark.parametrize("m,ns,k,shift", [
     (33, (1, 65, 31), 32, 0), (64, (64, 192), 96, 1), (65, (129, 3), 160, 2), (77, (320, 64, 64), 416, 3),
     (129, (50, 257), 352, 0), (40, (193, 33, 7, 64), 1600, 1), (200, (640, 96), 544, 2), (260, (2100,), 288, 3),
-    (50, (256, 64, 33), 512, 0)])  # (a bf16 group of whole stages, few tiles: split)
+    (50, (256, 64, 33), 512, 0)])  # (a group of whole stages: f32 split, bf16 not)
 def test_prompt_any_width(mx4, ctx, oracle, m, ns, k, shift):
     check_any_width(mx4, ctx, oracle, m + k, m, ns, k, shift)
 
