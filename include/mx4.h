@@ -188,9 +188,11 @@ mx4_status mx4_weight_drop_stored(mx4_weight *w);
  * (f32 accumulation of exact products). AUTO picks GEMV for m == 1, the
  * few-token GEMV or the exact skinny kernel for 2 <= m <= 32, and the exact
  * tiled GEMM on bf16 MFMA (MX4_PATH_GEMM) beyond -- the analogue of the
- * reference's M > 32 GEMM (engine/src/matmul.metal:65-97). Shapes the fast
- * kernels do not take (K not a multiple of 128, scale bytes outside 2..252)
- * run the exact generic kernel. */
+ * reference's M > 32 GEMM (engine/src/matmul.metal:65-97), each in a form for
+ * the tuned widths and one for any K % 32 == 0; bf16 weights have a GEMV, a
+ * skinny form and a GEMM of their own (K % 8 == 0). Weights with scale bytes
+ * outside 2..252 run the exact generic kernel. (Asked for by name, GEMV and
+ * SKINNY take their tuned widths and GEMM takes K % 128 == 0 only.) */
 mx4_status mx4_matmul(mx4_context *ctx, const void *x_dev, mx4_dtype x_type, uint32_t m,
                       const mx4_weight *w, float *y_dev);
 /* The same with an explicit kernel family (MX4_PATH_PREFILL is not exact:
@@ -200,10 +202,11 @@ mx4_status mx4_matmul_path(mx4_context *ctx, const void *x_dev, mx4_dtype x_type
 /* Up to 4 weights of the same width that read the same activations (q|k|v,
  * gate|up) in one launch: y_dev[i][m][w[i].rows] = x . W_i^T. For m == 1 this
  * is one GEMV over the concatenated rows; for 2 <= m <= 32 (a speculative
- * verify step) one launch of the few-token GEMV or the skinny kernel over all
+ * verify step) one launch of the few-token GEMV or a skinny kernel over all
  * the weights' rows, chosen as mx4_matmul would choose for one weight of the
  * group's total rows; for m > 32 one launch of the exact GEMM over all the
- * weights' column tiles (K unsplit); otherwise (bf16 weights, scale bytes
+ * weights' column tiles (and one that adds its K slices, if any); groups of
+ * bf16 weights likewise. Otherwise (MXFP4 and bf16 weights mixed, scale bytes
  * outside 2..252) the projections run one after another. Same arithmetic as
  * mx4_matmul: exact products, f32 sums, so each output equals mx4_matmul's
  * for its weight within f32 rounding (the same bits when both choose the same

@@ -428,8 +428,8 @@ hipError_t launch_decode_table(int mode, float* out, hipStream_t s) {
 // pairs. Bound by the read of the scales (1.5 MiB for 12288 x 4096), so the
 // bytes come in 16 at a time and nothing is written twice: a byte per thread
 // with two atomics per wave on one word each serialised on those words (16
-// thousand of them: 189 us at 12288 x 4096, and 318 -> 129 us for a quantize +
-// wrap + dequantize of that weight without them). The bytes before the
+// thousand of them: 189 us at 12288 x 4096, now 3.2; 318 -> 129 us for a
+// quantize + wrap + dequantize of that weight). The bytes before the
 // first and after the last whole 16-byte piece go one per thread to block 0.
 __global__ __launch_bounds__(256) void min_max_scale_kernel(const uint8_t* __restrict__ scales, uint64_t count,
                                                             uint32_t* __restrict__ out) {

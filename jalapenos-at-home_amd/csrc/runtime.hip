@@ -918,7 +918,7 @@ mx4_status mx4_matmul_group(mx4_context* ctx, const void* x, mx4_dtype xt, uint3
         return MX4_OK;
     }
     // more than 32 token rows (prefill in the reference's arithmetic): one
-    // exact-GEMM launch over all the weights' column tiles, unsplit
+    // exact-GEMM launch over all the weights' column tiles
     if (count > 1 && stored && foldable && m > 32) {
         mx4::GemvGroup gg{};
         gg.count = count;
