@@ -18,6 +18,9 @@ one by one.
 Algorithmic bytes of one GEMV: N*K/2 (nibbles) + N*K/32 (scales) + M*K*2 (bf16
 x) + M*N*4 (f32 y). value = bytes per step / wall time per step.
 
+stdout is one JSON line, the result; further figures ("extra") go to stderr, a
+line `extra.<name>: {...}` each.
+
 Timing protocol of every figure in `extra` (engine/src/model.rs:259-264,
 engine/src/main.rs:70): a recorded pass of distinct weight copies totalling at
 least 512 MiB per shape (cold: twice the Infinity Cache), 2 untimed launches,
@@ -96,6 +99,15 @@ def weight_bytes(n: int, k: int) -> int:
 
 def log(msg: str) -> None:
     print(msg, file=sys.stderr, flush=True)
+
+
+def report(out: dict, extra: dict) -> None:
+    """The result as the one line of stdout, and each entry of `extra` as a line
+    of stderr before it: with the per-shape figures in it the line was 22 KB,
+    more than a reader that keeps the end of the output has left of it."""
+    for name, entry in extra.items():
+        log(f"extra.{name}: {json.dumps(entry)}")
+    print(json.dumps(out), flush=True)
 
 
 def library_sha256() -> str:
@@ -1523,7 +1535,6 @@ def main() -> int:
             cpu_extra["verify_all_threads"] = cpu_verify(ctx, weights, nt)
             cpu_extra["prefill_all_threads"] = cpu_prefill(ctx, weights, nt)
         log("cpu legs: whole shapes (the single 6144 x 2048 GEMV, every Qwen3-1.7B M = 1 projection)")
-        # last in the line, so that the end of the printed line carries it whole
         cpu_extra["full_shapes"] = cpu_full_shapes(ctx, [1] + ([nt] if nt > 1 else []))
         extra["cpu"] = cpu_extra
 
@@ -1553,9 +1564,8 @@ def main() -> int:
                      "basis": "algorithmic bytes of one decode step / GPU event time of one step"},
         "cpu_baseline": cpu,
         "prefill": prefill_top,
-        "extra": extra,
     }
-    print(json.dumps(out), flush=True)
+    report(out, extra)
     ctx.synchronize()
     arena.release()
     ctx.close()

@@ -179,3 +179,17 @@ def test_prefill_summary_is_compact_and_reads_the_stamped_counters(tmp_path, mon
     assert top["mxfp4"]["gate"] == [18.123, 2843, 0.2815, 0.3, 24.5, 2100, 0.2079]
     assert top["requant_error_vs_unquantized"]["mxfp4"]["max_rel"] == 1.2e-2
     assert len(json.dumps(top)) < 1500
+
+
+def test_result_is_one_short_line(capsys):
+    """stdout holds the result alone, short enough to be read whole from the
+    end of a log; the further figures are lines of stderr."""
+    out = {"metric": "m", "value": 4250.0, "unit": "GB/s", "ms_per_step": 0.94, "prefill": {"q": [1.0] * 150}}
+    extra = {f"section{i}": {f"shape{j}": {"us": 12.345, "GBps": 1234.5} for j in range(60)} for i in range(12)}
+    bench.report(out, extra)
+    got = capsys.readouterr()
+    assert got.out.count("\n") == 1 and len(got.out) < 4096
+    assert json.loads(got.out) == out
+    lines = got.err.splitlines()
+    assert [line.split(": ", 1)[0] for line in lines] == [f"extra.{name}" for name in extra]
+    assert [json.loads(line.split(": ", 1)[1]) for line in lines] == list(extra.values())
