@@ -946,6 +946,7 @@ hipError_t launch_gemv_m1_group(const GemvGroup& g, int cus, const M1Config* for
     if (g.count < 1 || g.count > kMaxSegs || (any && !gemv_any_supported(g.k))) return hipErrorNotSupported;
     uint32_t rows = 0;
     for (uint32_t s = 0; s < g.count; ++s) rows += g.n[s];
+    const uint32_t nblk = g.k / 32;
     M1Config c;
     if (any) default_any_config(g.k, rows, g.x_bf16, cus, c);
     else default_m1_config(g.k, rows, g.x_bf16, cus, c);
@@ -953,9 +954,10 @@ hipError_t launch_gemv_m1_group(const GemvGroup& g, int cus, const M1Config* for
         if (forced->wg) c.wg = forced->wg;
         if (forced->r) c.r = forced->r;
         if (forced->tpw) c.tpw = forced->tpw;
+        // (the default is four teams of two waves: four of four do not fit a workgroup)
+        else if (forced->wg > 2 && nblk == 256) c.tpw = 1;
         if (forced->wg || forced->r || forced->grid) c.grid = forced->grid;
     }
-    const uint32_t nblk = g.k / 32;
     if (c.wg < 1 || (!any && nblk % (64u * c.wg) != 0)) return hipErrorNotSupported;
     if (c.tpw < 1 || 64 * c.wg * c.tpw > 512) return hipErrorNotSupported;
     // x staged in LDS with the partial sums: at most 64 KiB (the rule for any width sees to it)

@@ -277,3 +277,21 @@ def test_bf16_decode(mx4, ctx, oracle, ns, k):
     (200, (257, 64), 2056), (500, (1100, 40), 328), (70, (60, 9), 4100), (1000, (520,), 136)])
 def test_bf16_prompt(mx4, ctx, oracle, m, ns, k):
     check_bf16_weights(mx4, ctx, oracle, m + k, m, ns, k)
+
+
+@pytest.mark.parametrize("team", [1, 2, 4])
+def test_explicit_team_keeps_a_default_that_fits(mx4, ctx, oracle, team):
+    """An explicit team size with the default number of teams a workgroup, at
+    the width whose default is several two-wave teams (K = 8192)."""
+    rng = np.random.default_rng(team)
+    n, k = 70, 8192
+    packed, scales = planted(rng, n, k)
+    w = wrapped(ctx, packed, scales, 0)
+    for xt in (mx4.BF16, mx4.F32):
+        xb, x = activations(mx4, ctx, rng, 1, k, xt)
+        ref = oracle.matmul(x, packed.reshape(-1), scales.reshape(-1))
+        for teams in (0, 7):
+            y = ctx.to_device(np.full(n, np.nan, np.float32))
+            ctx.gemv_config(xb.ptr, xt, w, y.ptr, team, 1, teams, 0)
+            assert_close(y.download(np.float32).reshape(1, n), ref, f"team={team} xt={xt} teams={teams}", scaled=True)
+    w.release()
