@@ -90,6 +90,14 @@ __device__ __forceinline__ void mfma_drain() {
     __builtin_amdgcn_sched_barrier(0);
 }
 
+// Between one lane's LDS writes and another's reads in the same wave: the LDS
+// serves a wave's accesses in order, so this only keeps the compiler, which
+// sees each lane's own addresses, from turning the order round.
+__device__ __forceinline__ void wave_handover() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // FP4: weights are MXFP4 (else bf16). MT: token tiles of 16. NC: chunks per
 // wave and slice. T: 16-row weight tiles per workgroup at a time.
 // Workgroups with blockIdx.y = 1 take the token rows from 16 MT on.
@@ -265,8 +273,10 @@ __global__ __launch_bounds__(64 * TW) void skinny_any_kernel(const void* __restr
         if constexpr (TRANS) {
 #pragma unroll
             for (int q = 0; q < NC; ++q) stage[wave][slot(q, lane / BPR, lane % BPR)] = u.w[q][0];
+            wave_handover();
 #pragma unroll
             for (int q = 0; q < NC; ++q) w4[q] = stage[wave][slot(col / RPL, col % RPL, 4 * q + gq)];
+            wave_handover();
         } else if constexpr (FP4) {
 #pragma unroll
             for (int q = 0; q < NC; ++q) w4[q] = u.w[q][0];

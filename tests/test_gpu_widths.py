@@ -154,6 +154,16 @@ def test_verify_any_width(mx4, ctx, oracle, m, ns, k, shift):
     check_any_width(mx4, ctx, oracle, m + ns[0] + k, m, ns, k, shift)
 
 
+# the instances that turn the weights through the wave's LDS stage with several
+# tiles and slices in a row: four chunks a wave (two tiles; more than 256 row
+# tiles of K > 2048), two (one and two tiles; two and four with two token tiles)
+@pytest.mark.parametrize("m,ns,k,shift", [
+    (7, (4200, 16), 3264, 0), (16, (9000, 40), 2592, 1), (9, (5000,), 8224, 2), (5, (600, 50), 2080, 3),
+    (12, (4500,), 1056, 1), (29, (4300, 17), 1600, 0), (20, (9000,), 3104, 3)])
+def test_verify_staged_weights(mx4, ctx, oracle, m, ns, k, shift):
+    check_any_width(mx4, ctx, oracle, m + ns[0] + k, m, ns, k, shift)
+
+
 @pytest.mark.parametrize("m,k", [(1, 416), (5, 416), (13, 1600), (29, 544), (40, 352)])
 def test_nonfinite_activations_any_width(mx4, ctx, oracle, m, k):
     """An inf, a NaN or the largest finite value in one token row shows in that
