@@ -191,7 +191,11 @@ mx4_status mx4_weight_drop_stored(mx4_weight *w);
  * reference's M > 32 GEMM (engine/src/matmul.metal:65-97), each in a form for
  * the tuned widths and one for any K % 32 == 0; bf16 weights have a GEMV, a
  * skinny form and a GEMM of their own (K % 8 == 0). Weights with scale bytes
- * outside 2..252 run the exact generic kernel. (Asked for by name, GEMV and
+ * outside 2..252 run the exact generic kernel. f32 activations meet the matrix
+ * cores as three bf16 terms: every bit of every f32 on the any-width and bf16
+ * kernels; on the tuned widths' own (beyond 32 rows K % 128 == 0, and the tuned
+ * skinny kernel) bits below 2^-133, so of activations below 2^-110, are lost, as
+ * they always were there. (Asked for by name, GEMV and
  * SKINNY take their tuned widths and GEMM takes K % 128 == 0 only.) */
 mx4_status mx4_matmul(mx4_context *ctx, const void *x_dev, mx4_dtype x_type, uint32_t m,
                       const mx4_weight *w, float *y_dev);

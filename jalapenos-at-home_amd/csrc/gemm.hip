@@ -30,7 +30,11 @@
 //    are not stored;
 //  * widths that are no whole number of stages (any K % 32 == 0: the ANY
 //    instances) zero the last stage's columns past K the same way, and take
-//    the scale bytes, whose rows then start at any byte, as aligned words.
+//    the scale bytes, whose rows then start at any byte, as aligned words. With
+//    f32 activations they look at each stage's largest magnitude a lane, and a
+//    workgroup that met tiny or non-finite ones walks K again with care for them
+//    (mx4_device.h): 1600 x 1600 at 77 rows 18.8 -> 13.5 us against a check (for
+//    non-finite ones only) at every eight values, other shapes within 3%.
 #include <type_traits>
 #include "mx4_device.h"
 #include "mx4_kernels.h"
@@ -166,53 +170,6 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_exact_kernel(const uint8_t*
     const __amdgpu_buffer_rsrc_t sr =
         ANY ? rsrc(scales - mis, (n * (k / 32) + mis + 3) & ~3u) : rsrc(scales, n * (k / 32));
 
-    // this lane's global offsets (stage 0) of its loads; LDS slot p = (q NW + wave) 64 + lane
-    uint32_t a_goff[G::A_INSTR], b_goff[G::B_INSTR], s_goff[G::S_INSTR];
-    uint32_t a_col[G::A_INSTR], b_col[G::B_INSTR];  // first element within the stage (ANY)
-#pragma unroll
-    for (int q = 0; q < G::A_INSTR; ++q) {
-        const uint32_t p = (q * G::NW + wave) * 64 + lane, row = p / G::A_CPR, c = (p % G::A_CPR) ^ (row % 16);
-        a_goff[q] = (row0 + row) * k * G::XB + k0 * G::XB + c * 16;
-        a_col[q] = c * 16 / G::XB;
-    }
-#pragma unroll
-    for (int q = 0; q < G::B_INSTR; ++q) {
-        const uint32_t p = (q * G::NW + wave) * 64 + lane, row = p / 4, c = (p % 4) ^ ((row >> 2) & 3);
-        b_goff[q] = (col0 + row) * (k / 2) + k0 / 2 + c * 16;
-        b_col[q] = c * 32;
-    }
-#pragma unroll
-    for (int q = 0; q < G::S_INSTR; ++q) {
-        const uint32_t p = wave * G::S_WORDS + q * 64 + lane, row = ANY ? p / 2 : p;
-        s_goff[q] = (col0 + row) * (k / 32) + k0 / 32 + mis;
-        if (ANY) s_goff[q] = (s_goff[q] & ~3u) + 4 * (p % 2);
-    }
-
-    auto issue = [&](uint32_t st, uint32_t slot) {
-        uint8_t* base = lds + slot * G::STAGE;
-        const uint32_t live = klen - st * kBK;  // ANY: columns of the stage before K's end
-#pragma unroll
-        for (int q = 0; q < G::A_INSTR; ++q) {
-            uint32_t off = a_goff[q] + st * kBK * G::XB;
-            if (ANY) off = a_col[q] < live ? off : kPastEnd;
-            load_lds16(xr, (lds_ptr)(base + (q * G::NW + wave) * 1024), off);
-        }
-#pragma unroll
-        for (int q = 0; q < G::B_INSTR; ++q) {
-            uint32_t off = b_goff[q] + st * (kBK / 2);
-            if (ANY) off = b_col[q] < live ? off : kPastEnd;
-            load_lds16(pr, (lds_ptr)(base + G::A_BYTES + (q * G::NW + wave) * 1024), off);
-        }
-        // the wave's scale words; lanes past them stay inactive, so they
-        // write nothing into the next wave's words (the instruction still
-        // counts once in vmcnt: lane 0 is always active)
-#pragma unroll
-        for (int q = 0; q < G::S_INSTR; ++q)
-            if (q * 64 + lane < (uint32_t)G::S_WORDS)
-                load_lds4(sr, (lds_ptr)(base + G::A_BYTES + G::B_BYTES + (wave * G::S_WORDS + q * 64) * 4),
-                          s_goff[q] + st * (kBK / 32));
-    };
-
     using Acc = std::conditional_t<ANY, f64x16, f32x16>;
     Acc acc[TM][TN];
 #pragma unroll
@@ -226,6 +183,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_exact_kernel(const uint8_t*
 #pragma unroll
     for (int j = 0; j < TN; ++j)
         s_shift[j] = 8 * (((col0 + (wn * TN + j) * 32 + r32) * (k / 32) + k0 / 32 + mis) & 3);
+    bool care = false;  // ANY, f32 x: this lane's activations of some stage are not plain
     auto compute = [&](uint32_t st, uint32_t slot) {
         const uint8_t* base = lds + slot * G::STAGE;
         // ANY: blocks past K keep scale byte 0 (what follows the row in memory is no scale of theirs)
@@ -254,6 +212,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_exact_kernel(const uint8_t*
         // in 32 bits up to 1.7 times, in 64 bits no further. (The chains of
         // the other instances are what those widths always had.)
         f32x16 sum[ANY ? TM : 1][ANY ? TN : 1];
+        float most[TM];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) most[i] = 0.0f;
         auto mac = [&](int s, int i, int j, bf16x8 a, bf16x8 w, bool first) {
             if constexpr (ANY) {
                 f32x16 c;
@@ -288,7 +249,19 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_exact_kernel(const uint8_t*
                     const u32x4 v0 = *reinterpret_cast<const u32x4*>(ap + c0 * 16);
                     const u32x4 v1 = *reinterpret_cast<const u32x4*>(ap + c1 * 16);
                     bf16x8 hi, mid, lo;
-                    split3x8(v0, v1, hi, mid, lo);
+                    if constexpr (ANY) {
+                        split3_finite(v0, v1, hi, mid, lo);
+                        take_most(v0, most[i]);
+                        take_most(v1, most[i]);
+                        // several tiles a wave: each split between the MFMAs of the one
+                        // before it, and no further ahead (a branch keeps the compiler
+                        // to that in fewer registers than a scheduling barrier)
+                        if constexpr (TM * TN > 1)
+                            if (__any(!(most[i] < __builtin_inff())))
+                                hi = mid = lo = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
+                    } else {
+                        split3x8(v0, v1, hi, mid, lo);
+                    }
 #pragma unroll
                     for (int j = 0; j < TN; ++j) {
                         mac(s, i, j, hi, b[j], true);
@@ -306,23 +279,156 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_exact_kernel(const uint8_t*
                 for (int j = 0; j < TN; ++j)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) acc[i][j][r] += (double)sum[i][j][r];
+            if constexpr (!XBF16) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i) care |= !plain(most[i]);
+            }
+        }
+    };
+    // the same with the careful split, the tiny lanes' values in a pass of their own
+    auto compute_careful = [&](uint32_t st, uint32_t slot) {
+        const uint8_t* base = lds + slot * G::STAGE;
+        const uint32_t live = klen - st * kBK;
+        const uint32_t s_mask = live < (uint32_t)kBK ? (1u << (live / 4)) - 1 : ~0u;
+        auto x_piece = [&](int i, uint32_t s, u32x4& v0, u32x4& v1) {
+            const uint32_t r = (wm * TM + i) * 32 + r32, c = 16 * h + 2 * s;
+            const uint8_t* ap = base + r * (G::A_CPR * 16);
+            v0 = *reinterpret_cast<const u32x4*>(ap + (c ^ (r % 16)) * 16);
+            v1 = *reinterpret_cast<const u32x4*>(ap + ((c + 1) ^ (r % 16)) * 16);
+        };
+        float most[TM];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            most[i] = 0.0f;
+#pragma unroll 1
+            for (uint32_t s = 0; s < 8; ++s) {
+                u32x4 v0, v1;
+                x_piece(i, s, v0, v1);
+                take_most(v0, most[i]);
+                take_most(v1, most[i]);
+            }
+        }
+#pragma unroll 1
+        for (int pass = 0; pass < 2; ++pass) {
+            f32x16 sum[TM][TN];
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) sum[i][j][r] = 0.0f;
+#pragma unroll 1
+            for (uint32_t s = 0; s < 8; ++s) {
+                bf16x8 b[TN];
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    const uint32_t r = (wn * TN + j) * 32 + r32, c = (2 * h + s / 4) ^ ((r >> 2) & 3);
+                    const uint2 two = *reinterpret_cast<const uint2*>(base + G::A_BYTES + G::B_BYTES + r * 8);
+                    const uint32_t sw = __builtin_amdgcn_alignbit(two.y, two.x, s_shift[j]) & s_mask;
+                    b[j] = decode8(*reinterpret_cast<const uint32_t*>(base + G::A_BYTES + r * 64 + c * 16 + 4 * (s % 4)),
+                                   __uint_as_float(((sw >> (8 * (2 * h + s / 4))) & 0xffu) << 23));
+                }
+#pragma unroll
+                for (int i = 0; i < TM; ++i) {
+                    u32x4 v0, v1;
+                    x_piece(i, s, v0, v1);
+                    bf16x8 hi, mid, lo;
+                    split3_pass(pass, all_tiny(most[i]), v0, v1, hi, mid, lo);
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) {
+                        sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(hi, b[j], sum[i][j], 0, 0, 0);
+                        sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(mid, b[j], sum[i][j], 0, 0, 0);
+                        sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lo, b[j], sum[i][j], 0, 0, 0);
+                    }
+                }
+            }
+            mfma_drain();
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[i][j][r] += (double)sum[i][j][r] * (pass ? kTinyDown : 1.0);
         }
     };
 
     // D-stage ring: stages st + 1 .. st + D - 2 stay in flight while stage st
     // is computed; stage st + D - 1 is issued into the slot stage st - 1 used,
     // after the barrier that ends every wave's reads of it
+    auto walk = [&](auto&& step) {
+        // (opaque: a second walk computes its offsets again, instead of the first
+        // one's registers holding them)
+        uint32_t lane = threadIdx.x % 64;
+        asm volatile("" : "+v"(lane));
+        // this lane's global offsets (stage 0) of its loads; LDS slot p = (q NW + wave) 64 + lane
+        uint32_t a_goff[G::A_INSTR], b_goff[G::B_INSTR], s_goff[G::S_INSTR];
+        uint32_t a_col[G::A_INSTR], b_col[G::B_INSTR];  // first element within the stage (ANY)
 #pragma unroll
-    for (int p = 0; p < D - 1; ++p)
-        if ((uint32_t)p < stages) issue(p, p);
-    for (uint32_t st = 0; st < stages; ++st) {
-        const uint32_t ahead = stages - 1 - st;  // stages issued after st, at most D - 2
-        if (ahead >= (uint32_t)(D - 2)) wait_vm<(D - 2) * G::LPS>();
-        else if (D > 3 && ahead == 1) wait_vm<(D > 3 ? 1 : 0) * G::LPS>();
-        else wait_vm<0>();
-        lds_barrier();
-        if (st + D - 1 < stages) issue(st + D - 1, (st + D - 1) % D);
-        compute(st, st % D);
+        for (int q = 0; q < G::A_INSTR; ++q) {
+            const uint32_t p = (q * G::NW + wave) * 64 + lane, row = p / G::A_CPR, c = (p % G::A_CPR) ^ (row % 16);
+            a_goff[q] = (row0 + row) * k * G::XB + k0 * G::XB + c * 16;
+            a_col[q] = c * 16 / G::XB;
+        }
+#pragma unroll
+        for (int q = 0; q < G::B_INSTR; ++q) {
+            const uint32_t p = (q * G::NW + wave) * 64 + lane, row = p / 4, c = (p % 4) ^ ((row >> 2) & 3);
+            b_goff[q] = (col0 + row) * (k / 2) + k0 / 2 + c * 16;
+            b_col[q] = c * 32;
+        }
+#pragma unroll
+        for (int q = 0; q < G::S_INSTR; ++q) {
+            const uint32_t p = wave * G::S_WORDS + q * 64 + lane, row = ANY ? p / 2 : p;
+            s_goff[q] = (col0 + row) * (k / 32) + k0 / 32 + mis;
+            if (ANY) s_goff[q] = (s_goff[q] & ~3u) + 4 * (p % 2);
+        }
+        auto issue = [&](uint32_t st, uint32_t slot) {
+            uint8_t* base = lds + slot * G::STAGE;
+            const uint32_t live = klen - st * kBK;  // ANY: columns of the stage before K's end
+#pragma unroll
+            for (int q = 0; q < G::A_INSTR; ++q) {
+                uint32_t off = a_goff[q] + st * kBK * G::XB;
+                if (ANY) off = a_col[q] < live ? off : kPastEnd;
+                load_lds16(xr, (lds_ptr)(base + (q * G::NW + wave) * 1024), off);
+            }
+#pragma unroll
+            for (int q = 0; q < G::B_INSTR; ++q) {
+                uint32_t off = b_goff[q] + st * (kBK / 2);
+                if (ANY) off = b_col[q] < live ? off : kPastEnd;
+                load_lds16(pr, (lds_ptr)(base + G::A_BYTES + (q * G::NW + wave) * 1024), off);
+            }
+            // the wave's scale words; lanes past them stay inactive, so they
+            // write nothing into the next wave's words (the instruction still
+            // counts once in vmcnt: lane 0 is always active)
+#pragma unroll
+            for (int q = 0; q < G::S_INSTR; ++q)
+                if (q * 64 + lane < (uint32_t)G::S_WORDS)
+                    load_lds4(sr, (lds_ptr)(base + G::A_BYTES + G::B_BYTES + (wave * G::S_WORDS + q * 64) * 4),
+                              s_goff[q] + st * (kBK / 32));
+        };
+#pragma unroll
+        for (int p = 0; p < D - 1; ++p)
+            if ((uint32_t)p < stages) issue(p, p);
+        for (uint32_t st = 0; st < stages; ++st) {
+            const uint32_t ahead = stages - 1 - st;  // stages issued after st, at most D - 2
+            if (ahead >= (uint32_t)(D - 2)) wait_vm<(D - 2) * G::LPS>();
+            else if (D > 3 && ahead == 1) wait_vm<(D > 3 ? 1 : 0) * G::LPS>();
+            else wait_vm<0>();
+            lds_barrier();
+            if (st + D - 1 < stages) issue(st + D - 1, (st + D - 1) % D);
+            step(st, st % D);
+        }
+    };
+    walk(compute);
+    if constexpr (ANY && !XBF16) {
+        if (workgroup_any<G::NW>(__any(care), reinterpret_cast<uint32_t*>(lds), wave)) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[i][j][r] = 0;
+            walk(compute_careful);
+        }
     }
     mfma_drain();
 

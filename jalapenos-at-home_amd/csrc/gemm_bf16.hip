@@ -8,7 +8,8 @@
 // barrier per stage. A wave owns TM x TN 32x32 tiles of
 // V_MFMA_F32_32X32X16_BF16: lane l (row l % 32, half h = l / 32) takes elements
 // [32 h, 32 h + 32) of the stage, MFMA s elements [32 h + 8 s, +8), for both
-// operands alike. f32 activations are three bf16 terms (exact products).
+// operands alike. f32 activations are three bf16 terms (exact products; a workgroup that
+// met tiny or non-finite ones does its work again with care for them).
 //
 // Two stages are summed from zero and added to the running sums in 64 bits: as
 // far from the exact sum as the kernel that ran these shapes before, whose
@@ -145,64 +146,132 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_kernel(const void* __r
                 acc[i][j][r] = 0.0;
                 sum[i][j][r] = 0.0f;
             }
+    // the stages' sums so far into the running ones
+    auto fold = [&](double scale) {
+        mfma_drain();
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    acc[i][j][r] += (double)sum[i][j][r] * scale;
+                    sum[i][j][r] = 0.0f;
+                }
+    };
+    auto w_piece = [&](const uint8_t* base, int j, uint32_t s) {
+        const uint32_t r = (wn * TN + j) * 32 + r32;
+        return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(
+                                              base + G::A_BYTES + (r * G::B_CPR + turned<G::B_CPR>(r, 4 * h + s)) * 16));
+    };
+    // f32 x: eight values
+    auto x_piece = [&](const uint8_t* base, int i, uint32_t s, u32x4& v0, u32x4& v1) {
+        const uint32_t r = (wm * TM + i) * 32 + r32;
+        const uint8_t* ap = base + r * G::A_CPR * 16;
+        v0 = *reinterpret_cast<const u32x4*>(ap + turned<G::A_CPR>(r, 8 * h + 2 * s) * 16);
+        v1 = *reinterpret_cast<const u32x4*>(ap + turned<G::A_CPR>(r, 8 * h + 2 * s + 1) * 16);
+    };
+    auto mac3 = [&](int i, int j, bf16x8 hi, bf16x8 mid, bf16x8 lo, bf16x8 b) {
+        sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lo, b, sum[i][j], 0, 0, 0);
+        sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(mid, b, sum[i][j], 0, 0, 0);
+        sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(hi, b, sum[i][j], 0, 0, 0);
+    };
+    bool care = false;  // f32 x: this lane's activations of some stage are not plain
     auto compute = [&](uint32_t st) {
         const uint8_t* base = lds + st % D * G::STAGE;
+        float most[TM];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) most[i] = 0.0f;
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
             bf16x8 b[TN];
 #pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                const uint32_t r = (wn * TN + j) * 32 + r32;
-                b[j] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(
-                                                      base + G::A_BYTES + (r * G::B_CPR + turned<G::B_CPR>(r, 4 * h + s)) * 16));
-            }
+            for (int j = 0; j < TN; ++j) b[j] = w_piece(base, j, s);
 #pragma unroll
             for (int i = 0; i < TM; ++i) {
-                const uint32_t r = (wm * TM + i) * 32 + r32;
-                const uint8_t* ap = base + r * G::A_CPR * 16;
                 if constexpr (XBF16) {
-                    const bf16x8 a = __builtin_bit_cast(
-                        bf16x8, *reinterpret_cast<const u32x4*>(ap + turned<G::A_CPR>(r, 4 * h + s) * 16));
+                    const uint32_t r = (wm * TM + i) * 32 + r32;
+                    const bf16x8 a = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(
+                                                                    base + r * G::A_CPR * 16 + turned<G::A_CPR>(r, 4 * h + s) * 16));
 #pragma unroll
                     for (int j = 0; j < TN; ++j)
                         sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b[j], sum[i][j], 0, 0, 0);
                 } else {
-                    const u32x4 v0 = *reinterpret_cast<const u32x4*>(ap + turned<G::A_CPR>(r, 8 * h + 2 * s) * 16);
-                    const u32x4 v1 = *reinterpret_cast<const u32x4*>(ap + turned<G::A_CPR>(r, 8 * h + 2 * s + 1) * 16);
+                    u32x4 v0, v1;
+                    x_piece(base, i, s, v0, v1);
                     bf16x8 hi, mid, lo;
-                    split3x8(v0, v1, hi, mid, lo);
+                    split3_finite(v0, v1, hi, mid, lo);
+                    take_most(v0, most[i]);
+                    take_most(v1, most[i]);
 #pragma unroll
-                    for (int j = 0; j < TN; ++j) {
-                        sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lo, b[j], sum[i][j], 0, 0, 0);
-                        sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(mid, b[j], sum[i][j], 0, 0, 0);
-                        sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(hi, b[j], sum[i][j], 0, 0, 0);
-                    }
+                    for (int j = 0; j < TN; ++j) mac3(i, j, hi, mid, lo, b[j]);
                 }
             }
         }
-    };
+        if constexpr (!XBF16) {
 #pragma unroll
-    for (int p = 0; p < D - 1; ++p)
-        if ((uint32_t)p < stages) issue(p);
-    for (uint32_t st = 0; st < stages; ++st) {
-        const uint32_t ahead = stages - 1 - st;  // stages issued after st, at most D - 2
-        if (ahead >= (uint32_t)(D - 2)) wait_vm<(D - 2) * G::LPS>();
-        else if (D > 3 && ahead == 1) wait_vm<(D > 3 ? 1 : 0) * G::LPS>();
-        else wait_vm<0>();
-        lds_barrier();
-        if (st + D - 1 < stages) issue(st + D - 1);
-        compute(st);
-        if (st % kFold == kFold - 1 || ahead == 0) {
-            mfma_drain();
+            for (int i = 0; i < TM; ++i) care |= !plain(most[i]);
+        }
+        if (st % kFold == kFold - 1 || st + 1 == stages) fold(1.0);
+    };
+    // the same with the careful split, the tiny lanes' values in a pass of their own
+    auto compute_careful = [&](uint32_t st) {
+        const uint8_t* base = lds + st % D * G::STAGE;
+        float most[TM];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            most[i] = 0.0f;
+#pragma unroll 1
+            for (uint32_t s = 0; s < 4; ++s) {
+                u32x4 v0, v1;
+                x_piece(base, i, s, v0, v1);
+                take_most(v0, most[i]);
+                take_most(v1, most[i]);
+            }
+        }
+#pragma unroll
+        for (int pass = 0; pass < 2; ++pass) {
+#pragma unroll 1
+            for (uint32_t s = 0; s < 4; ++s)
+#pragma unroll
+                for (int i = 0; i < TM; ++i) {
+                    u32x4 v0, v1;
+                    x_piece(base, i, s, v0, v1);
+                    bf16x8 hi, mid, lo;
+                    split3_pass(pass, all_tiny(most[i]), v0, v1, hi, mid, lo);
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) mac3(i, j, hi, mid, lo, w_piece(base, j, s));
+                }
+            fold(pass ? kTinyDown : 1.0);
+        }
+    };
+    auto walk = [&](auto&& step) {
+#pragma unroll
+        for (int p = 0; p < D - 1; ++p)
+            if ((uint32_t)p < stages) issue(p);
+        for (uint32_t st = 0; st < stages; ++st) {
+            const uint32_t ahead = stages - 1 - st;  // stages issued after st, at most D - 2
+            if (ahead >= (uint32_t)(D - 2)) wait_vm<(D - 2) * G::LPS>();
+            else if (D > 3 && ahead == 1) wait_vm<(D > 3 ? 1 : 0) * G::LPS>();
+            else wait_vm<0>();
+            lds_barrier();
+            if (st + D - 1 < stages) issue(st + D - 1);
+            step(st);
+        }
+    };
+    walk(compute);
+    if constexpr (!XBF16) {
+        if (workgroup_any<G::NW>(__any(care), reinterpret_cast<uint32_t*>(lds), wave)) {
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
-                        acc[i][j][r] += (double)sum[i][j][r];
+                        acc[i][j][r] = 0.0;
                         sum[i][j][r] = 0.0f;
                     }
+            walk(compute_careful);
         }
     }
 

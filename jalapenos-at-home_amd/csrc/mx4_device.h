@@ -64,14 +64,11 @@ __device__ __forceinline__ void split3_bf16(float v, __bf16& hi, __bf16& mid, __
     lo = (__bf16)r2;
 }
 
-// The three terms of eight finite values, packed as MFMA operands: 5.5
-// operations a value where split3_bf16 takes twice that (its care for inf and
-// NaN). Those show in `bad`, which becomes NaN (or stays NaN); the caller then
-// splits again with split3_bf16. (A term of a tiny value may be cut at
-// bf16's least subnormal, 2^-133.)
+// The three terms of eight finite values, packed as MFMA operands: 5 operations
+// a value where split3_bf16 takes twice that (its care for inf and NaN).
 __device__ __forceinline__ void split3_finite(const u32x4 lo4, const u32x4 hi4, bf16x8& hi, bf16x8& mid, bf16x8& lo,
-                                              float& bad) {
-    uint32_t h[4], m[4], l[4];
+                                              float* bad = nullptr) {
+    uint32_t h[4], m[4];
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
         uint32_t r[2], d[2];
@@ -83,33 +80,67 @@ __device__ __forceinline__ void split3_finite(const u32x4 lo4, const u32x4 hi4, 
             r[e] = __float_as_uint(r1);
             rest[e] = r1 - __uint_as_float(r[e] & 0xFFFF0000u);
             d[e] = u;
+            lo[2 * p + e] = (__bf16)rest[e];
         }
-        bad = __builtin_fmaf(rest[0], rest[1], bad);
+        if (bad) *bad = __builtin_fmaf(rest[0], rest[1], *bad);
         // the upper halves of a pair: element 2 p below element 2 p + 1
         h[p] = __builtin_amdgcn_perm(d[1], d[0], 0x07060302u);
         m[p] = __builtin_amdgcn_perm(r[1], r[0], 0x07060302u);
-        l[p] = __builtin_amdgcn_perm(__float_as_uint(rest[1]), __float_as_uint(rest[0]), 0x07060302u);
     }
     hi = __builtin_bit_cast(bf16x8, u32x4{h[0], h[1], h[2], h[3]});
     mid = __builtin_bit_cast(bf16x8, u32x4{m[0], m[1], m[2], m[3]});
-    lo = __builtin_bit_cast(bf16x8, u32x4{l[0], l[1], l[2], l[3]});
+}
+
+// The terms of any eight values, by split3_bf16.
+__device__ __forceinline__ void split3_careful(const u32x4 a, const u32x4 b, bf16x8& hi, bf16x8& mid, bf16x8& lo) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        __bf16 h, m, l;
+        split3_bf16(__uint_as_float(e < 4 ? a[e] : b[e - 4]), h, m, l);
+        hi[e] = h;
+        mid[e] = m;
+        lo[e] = l;
+    }
 }
 
 // The terms of eight values, finite or not: the wave takes the short form and,
-// where some lane has an inf or a NaN (or the check overflows), the careful one.
+// where some lane has an inf or a NaN (or the check, a NaN from either on,
+// overflows), the careful one.
 __device__ __forceinline__ void split3x8(const u32x4 a, const u32x4 b, bf16x8& hi, bf16x8& mid, bf16x8& lo) {
     float bad = 0.0f;
-    split3_finite(a, b, hi, mid, lo, bad);
-    if (__any(bad != bad)) {
+    split3_finite(a, b, hi, mid, lo, &bad);
+    if (__any(bad != bad)) split3_careful(a, b, hi, mid, lo);
+}
+
+// Values below 2^-110 lose bits as three bf16 terms, whose least is 2^-133. The
+// kernels for any width and for bf16 weights lose none all the same: where a lane
+// holds, in a step of the reduction, only such values (zeros apart), or an inf or
+// a NaN, they do their work again with the careful split and two passes a step.
+// The first pass has the other lanes' values, the second those tiny ones, 2^64
+// times as large (every bit of an f32 then fits, and no product overflows: 2^-36
+// times weights below 2^128), and adds 2^-64 of its sum. (Beside a value above
+// 2^-100 a tiny one's bits below 2^-133 are 2^-33 of that value.) `most` is the
+// largest magnitude of a lane's values in the step, NaN if one of them is.
+constexpr double kTinyDown = 0x1p-64;
+__device__ __forceinline__ void take_most(const u32x4 v, float& most) {  // two instructions
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            __bf16 h, m, l;
-            split3_bf16(__uint_as_float(e < 4 ? a[e] : b[e - 4]), h, m, l);
-            hi[e] = h;
-            mid[e] = m;
-            lo[e] = l;
-        }
+    for (int p = 0; p < 4; p += 2)
+        most = __builtin_elementwise_maximum(__builtin_fabsf(__uint_as_float(v[p])),
+                                             __builtin_elementwise_maximum(__builtin_fabsf(__uint_as_float(v[p + 1])), most));
+}
+__device__ __forceinline__ bool all_tiny(float most) { return (most != 0.0f) & (most < 0x1p-100f); }
+__device__ __forceinline__ bool plain(float most) {  // the short split has it
+    return (most == 0.0f) | ((most >= 0x1p-100f) & (most < __builtin_inff()));
+}
+// The terms of a pass's share of eight values; `tiny`: the lane's all_tiny.
+__device__ __forceinline__ void split3_pass(int pass, bool tiny, u32x4 a, u32x4 b, bf16x8& hi, bf16x8& mid, bf16x8& lo) {
+    const float scale = pass ? 0x1p64f : 1.0f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        a[e] = tiny == (pass != 0) ? __float_as_uint(__uint_as_float(a[e]) * scale) : 0u;
+        b[e] = tiny == (pass != 0) ? __float_as_uint(__uint_as_float(b[e]) * scale) : 0u;
     }
+    split3_careful(a, b, hi, mid, lo);
 }
 
 __device__ __forceinline__ uint64_t wave_max_u64(uint64_t m) {
@@ -313,6 +344,20 @@ __device__ __forceinline__ bool row_writer(uint32_t lane) {
 }
 
 // ---------------------------------------------------------------- LDS pipelines
+
+// Does any of the NW waves of the workgroup say so (each with one wave-wide
+// answer)? Over LDS that no wave has a use for any more, by the first barrier.
+template <int NW>
+__device__ __forceinline__ bool workgroup_any(bool mine, uint32_t* words, uint32_t wave) {
+    __syncthreads();
+    if (threadIdx.x % 64 == 0) words[wave] = mine;
+    __syncthreads();
+    uint32_t any = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) any |= words[w];
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(any) != 0;
+}
 
 // LDS barrier that does not wait for outstanding global loads (the next
 // stage's prefetch stays in flight across it).

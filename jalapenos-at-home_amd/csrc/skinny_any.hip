@@ -13,7 +13,8 @@
 //    share the order, so it changes nothing in the result;
 //  * a workgroup of TW waves takes T 16-row tiles at a time and walks K in
 //    slices of TW x NC chunks, NC adjacent ones a wave: the slice's activation
-//    fragments are loaded (f32: split into three bf16 terms, exact products)
+//    fragments are loaded (f32: split into three bf16 terms, exact products;
+//    a wave that met tiny or non-finite ones does the set again with care for them)
 //    once and used for all T tiles, whose sums stay in registers. The next
 //    slice's (or the next tiles') weights of tile t are loaded as soon as tile
 //    t's are used, so T tiles (or two slices) are in flight;
@@ -117,7 +118,7 @@ __global__ __launch_bounds__(64 * TW) void skinny_any_kernel(const void* __restr
     const __amdgpu_buffer_rsrc_t xr = rsrc(static_cast<const uint8_t*>(x) + (size_t)tok0 * k * XB, m * k * XB);
 
     // element of K that lane group gq's piece t of chunk c starts with
-    auto element = [&](uint32_t c, int t) { return 128 * c + (FP4 ? 32 * gq + 8 * t : 32 * t + 8 * gq); };
+    auto element = [](uint32_t gq, uint32_t c, int t) { return 128 * c + (FP4 ? 32 * gq + 8 * t : 32 * t + 8 * gq); };
 
     struct Unit {
         u32x4 w[NC][WL];
@@ -135,7 +136,8 @@ __global__ __launch_bounds__(64 * TW) void skinny_any_kernel(const void* __restr
         else return 64 * i + 8 * j + ((b + (j & ~1u)) & 7);
     };
     // the weights of slice `sl` of tile `tile` (tiles and slices past the end: zeros)
-    auto load = [&](uint32_t tile, uint32_t sl, Unit& u) {
+    auto load_at = [&](uint32_t lane, uint32_t tile, uint32_t sl, Unit& u) {
+        const uint32_t col = lane % 16, gq = lane / 16;
         const bool valid = tile < tiles;
         const Pick p = pick(g, tile);
         const uint32_t row0 = valid ? (tile - p.first) * 16 : 0;
@@ -164,13 +166,14 @@ __global__ __launch_bounds__(64 * TW) void skinny_any_kernel(const void* __restr
             for (int q = 0; q < NC; ++q)
 #pragma unroll
                 for (int t = 0; t < WL; ++t) {
-                    const uint32_t e = element(c0 + q, t);
+                    const uint32_t e = element(gq, c0 + q, t);
                     u.w[q][t] = __builtin_amdgcn_raw_buffer_load_b128(wr, e < k ? col * row_bytes + 2 * e : kPastEnd, 0,
                                                                       kStreamed);
                 }
         }
         __builtin_amdgcn_sched_barrier(0);
     };
+    auto load = [&](uint32_t tile, uint32_t sl, Unit& u) { load_at(lane, tile, sl, u); };
 
     // Activation fragments of the slice in use. f32: `raw` holds the next
     // slice's values on their way from memory (4096 x 4096 at 7 rows 10.6 -> 9.6
@@ -179,12 +182,13 @@ __global__ __launch_bounds__(64 * TW) void skinny_any_kernel(const void* __restr
     constexpr int H = XBF16 ? 1 : 2;  // 16-byte loads per piece
     u32x4 raw[XBF16 ? 1 : NC][4][MT][H];
     bf16x8 xa[NC][4][MT][XP];
-    auto x_piece = [&](uint32_t sl, int q, int t, int j, u32x4 (&out)[H]) {
-        const uint32_t e = element((sl * TW + wave) * NC + q, t);
+    auto x_piece_at = [&](uint32_t lane, uint32_t sl, int q, int t, int j, u32x4 (&out)[H]) {
+        const uint32_t col = lane % 16, e = element(lane / 16, (sl * TW + wave) * NC + q, t);
         const uint32_t off = e < k ? ((16 * j + col) * k + e) * XB : kPastEnd;
 #pragma unroll
         for (int h = 0; h < H; ++h) out[h] = __builtin_amdgcn_raw_buffer_load_b128(xr, off + 16 * h, 0, 0);
     };
+    auto x_piece = [&](uint32_t sl, int q, int t, int j, u32x4 (&out)[H]) { x_piece_at(lane, sl, q, t, j, out); };
     auto issue_x = [&](uint32_t sl) {
         if constexpr (XBF16) return;
 #pragma unroll
@@ -195,8 +199,9 @@ __global__ __launch_bounds__(64 * TW) void skinny_any_kernel(const void* __restr
                 for (int j = 0; j < MT; ++j) x_piece(sl, q, t, j, raw[XBF16 ? 0 : q][t][j]);
         __builtin_amdgcn_sched_barrier(0);
     };
+    bool care = false;  // f32: this lane's activations of some slice are not plain
     auto settle_x = [&](uint32_t sl) {
-        float bad = 0.0f;
+        float most = 0.0f;
 #pragma unroll
         for (int q = 0; q < NC; ++q)
 #pragma unroll
@@ -208,30 +213,24 @@ __global__ __launch_bounds__(64 * TW) void skinny_any_kernel(const void* __restr
                         x_piece(sl, q, t, j, v);
                         xa[q][t][j][0] = __builtin_bit_cast(bf16x8, v[0]);
                     } else {
-                        split3_finite(raw[q][t][j][0], raw[q][t][j][1], xa[q][t][j][0], xa[q][t][j][1], xa[q][t][j][2], bad);
+                        split3_finite(raw[q][t][j][0], raw[q][t][j][1], xa[q][t][j][0], xa[q][t][j][1], xa[q][t][j][2]);
+                        take_most(raw[q][t][j][0], most);
+                        take_most(raw[q][t][j][1], most);
                     }
                 }
         if constexpr (!XBF16) {
-            if (__any(bad != bad)) {
-                // an inf or a NaN (or an overflow of the check itself): the
-                // careful split, on values loaded again rather than kept
+            // (zeros for what is done again anyway: without this branch the compiler
+            // takes more registers than there are with four tiles of bf16 weights)
+            if (__any(!plain(most))) {
+                care = true;
 #pragma unroll
                 for (int q = 0; q < NC; ++q)
 #pragma unroll
                     for (int t = 0; t < 4; ++t)
 #pragma unroll
-                        for (int j = 0; j < MT; ++j) {
-                            u32x4 v[H];
-                            x_piece(sl, q, t, j, v);
+                        for (int j = 0; j < MT; ++j)
 #pragma unroll
-                            for (int e = 0; e < 8; ++e) {
-                                __bf16 hi, mid, lo;
-                                split3_bf16(__uint_as_float(v[e / 4][e % 4]), hi, mid, lo);
-                                xa[q][t][j][0][e] = hi;
-                                xa[q][t][j][1][e] = mid;
-                                xa[q][t][j][2][e] = lo;
-                            }
-                        }
+                            for (int p = 0; p < 3; ++p) xa[q][t][j][p] = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
             }
         }
     };
@@ -309,6 +308,57 @@ __global__ __launch_bounds__(64 * TW) void skinny_any_kernel(const void* __restr
         }
     };
 
+    // the wave's sums of tile i of the set again, with the careful split and the
+    // tiny lanes' values in a pass of their own; everything is loaded again
+    auto again_with_care = [&](uint32_t tile, int i) {
+        if constexpr (!XBF16) {
+            static_assert(NC == 1 && MT == 1, "one chunk and one token tile of f32 activations");
+            // (opaque: what follows from it is computed here, not kept in registers
+            // over the sets)
+            uint32_t lane = threadIdx.x % 64;
+            asm volatile("" : "+v"(lane));
+            sums[i][0] = f64x4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll 1
+            for (uint32_t sl = 0; sl < slices; ++sl) {
+                Unit u;
+                load_at(lane, tile, sl, u);
+                float most = 0.0f, sc = 0.0f;
+#pragma unroll 1
+                for (int t = 0; t < 4; ++t) {
+                    u32x4 v[H];
+                    x_piece_at(lane, sl, 0, t, 0, v);
+                    take_most(v[0], most);
+                    take_most(v[1], most);
+                }
+                if constexpr (FP4) {
+                    const uint32_t blk = 4 * (sl * TW + wave) + lane / 16;
+                    sc = __uint_as_float((blk < nblk ? (u.s[0] >> u.shift) & 0xffu : 0u) << 23);
+                }
+#pragma unroll 1
+                for (int pass = 0; pass < 2; ++pass) {
+                    f32x4 whole{0.0f, 0.0f, 0.0f, 0.0f}, parts = whole;
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        bf16x8 b, hi, mid, lo;
+                        if constexpr (FP4) b = decode8(u.w[0][0][t], sc);
+                        else b = __builtin_bit_cast(bf16x8, u.w[0][t]);
+                        u32x4 v[H];
+                        x_piece_at(lane, sl, 0, t, 0, v);
+                        split3_pass(pass, all_tiny(most), v[0], v[1], hi, mid, lo);
+                        whole = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hi, b, whole, 0, 0, 0);
+                        parts = __builtin_amdgcn_mfma_f32_16x16x32_bf16(mid, b, parts, 0, 0, 0);
+                        parts = __builtin_amdgcn_mfma_f32_16x16x32_bf16(lo, b, parts, 0, 0, 0);
+                        __builtin_amdgcn_sched_barrier(0);  // one piece's registers at a time
+                    }
+                    mfma_drain();
+                    whole += parts;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) sums[i][0][r] += (double)whole[r] * (pass ? kTinyDown : 1.0);
+                }
+            }
+        }
+    };
+
     __shared__ f32x4 red[TW][T * MT][64];
     // tile i of the set that starts at `tile`; sets follow one another `grid` T tiles apart
     Unit u[D];
@@ -355,12 +405,26 @@ __global__ __launch_bounds__(64 * TW) void skinny_any_kernel(const void* __restr
             }
         }
         mfma_drain();
+#pragma unroll
+        for (int i = 0; i < T; ++i) fold(i);
+        if constexpr (!XBF16) {
+            if (__any(care)) {
+#pragma unroll
+                for (int i = 0; i < T; ++i) again_with_care(tile + i * grid, i);
+                // what the next set has a use for, loaded again rather than kept meanwhile
+                if constexpr (T > 1) {
+                    issue_x(0);
+                    if (slices == 1) settle_x(0);
+#pragma unroll
+                    for (int i = 0; i < T; ++i) load(next + i * grid, 0, u[i]);
+                }
+            }
+        }
         if (again) __syncthreads();  // the last set's sums have been read
 #pragma unroll
         for (int i = 0; i < T; ++i)
 #pragma unroll
             for (int j = 0; j < MT; ++j) {
-                if (j == 0) fold(i);
                 red[wave][i * MT + j][lane] = __builtin_convertvector(sums[i][j], f32x4);
             }
         __syncthreads();

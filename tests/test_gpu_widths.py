@@ -305,3 +305,48 @@ def test_explicit_team_keeps_a_default_that_fits(mx4, ctx, oracle, team):
             ctx.gemv_config(xb.ptr, xt, w, y.ptr, team, 1, teams, 0)
             assert_close(y.download(np.float32).reshape(1, n), ref, f"team={team} xt={xt} teams={teams}", scaled=True)
     w.release()
+
+
+# Largest distance of a row of outputs from the sum in 64 bits, relative to the
+# row's length. Products are exact and a chain of 32-bit additions is at most 24
+# long (three terms of eight MFMAs), then continues in 64 bits: measured 0.5 to
+# 1.3e-7 (2^-24 is 0.6e-7). One chain over K or a lost third term shows as 4e-7
+# and more.
+ROW_TOL = 2.5e-7
+
+
+def check_rows(out, x, w, what, tol=ROW_TOL):
+    """Every token row of out against x . w^T in 64 bits."""
+    ref = x.astype(np.float64) @ w.astype(np.float64).T
+    err = np.linalg.norm(out.astype(np.float64) - ref, axis=1) / np.linalg.norm(ref, axis=1)
+    assert np.all(err <= tol), f"{what}: row {int(np.argmax(err))} of {len(err)}: {np.max(err):.2e}"
+
+
+def tiny_rows(rng, m, k, exponent):
+    """f32 activations of size 2^-20 but for a few token rows: the first and the
+    last all of size 2^exponent, the second that in every other run of 64."""
+    x = np.ldexp(rng.standard_normal((m, k)), -20)
+    small = np.ldexp(rng.standard_normal((m, k)), exponent)
+    x[0], x[-1] = small[0], small[-1]
+    x[1, np.arange(k) // 64 % 2 == 0] = small[1, np.arange(k) // 64 % 2 == 0]
+    return x.astype(np.float32)
+
+
+@pytest.mark.parametrize("exponent", [-100, -112, -118, -126, -140])
+@pytest.mark.parametrize("m,n,k", [(2, 50, 416), (9, 4200, 992), (16, 8300, 160), (29, 70, 1600), (23, 600, 2048),
+                                   (40, 130, 352), (77, 70, 1632), (200, 320, 1600)])
+def test_tiny_f32_activations(mx4, ctx, oracle, m, n, k, exponent):
+    """Activations down to subnormal ones keep all their bits on the kernels for
+    any width (and f32 verify steps of the tuned ones) and for bf16 weights."""
+    rng = np.random.default_rng(m + n - exponent)
+    up = min(120 - exponent, 245)
+    packed = rng.integers(0, 256, (n, k // 2), dtype=np.uint8)
+    scales = rng.integers(up - 3, up + 1, (n, k // 32)).astype(np.uint8)
+    bits = (f32_bits(np.ldexp(rng.standard_normal((n, k)), up - 127).astype(np.float32)) >> 16).astype(np.uint16)
+    x = tiny_rows(rng, m, k, exponent)
+    xb, y = ctx.to_device(x), ctx.buffer(m * n * 4)
+    for what, w, values in (("mxfp4", wrapped(ctx, packed, scales, 1), oracle.dequantize(packed, scales)),
+                            ("bf16", ctx.upload_weight_bf16(bits, n, k), oracle.bf16_to_f32(bits))):
+        ctx.matmul(xb, mx4.F32, m, w, y)
+        check_rows(y.download(np.float32).reshape(m, n), x, values, f"{what} m={m} n={n} k={k} 2^{exponent}")
+        w.release()
