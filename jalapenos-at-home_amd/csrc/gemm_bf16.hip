@@ -215,6 +215,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_kernel(const void* __r
         if (st % kFold == kFold - 1 || st + 1 == stages) fold(1.0);
     };
     // the same with the careful split, the tiny lanes' values in a pass of their own
+    bool nan_lane[TM];  // this lane's token row holds a NaN
+#pragma unroll
+    for (int i = 0; i < TM; ++i) nan_lane[i] = false;
     auto compute_careful = [&](uint32_t st) {
         const uint8_t* base = lds + st % D * G::STAGE;
         float most[TM];
@@ -228,6 +231,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_kernel(const void* __r
                 take_most(v0, most[i]);
                 take_most(v1, most[i]);
             }
+            nan_lane[i] |= most[i] != most[i];
         }
 #pragma unroll
         for (int pass = 0; pass < 2; ++pass) {
@@ -281,30 +285,33 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_bf16_kernel(const void* __r
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-            const uint32_t col = col0 + (wn * TN + j) * 32 + r32;
+            const uint32_t tile_row = row0 + (wm * TM + i) * 32, tile_col = col0 + (wn * TN + j) * 32, col = tile_col + r32;
+            uint64_t nan_rows = 0, doubt = 0;  // NaN activations by token row; columns with a NaN beside those
+            if constexpr (!XBF16) {
+                nan_rows = __ballot(nan_lane[i]);
+                nan_rows |= nan_rows >> 32;
+            }
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const uint32_t row = row0 + (wm * TM + i) * 32 + 8 * (r / 4) + 4 * h + r % 4;
-                float v = (float)acc[i][j][r];
-                if constexpr (!XBF16) {
-                    // An inf weight times a zero mid or lo term is a NaN that
-                    // the reference's product of the whole value is not: what
-                    // came out as NaN is summed again from whole values, by
-                    // the wave, one output after the other.
-                    uint64_t todo = __ballot(v != v && row < m && col < n);
-                    while (todo) {
-                        const uint32_t l = (uint32_t)__builtin_ctzll(todo);
-                        todo &= todo - 1;
-                        const uint32_t rr = row - 4 * h + 4 * (l / 32), cc = col - r32 + l % 32;
-                        const float* xrow = static_cast<const float*>(x) + (size_t)rr * k + k0;
-                        const uint16_t* wrow = w + (size_t)cc * k + k0;
-                        float p = 0.0f;
-                        for (uint32_t e = lane; e < klen; e += 64) p = __builtin_fmaf(xrow[e], bf16_bits_to_f32(wrow[e]), p);
-                        p = wave_sum(p);
-                        if (lane == l) v = p;
+                const uint32_t at = 8 * (r / 4) + 4 * h + r % 4, row = tile_row + at;
+                const float v = (float)acc[i][j][r];
+                if constexpr (!XBF16) doubt |= __ballot(v != v && row < m && col < n && !((nan_rows >> at) & 1));
+                if (row < m && col < n) y[(size_t)row * n + col] = v;
+            }
+            if constexpr (!XBF16) {
+                doubt = (doubt | doubt >> 32) & 0xffffffffu;
+                if (doubt) wait_vm<0>();  // the sums below overwrite
+                while (doubt) {
+                    const uint32_t cc = tile_col + (uint32_t)__builtin_ctzll(doubt);
+                    doubt &= doubt - 1;
+                    const uint16_t* wrow = w + (size_t)cc * k + k0;
+                    if (!inf_and_no_nan(wrow, klen, lane)) continue;
+                    for (uint32_t at = 0; at < 32 && tile_row + at < m; ++at) {
+                        if ((nan_rows >> at) & 1) continue;
+                        const float p = dot_whole(static_cast<const float*>(x) + (size_t)(tile_row + at) * k + k0, wrow, klen, lane);
+                        if (lane == 0) y[(size_t)(tile_row + at) * n + cc] = p;
                     }
                 }
-                if (row < m && col < n) y[(size_t)row * n + col] = v;
             }
         }
 }

@@ -343,6 +343,44 @@ __device__ __forceinline__ bool row_writer(uint32_t lane) {
     return (lane & ~row_bits) == 0;
 }
 
+// ---------------------------------------------------------------- inf weights
+
+// bf16 weights and f32 activations: an inf weight times a zero middle or low term
+// is a NaN that the reference's product of the whole value is not. An output that
+// came out as NaN is summed again from whole values, but only where that can be
+// the reason (its token row has no NaN, and its weight row an inf and no NaN):
+// summing every NaN again, one output after the other, made a call whose
+// activations held one take a hundred times as long. Rows of whole 16-byte pieces.
+__device__ __forceinline__ bool inf_and_no_nan(const uint16_t* w, uint32_t len, uint32_t lane) {
+    bool inf = false, nan = false;
+#pragma unroll 4
+    for (uint32_t e = 8 * lane; e < len; e += 512) {
+        const u32x4 v = load_u32x4(reinterpret_cast<const uint8_t*>(w + e));
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            const uint32_t a = v[d] & 0x7fffu, b = (v[d] >> 16) & 0x7fffu;
+            inf |= (a == 0x7f80u) | (b == 0x7f80u);
+            nan |= (a > 0x7f80u) | (b > 0x7f80u);
+        }
+    }
+    return __any(inf) && !__any(nan);
+}
+__device__ __forceinline__ float dot_whole(const float* x, const uint16_t* w, uint32_t len, uint32_t lane) {
+    float p = 0.0f;
+#pragma unroll 2
+    for (uint32_t e = 8 * lane; e < len; e += 512) {
+        const u32x4 v = load_u32x4(reinterpret_cast<const uint8_t*>(w + e));
+        const f32x4 x0 = *reinterpret_cast<const f32x4*>(x + e), x1 = *reinterpret_cast<const f32x4*>(x + e + 4);
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+            const float a = d < 2 ? x0[2 * d] : x1[2 * d - 4], b = d < 2 ? x0[2 * d + 1] : x1[2 * d - 3];
+            p = __builtin_fmaf(a, bf16_bits_to_f32(v[d] & 0xffffu), p);
+            p = __builtin_fmaf(b, bf16_bits_to_f32(v[d] >> 16), p);
+        }
+    }
+    return wave_sum(p);
+}
+
 // ---------------------------------------------------------------- LDS pipelines
 
 // Does any of the NW waves of the workgroup say so (each with one wave-wide

@@ -308,6 +308,7 @@ __global__ __launch_bounds__(64 * TW) void skinny_any_kernel(const void* __restr
         }
     };
 
+    uint32_t nan_tokens = 0;  // bf16 weights: token rows with a NaN among the wave's activations
     // the wave's sums of tile i of the set again, with the careful split and the
     // tiny lanes' values in a pass of their own; everything is loaded again
     auto again_with_care = [&](uint32_t tile, int i) {
@@ -329,6 +330,10 @@ __global__ __launch_bounds__(64 * TW) void skinny_any_kernel(const void* __restr
                     x_piece_at(lane, sl, 0, t, 0, v);
                     take_most(v[0], most);
                     take_most(v[1], most);
+                }
+                if constexpr (!FP4) {
+                    const uint64_t nan = __ballot(most != most);
+                    nan_tokens |= (uint32_t)(nan | nan >> 16 | nan >> 32 | nan >> 48) & 0xffffu;
                 }
                 if constexpr (FP4) {
                     const uint32_t blk = 4 * (sl * TW + wave) + lane / 16;
@@ -360,6 +365,8 @@ __global__ __launch_bounds__(64 * TW) void skinny_any_kernel(const void* __restr
     };
 
     __shared__ f32x4 red[TW][T * MT][64];
+    constexpr bool INF = !FP4 && !XBF16;  // inf weights want a second look (inf_and_no_nan)
+    __shared__ uint32_t nans[INF ? TW : 1];
     // tile i of the set that starts at `tile`; sets follow one another `grid` T tiles apart
     Unit u[D];
     uint32_t tile = blockIdx.x;
@@ -425,6 +432,8 @@ __global__ __launch_bounds__(64 * TW) void skinny_any_kernel(const void* __restr
         for (int i = 0; i < T; ++i)
 #pragma unroll
             for (int j = 0; j < MT; ++j) {
+                if constexpr (INF)
+                    if (i == 0 && lane == 0) nans[wave] = nan_tokens;
                 red[wave][i * MT + j][lane] = __builtin_convertvector(sums[i][j], f32x4);
             }
         __syncthreads();
@@ -436,33 +445,35 @@ __global__ __launch_bounds__(64 * TW) void skinny_any_kernel(const void* __restr
             if (at < tiles) {
                 const Pick p = pick(g, at);
                 const uint32_t row = (at - p.first) * 16 + col;
-                if constexpr (!FP4 && !XBF16) {
-                    // An inf weight times a zero mid or lo term is a NaN that
-                    // the reference's product of the whole value is not: what
-                    // came out as NaN is summed again from whole values, by
-                    // the wave, one output after the other.
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        uint64_t todo = __ballot(sum[r] != sum[r] && row < p.n && 16 * j + 4 * gq + r < m);
-                        while (todo) {
-                            const uint32_t l = (uint32_t)__builtin_ctzll(todo);
-                            todo &= todo - 1;
-                            const uint32_t rr = (at - p.first) * 16 + l % 16, tok = tok0 + 16 * j + 4 * (l / 16) + r;
-                            const uint16_t* wr = reinterpret_cast<const uint16_t*>(p.data) + (size_t)rr * k;
-                            const float* xrow = static_cast<const float*>(x) + (size_t)tok * k;
-                            float part = 0.0f;
-                            for (uint32_t e = lane; e < k; e += 64)
-                                part = __builtin_fmaf(xrow[e], bf16_bits_to_f32(wr[e]), part);
-                            part = wave_sum(part);
-                            if (lane == l) sum[r] = (double)part;
-                        }
-                    }
-                }
                 if (row < p.n) {
 #pragma unroll
                     for (int r = 0; r < 4; ++r) {
                         const uint32_t tok = 16 * j + 4 * gq + r;
                         if (tok < m) p.y[(size_t)(tok0 + tok) * p.n + row] = (float)sum[r];
+                    }
+                }
+                if constexpr (INF) {
+                    uint32_t nan_rows = 0;  // token rows with a NaN; weight rows with one beside those
+#pragma unroll
+                    for (int w = 0; w < TW; ++w) nan_rows |= nans[w];
+                    uint64_t doubt = 0;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        doubt |= __ballot(sum[r] != sum[r] && row < p.n && 4 * gq + r < m && !((nan_rows >> (4 * gq + r)) & 1));
+                    doubt = (doubt | doubt >> 16 | doubt >> 32 | doubt >> 48) & 0xffffu;
+                    if (doubt) wait_vm<0>();  // the sums below overwrite
+                    uint32_t lane = threadIdx.x % 64;
+                    asm volatile("" : "+v"(lane));  // (its addresses are not for keeping, see above)
+                    while (doubt) {
+                        const uint32_t rr = (at - p.first) * 16 + (uint32_t)__builtin_ctzll(doubt);
+                        doubt &= doubt - 1;
+                        const uint16_t* wrow = reinterpret_cast<const uint16_t*>(p.data) + (size_t)rr * k;
+                        if (!inf_and_no_nan(wrow, k, lane)) continue;
+                        for (uint32_t tok = 0; tok < m; ++tok) {
+                            if ((nan_rows >> tok) & 1) continue;
+                            const float whole = dot_whole(static_cast<const float*>(x) + (size_t)(tok0 + tok) * k, wrow, k, lane);
+                            if (lane == 0) p.y[(size_t)(tok0 + tok) * p.n + rr] = whole;
+                        }
                     }
                 }
             }

@@ -350,3 +350,68 @@ def test_tiny_f32_activations(mx4, ctx, oracle, m, n, k, exponent):
         ctx.matmul(xb, mx4.F32, m, w, y)
         check_rows(y.download(np.float32).reshape(m, n), x, values, f"{what} m={m} n={n} k={k} 2^{exponent}")
         w.release()
+
+
+@pytest.mark.parametrize("m,n,k", [(5, 100, 264), (29, 5000, 1032), (40, 70, 264), (150, 200, 1608)])
+def test_bf16_inf_weight_rows(mx4, ctx, oracle, m, n, k):
+    """Weight rows with infs beside token rows with a NaN, an inf or both signs
+    of inf: every output is what the reference's loop gives."""
+    rng = np.random.default_rng(m + n)
+    w = (rng.standard_normal((n, k)) * 0.1).astype(np.float32)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[:, 8] = 1.0  # a value whose lower bf16 terms are zero
+    w[3, 8], w[n - 1, [8, 9]], w[20, k - 1] = np.inf, [-np.inf, np.inf], np.nan
+    x[1, 17], x[m - 1, k - 2] = np.nan, np.inf
+    x[2, [30, 31]] = [np.inf, -np.inf]
+    bits = (f32_bits(w) >> 16).astype(np.uint16) | (np.isnan(w) * 0x40).astype(np.uint16)
+    weight = ctx.upload_weight_bf16(bits, n, k)
+    y = ctx.buffer(m * n * 4)
+    ctx.matmul(ctx.to_device(x), mx4.F32, m, weight, y)
+    out = y.download(np.float32).reshape(m, n)
+    with np.errstate(all="ignore"):
+        ref = oracle.matmul_bf16(x, bits)
+    assert np.array_equal(np.isnan(out), np.isnan(ref))
+    assert np.array_equal(np.isposinf(out), np.isposinf(ref)) and np.array_equal(np.isneginf(out), np.isneginf(ref))
+    ok = np.isfinite(ref)
+    assert np.all(np.abs(out[ok].astype(np.float64) - ref[ok]) <= 1e-3 + 1e-5 * np.abs(ref[ok].astype(np.float64)))
+    weight.release()
+
+
+@pytest.mark.parametrize("kind", ["nan", "infs", "nan weights", "tiny"])
+@pytest.mark.parametrize("m", [16, 64])
+def test_odd_values_cost_no_more_than_a_few_calls(mx4, ctx, m, kind):
+    """Activations or bf16 weights full of NaNs, infs or subnormals take a small
+    multiple of the usual call (at most two passes over everything, the weights
+    read up to three times over; once every NaN was summed again by itself, a
+    hundred times the usual)."""
+    rng = np.random.default_rng(m)
+    n, k = 2048, 4096
+    w = (rng.standard_normal((n, k)) * 0.02).astype(np.float32)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    odd_w, odd_x = w, x
+    if kind == "nan":
+        odd_x = np.full_like(x, np.nan)
+    elif kind == "infs":
+        odd_x = x.copy()
+        odd_x[:, 100:110] = np.inf
+    elif kind == "nan weights":
+        odd_w = np.full_like(w, np.nan)
+    else:
+        odd_x = np.ldexp(x, -130).astype(np.float32)
+    times = []
+    for ww, xx in ((w, x), (odd_w, odd_x)):
+        bits = (f32_bits(ww) >> 16).astype(np.uint16)
+        weight = ctx.upload_weight_bf16(bits, n, k)
+        xb, y = ctx.to_device(xx), ctx.buffer(m * n * 4)
+        step = ctx.record(lambda: [ctx.matmul(xb, mx4.F32, m, weight, y) for _ in range(8)])
+        step.launch()
+        runs = []
+        for _ in range(5):
+            ctx.timer_begin()
+            step.launch()
+            runs.append(ctx.timer_end())
+        times.append(sorted(runs)[2])
+        step.release()
+        weight.release()
+    print(f"m={m} {kind}: {times[0] / 8 * 1e3:.1f} -> {times[1] / 8 * 1e3:.1f} us", flush=True)
+    assert times[1] <= 25 * times[0], (m, kind, times)
