@@ -8,8 +8,9 @@
 // reference's sequential loop is the summation order.
 //
 // One token row (decode): bf16_gemv_kernel streams the weights, up to four
-// matrices that share x in a launch. Two to 32 rows run skinny_any.hip. The
-// rest, and rows that are not whole 16-byte pieces:
+// matrices that share x in a launch. Two to 32 rows run skinny_any.hip, more
+// gemm_bf16.hip. Small weights, where those leave most of the chip idle
+// (bf16_rows_faster, bf16_matmul_us), and rows that are not whole 16-byte pieces:
 //
 // One wave per weight row, MT tokens per wave: each lane streams 16-byte
 // pieces (8 weights) of the row, fully coalesced, and reuses each piece for the
@@ -280,6 +281,41 @@ hipError_t launch_bf16_gemv(const uint16_t* const* w, float* const* y, const uin
     grid = (rows + each * 8 - 1) / (each * 8);
     if (k <= 1024) return x_bf16 ? go_gemv<true, 2>(g, x, k, rows, grid, s) : go_gemv<false, 2>(g, x, k, rows, grid, s);
     return x_bf16 ? go_gemv<true, 4>(g, x, k, rows, grid, s) : go_gemv<false, 4>(g, x, k, rows, grid, s);
+}
+
+// Two to 32 token rows: the row-per-wave kernel has n waves for every four of
+// them, skinny_any.hip a workgroup of eight for every 16 weight rows; it reads
+// the weights once, which pays where they are long. From a sweep of 16 to 16384
+// weight rows, K = 256 .. 12288 and 2 to 32 token rows on MI355X (cold weights,
+// recorded passes; no call is more than 8% slower than the other kernel would be,
+// where skinny_any alone took up to 2.9 times as long), us, this one / skinny_any:
+//  * bf16 x: 2048 x 2048 at 4 rows 5.5 / 6.0, 4096 x 2048 7.4 / 6.8, 4096 x 4096
+//    11.9 / 12.3; 1024 x 4096 at 16 rows 9.3 / 11.6, 2048 x 4096 15.2 / 12.2; 512
+//    x 8192 at 32 rows 13.6 / 26.1, 1024 x 8192 25.2 / 26.6. Up to four rows it
+//    reads the weights once too: short rows stay here at any number of them
+//    (16384 x 512 8.6 / 9.6);
+//  * f32 x: 2048 x 2048 at 4 rows 5.7 / 7.8, 4096 x 2048 10.7 / 8.7; 2048 x 1024
+//    at 8 rows 5.1 / 5.6; 1024 x 4096 at 16 rows 13.5 / 16.2, 2048 x 4096 22.9 /
+//    16.7; 512 x 4096 at 32 rows 11.2 / 15.9, 1024 x 4096 21.7 / 16.1.
+bool bf16_rows_faster(uint32_t m, uint32_t n, uint32_t k, bool x_bf16, int cus) {
+    const uint64_t four = (m + 3) / 4, waves = (uint64_t)n * four;
+    if (x_bf16 && m <= 4 && k <= 512) return true;
+    uint64_t most = x_bf16 ? 3072 + 640 * four : 2560 + 384 * four;
+    if (x_bf16 && m <= 4 && k >= 4096) most = 4096;
+    if (!x_bf16 && k <= 2048) most = most * (k <= 512 ? 6 : 5) / 4;
+    if (k <= 256 && most > (x_bf16 ? 3584u : 6144u)) most = x_bf16 ? 3584 : 6144;
+    return waves * 256 <= most * (uint64_t)(cus > 0 ? cus : 256);
+}
+
+// Estimated time of the row-per-wave kernel for more than a few token rows: its
+// waves at the rate they are launched at or, from K = 780 (f32 x: 510) on, at that
+// of their products (within 10% of 1.4 thousand measured calls near where the
+// matrix cores take over: 640 x 1024 at 33 / 300 rows 5.0 / 30 us, 128 x 12288 at
+// 128 rows of f32 29).
+double bf16_matmul_us(uint32_t m, uint32_t n, uint32_t k, bool x_bf16, int cus) {
+    const double waves = (double)n * ((m + 3) / 4) * 256.0 / (cus > 0 ? cus : 256);
+    const double each = (x_bf16 ? 3.6e-7 : 5.5e-7) * k;
+    return 2.2 + waves * (each > 2.8e-4 ? each : 2.8e-4);
 }
 
 hipError_t launch_bf16_matmul(const uint16_t* w, const void* x, bool x_bf16, float* y, uint32_t m, uint32_t n,

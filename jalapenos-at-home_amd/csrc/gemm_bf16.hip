@@ -337,52 +337,61 @@ hipError_t go(Weights g, const void* x, uint32_t m, uint32_t k, uint32_t ks, flo
     return launch_split_sum(part, ks, m * g.n[0], g.y[0], s);
 }
 
+// The tile and K split (1 to 4 slices, one weight) with the least estimated
+// time: whole rounds of workgroups, one per CU, times the tile's time for its
+// stages, plus the pass that adds the slices. Stage times from a sweep of nine
+// wave arrangements and 1-4 slices on the 1.7B and 8B shapes and 1600 x 4288 at
+// 40 .. 800 rows on MI355X (cold weights). Eight waves, two a SIMD, so that one
+// adds its 64-bit sums while the other multiplies: 128 x 128 with four waves of
+// 2 x 2 tiles ran 24576 x 4096 at 200 rows in 152 us, eight of 1 x 2 in 94, 128 x
+// 256 with eight of 2 x 2 in 80; 2048 x 6144 at 200 rows 18.9 us (128 x 64, four
+// slices).
+struct Plan {
+    int tile = 0;
+    uint32_t ks = 1;
+    double us = 0.0;
+};
+Plan plan(const uint32_t* n, uint32_t count, uint32_t m, uint32_t k, bool x_bf16, int cus, uint64_t part_bytes) {
+    struct Cand { int bm, bn; double stage_us; };
+    const Cand cands[] = {{128, 128, x_bf16 ? 0.65 : 1.64}, {64, 128, x_bf16 ? 0.43 : 1.2}, {128, 64, x_bf16 ? 0.41 : 1.28},
+                          {64, 64, x_bf16 ? 0.42 : 1.04}, {128, 256, 1.19}};
+    const int count_c = x_bf16 ? 5 : 4;  // (128 x 256 of f32 activations does not fit the registers)
+    const uint64_t nc = (uint64_t)(cus > 0 ? cus : 256);
+    Plan best;
+    for (int c = 0; c < count_c; ++c) {
+        uint64_t tiles = 0;
+        for (uint32_t q = 0; q < count; ++q) tiles += (n[q] + cands[c].bn - 1) / cands[c].bn;
+        tiles *= (m + cands[c].bm - 1) / cands[c].bm;
+        for (uint32_t ks = 1; ks <= 4; ++ks) {
+            if (ks > 1 && (count > 1 || (uint64_t)(ks - 1) * slice_k(k, ks) >= k || (uint64_t)ks * m * n[0] * 4 > part_bytes))
+                continue;
+            const double t = (double)((tiles * ks + nc - 1) / nc) * (4.0 + cands[c].stage_us * (slice_k(k, ks) / kBK)) +
+                             (ks > 1 ? 3.0 + 4.0 * (ks + 1) * m * n[0] / 4e6 : 0.0);
+            if (best.us == 0.0 || t < best.us) best = {c, ks, t};
+        }
+    }
+    return best;
+}
+
 template <bool XBF16>
 hipError_t dispatch(const Weights& g, const void* x, uint32_t m, uint32_t k, int cus, float* part, uint64_t part_bytes,
                     hipStream_t s) {
-    // The tile and K split (1 to 4 slices, one weight) with the least
-    // estimated time: whole rounds of workgroups, one per CU, times the
-    // tile's time for its stages, plus the pass that adds the slices. Stage
-    // times from a sweep of nine wave arrangements and 1-4 slices on the 1.7B
-    // and 8B shapes and 1600 x 4288 at 40 .. 800 rows on MI355X (cold weights).
-    // Eight waves, two a SIMD, so that one adds its 64-bit sums while the other
-    // multiplies: 128 x 128 with four waves of 2 x 2 tiles ran 24576 x 4096 at
-    // 200 rows in 152 us, eight of 1 x 2 in 94, 128 x 256 with eight of 2 x 2
-    // in 80; 2048 x 6144 at 200 rows 18.9 us (128 x 64, four slices).
-    struct Cand { int bm, bn; double stage_us; };
-    const Cand cands[] = {{128, 128, XBF16 ? 0.65 : 1.64}, {64, 128, XBF16 ? 0.43 : 1.2}, {128, 64, XBF16 ? 0.41 : 1.28},
-                          {64, 64, XBF16 ? 0.42 : 1.04}, {128, 256, 1.19}};
-    constexpr int kCands = XBF16 ? 5 : 4;  // (128 x 256 of f32 activations does not fit the registers)
-    const uint64_t nc = (uint64_t)(cus > 0 ? cus : 256);
-    int best = 0;
-    uint32_t best_ks = 1;
-    double best_t = 0.0;
-    for (int c = 0; c < kCands; ++c) {
-        uint64_t tiles = 0;
-        for (uint32_t q = 0; q < g.count; ++q) tiles += (g.n[q] + cands[c].bn - 1) / cands[c].bn;
-        tiles *= (m + cands[c].bm - 1) / cands[c].bm;
-        for (uint32_t ks = 1; ks <= 4; ++ks) {
-            if (ks > 1 && (g.count > 1 || !part || (uint64_t)(ks - 1) * slice_k(k, ks) >= k ||
-                           (uint64_t)ks * m * g.n[0] * 4 > part_bytes))
-                continue;
-            const double t = (double)((tiles * ks + nc - 1) / nc) * (4.0 + cands[c].stage_us * (slice_k(k, ks) / kBK)) +
-                             (ks > 1 ? 3.0 + 4.0 * (ks + 1) * m * g.n[0] / 4e6 : 0.0);
-            if (best_t == 0.0 || t < best_t) {
-                best = c;
-                best_ks = ks;
-                best_t = t;
-            }
-        }
-    }
+    const Plan p = plan(g.n, g.count, m, k, XBF16, cus, part ? part_bytes : 0);
     if constexpr (XBF16)
-        if (best == 4) return go<XBF16, 2, 4, 2, 2>(g, x, m, k, best_ks, part, s);
-    if (best == 0) return go<XBF16, 4, 2, 1, 2>(g, x, m, k, best_ks, part, s);
-    if (best == 1) return go<XBF16, 2, 4, 1, 1>(g, x, m, k, best_ks, part, s);
-    if (best == 2) return go<XBF16, 4, 2, 1, 1>(g, x, m, k, best_ks, part, s);
-    return go<XBF16, 2, 2, 1, 1>(g, x, m, k, best_ks, part, s);
+        if (p.tile == 4) return go<XBF16, 2, 4, 2, 2>(g, x, m, k, p.ks, part, s);
+    if (p.tile == 0) return go<XBF16, 4, 2, 1, 2>(g, x, m, k, p.ks, part, s);
+    if (p.tile == 1) return go<XBF16, 2, 4, 1, 1>(g, x, m, k, p.ks, part, s);
+    if (p.tile == 2) return go<XBF16, 4, 2, 1, 1>(g, x, m, k, p.ks, part, s);
+    return go<XBF16, 2, 2, 1, 1>(g, x, m, k, p.ks, part, s);
 }
 
 }  // namespace
+
+// Estimated time of a launch (measured ones are about 1.2 us shorter: small
+// weights at 33 .. 300 rows 1024 x 64 10.7 / 9.2 f32, 12288 x 64 27.2 / 26.5 bf16).
+double gemm_bf16_us(const uint32_t* n, uint32_t count, uint32_t m, uint32_t k, bool x_bf16, int cus, uint64_t part_bytes) {
+    return plan(n, count, m, k, x_bf16, cus, part_bytes).us - 1.2;
+}
 
 bool gemm_bf16_supported(uint32_t m, uint32_t n, uint32_t k, bool x_bf16) {
     // rows of whole 16-byte pieces; 32-bit offsets over the padded operands

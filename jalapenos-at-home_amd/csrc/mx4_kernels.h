@@ -106,6 +106,10 @@ hipError_t launch_gemm_exact(const GemvArgs& a, int cus, const GemmConfig* force
 // bf16 weights [n][k] (engine/src/lib.rs:255, None arm), any m, f32 accumulation.
 hipError_t launch_bf16_matmul(const uint16_t* w, const void* x, bool x_bf16, float* y, uint32_t m, uint32_t n,
                               uint32_t k, hipStream_t s);
+// 2 <= m <= 32 over one weight: does it beat launch_skinny_any? And its
+// estimated time in microseconds, for more rows (beside gemm_bf16_us).
+bool bf16_rows_faster(uint32_t m, uint32_t n, uint32_t k, bool x_bf16, int cus);
+double bf16_matmul_us(uint32_t m, uint32_t n, uint32_t k, bool x_bf16, int cus);
 
 // One token row over up to four bf16 weights of width k sharing x (16-byte
 // aligned): k % 8 == 0 and x within the LDS.
@@ -120,6 +124,7 @@ bool gemm_bf16_supported(uint32_t m, uint32_t n, uint32_t k, bool x_bf16);
 hipError_t launch_gemm_bf16(const uint16_t* const* w, float* const* y, const uint32_t* n, uint32_t count, const void* x,
                             bool x_bf16, uint32_t m, uint32_t k, int cus, float* part, uint64_t part_bytes,
                             hipStream_t s);
+double gemm_bf16_us(const uint32_t* n, uint32_t count, uint32_t m, uint32_t k, bool x_bf16, int cus, uint64_t part_bytes);
 // y = sum over ks slices of part[s] (count floats each), in slice order.
 hipError_t launch_split_sum(const float* part, uint32_t ks, uint32_t count, float* y, hipStream_t s);
 

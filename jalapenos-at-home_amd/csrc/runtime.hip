@@ -328,6 +328,19 @@ bool scales_foldable(const mx4_weight* w) { return w->min_scale >= 2 && w->max_s
 // call (rows of whole 16-byte pieces)?
 bool bf16_skinny(const mx4_weight* w, uint32_t m) { return w->bf16 && mx4::skinny_any_supported(m, w->cols, false); }
 
+// bf16 weights, more than 32 token rows: the matrix-core GEMM over these weights
+// in one launch, or the row-per-wave kernel over one after the other?
+bool bf16_gemm(const mx4_weight* const* w, uint32_t count, uint32_t m, bool x_bf16, int cus) {
+    uint32_t rows[4] = {};
+    double one_by_one = 0.0;
+    for (uint32_t i = 0; i < count; ++i) {
+        if (!w[i]->bf16 || !mx4::gemm_bf16_supported(m, w[i]->rows, w[0]->cols, x_bf16)) return false;
+        rows[i] = w[i]->rows;
+        one_by_one += mx4::bf16_matmul_us(m, rows[i], w[0]->cols, x_bf16, cus);
+    }
+    return m > 32 && mx4::gemm_bf16_us(rows, count, m, w[0]->cols, x_bf16, cus, kSplitPartBytes) <= one_by_one;
+}
+
 // Entry points that read the weight's stored row-major layout refuse a weight
 // whose layout was dropped (mx4_weight_drop_stored).
 mx4_status need_stored(const mx4_weight* w) {
@@ -347,10 +360,11 @@ mx4_status run_matmul(mx4_context* ctx, const void* x, mx4_dtype xt, uint32_t m,
         hipError_t e;
         if (path == MX4_PATH_AUTO && m == 1 && mx4::bf16_gemv_supported(w->cols, xt == MX4_BF16)) {
             e = mx4::launch_bf16_gemv(&w->bf16, &y, &w->rows, 1, x, xt == MX4_BF16, w->cols, ctx->cus, ctx->stream);
-        } else if (path == MX4_PATH_AUTO && m > 32 && mx4::gemm_bf16_supported(m, w->rows, w->cols, xt == MX4_BF16)) {
+        } else if (path == MX4_PATH_AUTO && bf16_gemm(&w, 1, m, xt == MX4_BF16, ctx->cus)) {
             e = mx4::launch_gemm_bf16(&w->bf16, &y, &w->rows, 1, x, xt == MX4_BF16, m, w->cols, ctx->cus, ctx->split_part,
                                       kSplitPartBytes, ctx->stream);
-        } else if (path == MX4_PATH_AUTO && bf16_skinny(w, m)) {
+        } else if (path == MX4_PATH_AUTO && bf16_skinny(w, m) &&
+                   !mx4::bf16_rows_faster(m, w->rows, w->cols, xt == MX4_BF16, ctx->cus)) {
             mx4::GemvArgs a{nullptr, nullptr, x, y, m, w->rows, w->cols, xt == MX4_BF16, ctx->stream};
             e = mx4::launch_skinny_any(a, &w->bf16, ctx->cus);
         } else {
@@ -882,10 +896,9 @@ mx4_status mx4_matmul_group(mx4_context* ctx, const void* x, mx4_dtype xt, uint3
     }
     // bf16 weights: one launch over all of them
     bool bf16_group = count > 1, bf16_one = m == 1 && mx4::bf16_gemv_supported(k, xt == MX4_BF16);
-    bool bf16_many = m > 32;
+    const bool bf16_many = bf16_gemm(w, count, m, xt == MX4_BF16, ctx->cus);
     for (uint32_t i = 0; i < count; ++i) {
         bf16_one &= w[i]->bf16 != nullptr;
-        bf16_many &= w[i]->bf16 != nullptr && mx4::gemm_bf16_supported(m, w[i]->rows, k, xt == MX4_BF16);
         bf16_group &= bf16_skinny(w[i], m);
     }
     if (bf16_one || bf16_many) {

@@ -377,6 +377,18 @@ def test_bf16_inf_weight_rows(mx4, ctx, oracle, m, n, k):
     weight.release()
 
 
+def call_us(ctx, call):
+    """Microseconds of a call, from recorded passes of sixteen."""
+    step = ctx.record(lambda: [call() for _ in range(16)])
+    runs = []
+    for _ in range(7):
+        ctx.timer_begin()
+        step.launch()
+        runs.append(ctx.timer_end())
+    step.release()
+    return sorted(runs)[3] / 16 * 1e3
+
+
 @pytest.mark.parametrize("kind", ["nan", "infs", "nan weights", "tiny"])
 @pytest.mark.parametrize("m", [16, 64])
 def test_odd_values_cost_no_more_than_a_few_calls(mx4, ctx, m, kind):
@@ -403,15 +415,28 @@ def test_odd_values_cost_no_more_than_a_few_calls(mx4, ctx, m, kind):
         bits = (f32_bits(ww) >> 16).astype(np.uint16)
         weight = ctx.upload_weight_bf16(bits, n, k)
         xb, y = ctx.to_device(xx), ctx.buffer(m * n * 4)
-        step = ctx.record(lambda: [ctx.matmul(xb, mx4.F32, m, weight, y) for _ in range(8)])
-        step.launch()
-        runs = []
-        for _ in range(5):
-            ctx.timer_begin()
-            step.launch()
-            runs.append(ctx.timer_end())
-        times.append(sorted(runs)[2])
-        step.release()
+        times.append(call_us(ctx, lambda: ctx.matmul(xb, mx4.F32, m, weight, y)))
         weight.release()
-    print(f"m={m} {kind}: {times[0] / 8 * 1e3:.1f} -> {times[1] / 8 * 1e3:.1f} us", flush=True)
+    print(f"m={m} {kind}: {times[0]:.1f} -> {times[1]:.1f} us", flush=True)
     assert times[1] <= 25 * times[0], (m, kind, times)
+
+
+def check_not_slower(mx4, ctx, w, m, k, n, what):
+    """The default path's time within a third of the general kernel's."""
+    y = ctx.buffer(m * n * 4)
+    for xt in (mx4.BF16, mx4.F32):
+        x = ctx.to_device(np.ones(m * k * (1 if xt == mx4.F32 else 2), np.float32 if xt == mx4.F32 else np.uint16))
+        auto, general = (call_us(ctx, lambda: ctx.matmul(x, xt, m, w, y, path)) for path in (mx4.PATH_AUTO, mx4.PATH_GENERIC))
+        print(f"{what} m={m} n={n} k={k} xt={xt}: {auto:.1f} us, general {general:.1f}", flush=True)
+        assert auto <= 1.33 * general + 0.5, (what, m, n, k, xt, auto, general)
+
+
+@pytest.mark.parametrize("n,k", [(16, 1024), (64, 4096), (64, 12288), (320, 1600), (640, 1024), (1024, 4096), (2048, 2048),
+                                 (4096, 4096)])
+@pytest.mark.parametrize("m", [2, 4, 8, 16, 32, 33, 64, 300])
+def test_bf16_small_weights_speed(mx4, ctx, m, n, k):
+    """Where the matrix cores would leave most of the chip idle, the row-per-wave
+    kernel runs: no call takes much longer than that one."""
+    w = ctx.upload_weight_bf16(np.full(n * k, 0x3c00, np.uint16), n, k)
+    check_not_slower(mx4, ctx, w, m, k, n, "bf16 weights")
+    w.release()
