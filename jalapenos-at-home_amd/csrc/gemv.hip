@@ -1203,6 +1203,33 @@ static hipError_t launch_generic_t(const GemvArgs& a) {
     return hipGetLastError();
 }
 
+// Widths off the tuned ones, one weight: does the generic kernel beat the
+// matrix cores' (skinny_any.hip up to 32 token rows, gemm.hip's any-width form
+// beyond)? They take the same time for one tile of weight rows as for a chip full
+// of them; its time is that of its waves, one for each weight row and four token
+// rows, in steps of 2048 of K. From a sweep of 16 to 8192 rows, K = 96 .. 12320, 1
+// to 300 token rows on MI355X (cold weights, recorded passes), us, this kernel /
+// the matrix cores:
+//  * bf16 x, 17 to 32 rows, K > 1024: 256 x 1600 at 32 rows 5.7 / 6.1, 256 x 8992
+//    18.1 / 20.5; 512 x 1600 7.5 / 6.2, 512 x 8992 25.5 / 21; beyond 32 rows 64 x
+//    1600 at 64 4.9 / 7.3, 256 x 1600 7.5 / 7.5, 64 x 8992 at 128 18.2 / 21.5, 256 x
+//    3264 at 64 11.8 / 10.8, 64 x 96 at 33 6.0 / 3.0;
+//  * f32 x, 12 to 32 rows, K > 1024: 256 x 1056 at 16 rows 6.2 / 7.5, 256 x 8992
+//    26 / 29; 512 x 8992 42 / 30 (rows that leave most of the last of several steps
+//    idle gain nothing: 256 x 4288 16.5 / 16.7, 16 x 4288 16.6 / 12.2); beyond 32 rows 64 x
+//    1600 at 33 6.8 / 11.0, 128 x 1600 at 64 9.7 / 11.5, 64 x 8992 at 64 26 / 39,
+//    128 x 8992 at 33 42 / 39.
+bool generic_faster(uint32_t m, uint32_t n, uint32_t k, bool x_bf16, int cus) {
+    const uint64_t waves = (uint64_t)n * ((m + 3) / 4) * 256 / (uint64_t)(cus > 0 ? cus : 256);
+    const uint32_t blocks = k / 32, steps = (blocks + 63) / 64;
+    if (m <= 32) {
+        if (k <= 1024) return false;
+        return x_bf16 ? m > 16 && waves <= 2048 : m > 11 && waves <= 1024 && (steps == 1 || 4 * blocks >= 3 * 64 * steps);
+    }
+    const bool one_full_step = k > 1024 && k <= 2048;
+    return k >= 448 && waves <= (x_bf16 ? 2048u : 1024u) * (one_full_step ? 2u : 1u);
+}
+
 hipError_t launch_gemv_generic(const GemvArgs& a) {
     if (a.m == 1) return a.x_bf16 ? launch_generic_t<true, 1>(a) : launch_generic_t<false, 1>(a);
     return a.x_bf16 ? launch_generic_t<true, 4>(a) : launch_generic_t<false, 4>(a);

@@ -53,6 +53,9 @@ bool gemv_mt_supported(uint32_t m, uint32_t k, bool x_bf16);
 // teams / tpw (teams per workgroup): 0 = the default launch shape.
 hipError_t launch_gemv_mt(const GemvArgs& a, int cus, uint32_t teams = 0, uint32_t tpw = 0);
 hipError_t launch_gemv_generic(const GemvArgs& a);
+// One weight of a width off the tuned ones, m >= 2: does it beat the kernels on the
+// matrix cores that take any width?
+bool generic_faster(uint32_t m, uint32_t n, uint32_t k, bool x_bf16, int cus);
 // M = 1 projection + greedy argmax epilogue (a.y may be null); hipErrorNotSupported
 // for configurations without the epilogue instance. partial: max_partials keys.
 hipError_t launch_gemv_m1_argmax(const GemvArgs& a, uint64_t* partial, uint32_t max_partials, uint32_t* idx,

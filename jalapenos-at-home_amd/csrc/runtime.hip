@@ -384,17 +384,19 @@ mx4_status run_matmul(mx4_context* ctx, const void* x, mx4_dtype xt, uint32_t m,
         const bool tokens = mx4::gemv_mt_supported(m, w->cols, xt == MX4_BF16) &&
                             ((m == 2 && w->rows < 65536) || (w->rows <= 1024 && w->cols >= 4096));
         // (asked for by name, the GEMV path takes its tuned widths only)
+        const bool tuned = m <= 32 ? mx4::skinny_supported(m, w->cols) : mx4::gemm_exact_supported(m, w->rows, w->cols, xt == MX4_BF16);
+        const bool small = m >= 2 && !tuned && mx4::generic_faster(m, w->rows, w->cols, xt == MX4_BF16, ctx->cus);
         const bool one = m == 1 && (mx4::gemv_m1_supported(w->cols) || mx4::gemv_any_supported(w->cols));
         if ((one || tokens) && scales_foldable(w))
             path = MX4_PATH_GEMV;
         else if (m >= 2 && mx4::skinny_supported(m, w->cols) && scales_foldable(w) &&
                  !mx4::skinny_any_faster(m, w->cols, (w->rows + 15) / 16, xt == MX4_BF16, ctx->cus))
             path = MX4_PATH_SKINNY;
-        else if (mx4::skinny_any_supported(m, w->cols, true) && scales_foldable(w)) {
+        else if (!small && mx4::skinny_any_supported(m, w->cols, true) && scales_foldable(w)) {
             path = MX4_PATH_SKINNY;  // (asked for by name, the path takes its tuned widths only)
             any_skinny = true;
         }
-        else if (m > 32 && mx4::gemm_any_supported(m, w->rows, w->cols, xt == MX4_BF16) && scales_foldable(w))
+        else if (!small && m > 32 && mx4::gemm_any_supported(m, w->rows, w->cols, xt == MX4_BF16) && scales_foldable(w))
             path = MX4_PATH_GEMM;  // (asked for by name, the path takes K % 128 == 0 only)
         else
             path = MX4_PATH_GENERIC;

@@ -440,3 +440,13 @@ def test_bf16_small_weights_speed(mx4, ctx, m, n, k):
     w = ctx.upload_weight_bf16(np.full(n * k, 0x3c00, np.uint16), n, k)
     check_not_slower(mx4, ctx, w, m, k, n, "bf16 weights")
     w.release()
+
+
+@pytest.mark.parametrize("n,k", [(16, 1600), (64, 480), (64, 8992), (128, 1600), (256, 3264), (256, 8992), (512, 1600),
+                                 (1024, 4288)])
+@pytest.mark.parametrize("m", [2, 8, 16, 32, 33, 64, 128, 300])
+def test_any_width_small_weights_speed(mx4, ctx, m, n, k):
+    """The same for widths off the tuned ones and the generic kernel."""
+    w = ctx.synth_weight(n + k, n, k)
+    check_not_slower(mx4, ctx, w, m, k, n, "any width")
+    w.release()
