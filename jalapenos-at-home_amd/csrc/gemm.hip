@@ -35,6 +35,7 @@
 //    workgroup that met tiny or non-finite ones walks K again with care for them
 //    (mx4_device.h): 1600 x 1600 at 77 rows 18.8 -> 13.5 us against a check (for
 //    non-finite ones only) at every eight values, other shapes within 3%.
+#include <algorithm>
 #include <type_traits>
 #include "mx4_device.h"
 #include "mx4_kernels.h"
@@ -359,7 +360,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_exact_kernel(const uint8_t*
         // (opaque: a second walk computes its offsets again, instead of the first
         // one's registers holding them)
         uint32_t lane = threadIdx.x % 64;
-        asm volatile("" : "+v"(lane));
+        if constexpr (ANY && !XBF16) asm volatile("" : "+v"(lane));
         // this lane's global offsets (stage 0) of its loads; LDS slot p = (q NW + wave) 64 + lane
         uint32_t a_goff[G::A_INSTR], b_goff[G::B_INSTR], s_goff[G::S_INSTR];
         uint32_t a_col[G::A_INSTR], b_col[G::B_INSTR];  // first element within the stage (ANY)
@@ -663,7 +664,15 @@ hipError_t launch_gemm_exact(const GemvArgs& a, int cus, const GemmConfig* force
         // CUs idle: one short round of them beats a split and the pass that
         // adds it (a small model's layer 28.0 against 30.3 us, 4096 wide at 48
         // rows 89.8 against 90.3), and its weights' separate launches.
+        // A split saves time with K and costs it with the outputs, so that a group
+        // cuts K only while its partials stay below 8 KiB for every element of K
+        // (two weights of 1536 x 512, f32 x, at 64 rows 10.7 -> 8.7 us with 3 MiB in
+        // four slices, at 200 and 300 rows 11.1 and 11.5 -> 13.0 and 20.5 with 5 and
+        // 14 MiB; 2048 + 512 + 512 x 2048 at 300 rows 33.8 -> 30.0 with 14 MiB) and,
+        // where the tiles are few, not into a second round of the CUs (768 + 192 +
+        // 192 x 768 at 300 rows 14.6 -> 15.5 us).
         const bool may_split = !(a.group && a.x_bf16 && a.k % kBK == 0);
+        if (a.group && part_bytes > 8192ull * a.k) part_bytes = 8192ull * a.k;
         uint32_t rows = a.n;  // weight rows, of all the group's weights
         if (a.group) {
             rows = 0;
@@ -724,7 +733,8 @@ hipError_t launch_gemm_exact(const GemvArgs& a, int cus, const GemmConfig* force
         const uint64_t tiles = (uint64_t)((a.m + pick.bm - 1) / pick.bm) * col_tiles(pick.bn);
         c.ks = 1;
         for (uint32_t ks = 4; ks >= 2 && tiles < want && may_split; --ks) {
-            if (slices_fit(a.k, ks) && part && (uint64_t)ks * a.m * rows * 4 <= kFewRowsSplitBytes) {
+            if (slices_fit(a.k, ks) && part && !(a.group && tiles * ks > nc) &&
+                (uint64_t)ks * a.m * rows * 4 <= std::min(part_bytes, kFewRowsSplitBytes)) {
                 c.ks = (int)ks;
                 break;
             }

@@ -450,3 +450,18 @@ def test_any_width_small_weights_speed(mx4, ctx, m, n, k):
     w = ctx.synth_weight(n + k, n, k)
     check_not_slower(mx4, ctx, w, m, k, n, "any width")
     w.release()
+
+
+def test_group_split_pays(mx4, ctx):
+    """A group of short rows and many outputs is not cut along K, where adding
+    the slices would cost more than it saves: well below its members, which are
+    cut."""
+    m, n, k = 300, 1536, 512
+    ws = [ctx.synth_weight(i, n, k) for i in (1, 2)]
+    x, ys = ctx.to_device(np.ones(m * k, np.float32)), [ctx.buffer(m * n * 4) for _ in ws]
+    group = call_us(ctx, lambda: ctx.matmul_group(x.ptr, mx4.F32, m, ws, [y.ptr for y in ys]))
+    apart = call_us(ctx, lambda: [ctx.matmul(x, mx4.F32, m, w, y) for w, y in zip(ws, ys)])
+    print(f"group {group:.1f} us, apart {apart:.1f}", flush=True)
+    assert group <= 0.75 * apart, (group, apart)
+    for w in ws:
+        w.release()
