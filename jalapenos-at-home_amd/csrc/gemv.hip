@@ -846,8 +846,9 @@ static void default_m1_config(uint32_t k, uint32_t rows, bool x_bf16, int cus, M
             // 4.37 -> 3.95 us)
             c.wg = 1; c.r = 1; c.tpw = x_bf16 ? 8 : 4;
             c.grid = (rows <= 4096 ? 8 : x_bf16 ? 32 : 16) * scale;
-            // gate|up: two rows, bf16 x not shared (4.7 against 5.0 us), f32 x by
-            // four teams (6.49 -> 5.56 us)
+            // gate|up: two rows, bf16 x not shared (4.7 against 5.0 us); shared by
+            // four teams with more rows (12289 / 24576 / 65536 rows 4.84 / 7.61 / 15.6
+            // -> 4.44 / 6.79 / 14.6 us) and with f32 x (6.49 -> 5.56)
             if (rows > 8192) { c.r = 2; c.tpw = x_bf16 && rows <= 12288 ? 1 : 4; c.grid = 16 * scale; }
             if (rows > 65536) { c.r = 4; c.tpw = 8; c.grid = 8 * scale; }  // vocabulary-sized
             break;
@@ -857,9 +858,10 @@ static void default_m1_config(uint32_t k, uint32_t rows, bool x_bf16, int cus, M
             // workgroup sharing x, fetched ahead of the weights
             if (rows <= 8192) { c.r = 1; c.grid = 8 * scale; c.tpw = 4; }
             if (rows > 8192) c.tpw = 8;
-            // up to 16384 rows (gate alone 7.02 -> 6.52 us), and with f32 x (gate
-            // 8.91 -> 6.95, gate|up 12.1 -> 11.4 us), one-row teams too
-            if (rows > 8192 && (rows <= 16384 || !x_bf16)) { c.r = 1; c.grid = (x_bf16 ? 32 : 16) * scale; c.tpw = 4; }
+            // up to 16384 rows (gate alone 7.02 -> 6.52 us), with f32 x up to 32768
+            // (gate 8.91 -> 6.95, gate|up 12.1 -> 11.4 us; 65536 rows 27.4 -> 28.4,
+            // so not there), one-row teams too
+            if (rows > 8192 && rows <= (x_bf16 ? 16384 : 32768)) { c.r = 1; c.grid = (x_bf16 ? 32 : 16) * scale; c.tpw = 4; }
             if (rows > 65536) { c.r = 2; c.wg = 2; c.grid = 8 * scale; c.tpw = 4; }  // vocabulary-sized
             break;
         case 192:  // K = 6144: four one-wave teams per workgroup sharing x,
@@ -1053,8 +1055,14 @@ hipError_t launch_gemv_m1_argmax(const GemvArgs& a, uint64_t* partial, uint32_t 
     if (any) {
         if (c.wg != 1) return hipErrorNotSupported;
     } else if (!am_compiled(c.wg, bpl, c.r) || c.tpw * c.wg > 8) {
-        // the one-wave vocabulary-sized configuration (4 rows, 4 teams per CU, 4 per workgroup)
-        c.wg = 1; c.r = 4; c.grid = 4 * (uint32_t)(cus > 0 ? cus : 256); c.tpw = 4;
+        // the one-wave vocabulary-sized configuration (4 rows, 4 teams per CU, 4 per
+        // workgroup): against two rows with a copy of x a team, K = 2048 at 5000 /
+        // 8192 / 32768 rows 6.6 / 8.0 / 15.2 -> 6.0 / 6.5 / 11.8 us, K = 4096 at 9000 /
+        // 12288 9.6 / 10.4 -> 9.1 / 10.1. At K = 4096 with more rows of bf16 x two rows
+        // and eight teams a workgroup (16384 rows 11.4 against 11.7 us).
+        const uint32_t scale = (uint32_t)(cus > 0 ? cus : 256);
+        c.wg = 1; c.r = 4; c.grid = 4 * scale; c.tpw = 4;
+        if (nblk == 128 && a.x_bf16 && a.n > 12288) { c.r = 2; c.grid = 16 * scale; c.tpw = 8; }
         bpl = (int)(nblk / 64);
         if (!am_compiled(c.wg, bpl, c.r)) return hipErrorNotSupported;
     }

@@ -546,15 +546,19 @@ bool skinny_any_supported(uint32_t m, uint32_t k, bool fp4) {
 }
 
 // The tuned widths (skinny.hip). f32 activations: skinny.hip splits a token's
-// values again for every 16-row tile, here once for up to four of them (8B gate|up
-// at 7 / 29 rows 48 / 110 against 32 / 64 us, o 10.4 / 20.4 against 9.9 / 17.5,
-// down 25.9 / 63 against 22.4 / 45; 1.7B gate|up 17.1 / 37.3 against 11.1 / 24.8).
-// At K = 2048 with a tile or less a CU and one token tile it stays ahead (1.7B
-// q|k|v 6.3 against 6.7 us). bf16 ones: up to 16 rows it stays ahead everywhere
-// (its activations are resident too); beyond, where its weights are too long for
-// one tile a workgroup and too short for the tile ring, it loads them for every
-// tile (1.7B gate|up 20.8 against 10.5 us, 8B q|k|v 20.9 against 13.2; with fewer
-// tiles 11.2 against 11.4, with the ring 26.7 against 32).
+// values again for every 16-row tile, here once for up to four of them (us,
+// skinny.hip / here: 8B gate|up at 7 / 29 rows 48 / 110 against 35 / 65, o 10.4 /
+// 20.4 against 9.8 / 17.1, down 25.9 / 63 against 23 / 48; 4096 x 6144 at 6 rows
+// 12.1 / 11.4, 4096 x 8192 15.9 / 15.0; 1.7B gate|up 17.1 / 37.3 against 11.1 /
+// 24.8). At K = 2048 with a tile or less a CU and one token tile it stays ahead
+// (1.7B q|k|v 6.3 against 6.7 us). It would at 11 to 16 rows there too (4096 rows,
+// K = 4096 / 6144 / 8192 / 12288 at 16 rows 14.3 / 21.4 / 24.7 / 39.4 against 16.3 /
+// 23.3 / 28.5 / 42.4), but its sums are two to four times as far from the exact
+// ones (2.2e-7 against 0.5 to 1.1e-7), so those stay here. bf16 ones: up to 16 rows
+// it stays ahead everywhere (its activations are resident too); beyond, where its
+// weights are too long for one tile a workgroup and too short for the tile ring, it
+// loads them for every tile (1.7B gate|up 20.8 against 10.5 us, 8B q|k|v 20.9
+// against 13.2; with fewer tiles 11.2 against 11.4, with the ring 26.7 against 32).
 bool skinny_any_faster(uint32_t m, uint32_t k, uint32_t tiles, bool x_bf16, int cus) {
     const uint32_t nc = (uint32_t)(cus > 0 ? cus : 256);
     if (!x_bf16) return m > 16 || k != 2048 || tiles > nc;

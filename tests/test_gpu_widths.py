@@ -142,6 +142,24 @@ def test_argmax_any_width(mx4, ctx, oracle, n, k):
     w.release()
 
 
+# one-row projections, whose fused form takes another launch shape
+@pytest.mark.parametrize("n,k", [(5000, 2048), (20002, 2048), (9001, 4096), (16383, 4096), (33000, 4096), (5001, 8192)])
+def test_argmax_tuned_widths(mx4, ctx, oracle, n, k):
+    if k == 8192:  # (two waves a team there, one here: another order of the same sums)
+        rng = np.random.default_rng(n)
+        packed, scales = planted(rng, n, k)
+        w = wrapped(ctx, packed, scales, 0)
+        xb, x = activations(mx4, ctx, rng, 1, k, mx4.BF16)
+        z, idx = ctx.buffer(n * 4), ctx.buffer(4)
+        ctx.matmul_argmax(xb, mx4.BF16, w, z, idx)
+        logits = z.download(np.float32)
+        assert_close(logits.reshape(1, n), oracle.matmul(x, packed.reshape(-1), scales.reshape(-1)), (n, k), scaled=True)
+        assert idx.download(np.uint32)[0] == int(np.argmax(logits))
+        w.release()
+    else:
+        test_argmax_any_width(mx4, ctx, oracle, n, k)
+
+
 # 2 to 32 token rows: one and two token tiles, chunks of 128 that leave 1 to 3
 # blocks, fewer chunks than waves, one to four chunks a wave, several slices of
 # K, and one, two and four row tiles a workgroup with several sets of them
