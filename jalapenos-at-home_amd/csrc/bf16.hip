@@ -110,15 +110,14 @@ struct Bf16Group {
     const uint16_t* w[4];
     float* y[4];
     uint32_t n[4];
-    uint32_t first[5];  // row-sets of each weight; first[count] .. first[4] are all of them
+    uint32_t first[5];  // rows before each weight; first[count] .. first[4] are all of them
     uint32_t count;
 };
 
 template <bool XBF16, int U>
 __global__ __launch_bounds__(512) void bf16_gemv_kernel(const void* __restrict__ x, uint32_t k, uint32_t turns,
-                                                        uint32_t rowsets, uint32_t stride, const Bf16Group g) {
+                                                        uint32_t rows, uint32_t stride, const Bf16Group g) {
     extern __shared__ __attribute__((aligned(16))) uint8_t xl[];
-    constexpr int R = 1;  // rows a wave
     constexpr uint32_t XB = XBF16 ? 2 : 4;
     const uint32_t lane = threadIdx.x % 64;
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -130,43 +129,38 @@ __global__ __launch_bounds__(512) void bf16_gemv_kernel(const void* __restrict__
         __builtin_amdgcn_sched_barrier(0);
     }
     struct Turn {
-        u32x4 w[R][U];
+        u32x4 w[U];
     };
-    auto pick = [&](uint32_t set, const uint16_t*& w, float*& y, uint32_t& n, uint32_t& row0) {
+    auto pick = [&](uint32_t at, const uint16_t*& w, float*& y, uint32_t& row) {
         w = g.w[0];
         y = g.y[0];
-        n = g.n[0];
         uint32_t first = 0;
 #pragma unroll
         for (int q = 1; q < 4; ++q) {
-            const bool in = q < (int)g.count && set >= g.first[q];
+            const bool in = q < (int)g.count && at >= g.first[q];
             w = in ? g.w[q] : w;
             y = in ? g.y[q] : y;
-            n = in ? g.n[q] : n;
             first = in ? g.first[q] : first;
         }
-        row0 = (set - first) * R;
+        row = at - first;
     };
-    // a row-set past the end loads zeros without touching memory
-    auto load = [&](uint32_t set, uint32_t turn, Turn& t) {
+    // a row past the end loads zeros without touching memory
+    auto load = [&](uint32_t at, uint32_t turn, Turn& t) {
         const uint16_t* w;
         float* y;
-        uint32_t n, row0;
-        pick(set, w, y, n, row0);
-        const bool valid = set < rowsets;
-        row0 = valid ? row0 : 0;
-        const uint32_t rows = valid ? (n - row0 < (uint32_t)R ? n - row0 : (uint32_t)R) : 0;
-        const __amdgpu_buffer_rsrc_t r = rsrc(w + (size_t)row0 * k, rows * k * 2);
+        uint32_t row;
+        pick(at, w, y, row);
+        const bool valid = at < rows;
+        const __amdgpu_buffer_rsrc_t r = rsrc(w + (size_t)(valid ? row : 0) * k, valid ? k * 2 : 0);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const uint32_t e = (turn * U + u) * 512 + 8 * lane;
-#pragma unroll
-            for (int i = 0; i < R; ++i)
-                t.w[i][u] = __builtin_amdgcn_raw_buffer_load_b128(r, e < k ? 2 * (i * k + e) : 0x80000000u, 0, 2);
+            t.w[u] = __builtin_amdgcn_raw_buffer_load_b128(r, e < k ? 2 * e : kPastEnd, 0, 2);
         }
         __builtin_amdgcn_sched_barrier(0);
     };
-    float acc[R];
+    float acc = 0.0f;
+    // (v_dot2_f32_bf16 keeps subnormal values and results)
     auto consume = [&](uint32_t turn, const Turn& t) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -174,54 +168,46 @@ __global__ __launch_bounds__(512) void bf16_gemv_kernel(const void* __restrict__
             if constexpr (XBF16) {
                 const u32x4 v = *reinterpret_cast<const u32x4*>(xp);
 #pragma unroll
-                for (int i = 0; i < R; ++i)
-#pragma unroll
-                    for (int d = 0; d < 4; ++d)
-                        acc[i] = __builtin_amdgcn_fdot2_f32_bf16(as_bf16x2(t.w[i][u][d]), as_bf16x2(v[d]), acc[i], false);
+                for (int d = 0; d < 4; ++d)
+                    acc = __builtin_amdgcn_fdot2_f32_bf16(as_bf16x2(t.w[u][d]), as_bf16x2(v[d]), acc, false);
             } else {
                 const f32x4 a = *reinterpret_cast<const f32x4*>(xp), b = *reinterpret_cast<const f32x4*>(xp + 16);
                 const float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
 #pragma unroll
-                for (int i = 0; i < R; ++i)
-#pragma unroll
-                    for (int d = 0; d < 4; ++d) {
-                        const uint32_t p = t.w[i][u][d];
-                        acc[i] = __builtin_fmaf(v[2 * d], __uint_as_float(p << 16), acc[i]);
-                        acc[i] = __builtin_fmaf(v[2 * d + 1], __uint_as_float(p & 0xffff0000u), acc[i]);
-                    }
+                for (int d = 0; d < 4; ++d) {
+                    acc = __builtin_fmaf(v[2 * d], __uint_as_float(t.w[u][d] << 16), acc);
+                    acc = __builtin_fmaf(v[2 * d + 1], __uint_as_float(t.w[u][d] & 0xffff0000u), acc);
+                }
             }
         }
     };
-    auto finish = [&](uint32_t set) {
+    auto finish = [&](uint32_t at) {
         const uint16_t* w;
         float* y;
-        uint32_t n, row0;
-        pick(set, w, y, n, row0);
-        const float total = wave_reduce_rows<R>(acc, lane);
-        const uint32_t row = row0 + reduced_row_of_lane<R>(lane);
-        if (row_writer<R>(lane) && row < n) y[row] = total;
+        uint32_t row;
+        pick(at, w, y, row);
+        float sums[1] = {acc};
+        const float total = wave_reduce_rows<1>(sums, lane);
+        if (lane == 0) y[row] = total;
+        acc = 0.0f;
     };
-    uint32_t set = blockIdx.x * 8 + wave, turn = 0;
+    uint32_t at = blockIdx.x * 8 + wave, turn = 0;
     Turn a, b;
-    load(set, 0, a);
-    wait_vm<R * U>();  // x is in, the weights need not be
+    load(at, 0, a);
+    wait_vm<U>();  // x is in, the weights need not be
     __syncthreads();
-    if (set >= rowsets) return;
-#pragma unroll
-    for (int i = 0; i < R; ++i) acc[i] = 0.0f;
+    if (at >= rows) return;
     auto step = [&](const Turn& cur, Turn& nxt) -> bool {
         const bool last = turn + 1 == turns;
-        const uint32_t nset = last ? set + stride : set, nturn = last ? 0 : turn + 1;
-        load(nset, nturn, nxt);
+        const uint32_t next = last ? at + stride : at;
+        load(next, last ? 0 : turn + 1, nxt);
         consume(turn, cur);
         if (last) {
-            finish(set);
-#pragma unroll
-            for (int i = 0; i < R; ++i) acc[i] = 0.0f;
-            if (nset >= rowsets) return true;
+            finish(at);
+            if (next >= rows) return true;
         }
-        set = nset;
-        turn = nturn;
+        at = next;
+        turn = last ? 0 : turn + 1;
         return false;
     };
     for (;;) {
@@ -231,10 +217,10 @@ __global__ __launch_bounds__(512) void bf16_gemv_kernel(const void* __restrict__
 }
 
 template <bool XBF16, int U>
-hipError_t go_gemv(const Bf16Group& g, const void* x, uint32_t k, uint32_t rowsets, uint32_t grid, hipStream_t s) {
+hipError_t go_gemv(const Bf16Group& g, const void* x, uint32_t k, uint32_t rows, uint32_t grid, hipStream_t s) {
     const uint32_t turns = (k + 512 * U - 1) / (512 * U);
     hipLaunchKernelGGL((bf16_gemv_kernel<XBF16, U>), dim3(grid), dim3(512), turns * U * 512 * (XBF16 ? 2 : 4), s, x, k,
-                       turns, rowsets, grid * 8, g);
+                       turns, rows, grid * 8, g);
     return hipGetLastError();
 }
 

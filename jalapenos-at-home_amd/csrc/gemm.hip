@@ -44,19 +44,6 @@ namespace mx4 {
 
 namespace {
 
-// Eight weights of one lane at one k-step: packed word `word` (elements
-// [8s, 8s + 8) of the lane's 64), block scale 2^(s - 127) folded in.
-__device__ __forceinline__ bf16x8 decode8(uint32_t word, float sc) {
-    const bf16x2 p0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, sc, 0);
-    const bf16x2 p1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, sc, 1);
-    const bf16x2 p2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, sc, 2);
-    const bf16x2 p3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, sc, 3);
-    bf16x8 r;
-    r[0] = p0[0]; r[1] = p0[1]; r[2] = p1[0]; r[3] = p1[1];
-    r[4] = p2[0]; r[5] = p2[1]; r[6] = p3[0]; r[7] = p3[1];
-    return r;
-}
-
 // Wait states after the last MFMAs before their accumulators are read (the
 // compiler has placed such reads after a branch without them on gfx950).
 __device__ __forceinline__ void mfma_drain() {
@@ -66,8 +53,6 @@ __device__ __forceinline__ void mfma_drain() {
 }
 
 constexpr int kBK = 128;  // K elements per stage
-
-typedef double f64x16 __attribute__((ext_vector_type(16)));
 
 // Stage layout in LDS (no padding): activations BM rows x A_CPR 16-byte slots,
 // packed weights BN rows x 4 slots, then BN scale words. Slots are written by
@@ -115,8 +100,6 @@ struct GemmSegs {
     uint32_t rows;
     uint32_t count;
 };
-
-constexpr uint32_t kPastEnd = 0x80000000u;  // past every buffer resource: a load there returns zeros
 
 template <bool XBF16, int WM, int WN, int TM, int TN, int D, bool ANY = false, class SG = NoGemmSegs>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_exact_kernel(const uint8_t* __restrict__ packed,
@@ -546,11 +529,16 @@ hipError_t go(const GemvArgs& a, uint32_t ks, float* part) {
 template <bool XBF16, bool ANY>
 hipError_t dispatch_rule(const GemvArgs& a, const GemmConfig& c, uint32_t ks, float* part) {
     if (c.wm == 2 && c.wn == 2 && c.tm == 2 && c.tn == 3) return go<XBF16, 2, 2, 2, 3, ANY>(a, ks, part);
-    if (c.wm == 2 && c.wn == 2 && c.tm == 2 && c.tn == 2) return go<XBF16, 2, 2, 2, 2, ANY>(a, ks, part);
     if (c.wm == 2 && c.wn == 2 && c.tm == 1 && c.tn == 1) return go<XBF16, 2, 2, 1, 1, ANY>(a, ks, part);
-    if (c.wm == 1 && c.wn == 4 && c.tm == 2 && c.tn == 2) return go<XBF16, 1, 4, 2, 2, ANY>(a, ks, part);
-    if (c.wm == 1 && c.wn == 4 && c.tm == 2 && c.tn == 1) return go<XBF16, 1, 4, 2, 1, ANY>(a, ks, part);
-    if (c.wm == 2 && c.wn == 4 && c.tm == 1 && c.tn == 2) return go<XBF16, 2, 4, 1, 2, ANY>(a, ks, part);
+    // (bf16 of any width: eight_waves has others in their place)
+    if constexpr (!(XBF16 && ANY)) {
+        if (c.wm == 2 && c.wn == 2 && c.tm == 2 && c.tn == 2) return go<XBF16, 2, 2, 2, 2, ANY>(a, ks, part);
+        if (c.wm == 1 && c.wn == 4 && c.tm == 2 && c.tn == 2) return go<XBF16, 1, 4, 2, 2, ANY>(a, ks, part);
+        if (c.wm == 1 && c.wn == 4 && c.tm == 2 && c.tn == 1) return go<XBF16, 1, 4, 2, 1, ANY>(a, ks, part);
+    }
+    // (f32 of any width: picked by nothing)
+    if constexpr (XBF16 || !ANY)
+        if (c.wm == 2 && c.wn == 4 && c.tm == 1 && c.tn == 2) return go<XBF16, 2, 4, 1, 2, ANY>(a, ks, part);
     // (picked by eight_waves only)
     if constexpr (XBF16 == ANY) {
         if (c.wm == 4 && c.wn == 2 && c.tm == 1 && c.tn == 2) return go<XBF16, 4, 2, 1, 2, ANY>(a, ks, part);
@@ -566,7 +554,7 @@ hipError_t dispatch_rule(const GemvArgs& a, const GemmConfig& c, uint32_t ks, fl
 // activations, whole stages: 24576 x 4096 at 64 rows 96 -> 75 us, 12288 x 2048
 // at 300 rows 58.6 -> 50.7) or 64-bit sums (bf16, any width: 8576 x 1600 at 200
 // rows 27.5 -> 24.4 us) hold up its MFMAs. f32 at any width has both, and four
-// waves measured faster (8576 x 1600 at 77 rows 47 against 63 us); bf16 of whole
+// waves measured faster (by a quarter at 8576 x 1600, 77 rows); bf16 of whole
 // stages has neither, and runs the same in both.
 GemmConfig eight_waves(GemmConfig c, bool x_bf16, bool any) {
     if (x_bf16 != any) return c;

@@ -34,9 +34,6 @@ namespace {
 
 constexpr int kBK = 64;                     // K elements per stage
 constexpr int kFold = 2;                    // stages summed in 32 bits
-constexpr uint32_t kPastEnd = 0x80000000u;  // past every buffer resource: a load there returns zeros
-typedef double f64x16 __attribute__((ext_vector_type(16)));
-
 // The weights of a launch: up to four of one width sharing x, weight s owning
 // the column tiles [tile0[s], tile0[s + 1]) of the grid.
 struct Weights {

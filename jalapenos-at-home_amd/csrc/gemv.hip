@@ -179,7 +179,6 @@ __device__ __forceinline__ Seg pick_seg(const Segs& sg, uint32_t rs) {
 // that many blocks; SUB rows lie side by side in a wave (64 / SUB lanes each),
 // row-set row i SUB + part is load i of part `part`, and lanes past the row's
 // blocks load zeros (codes and scale byte 0, so they add nothing).
-constexpr uint32_t kPastEnd = 0x80000000u;  // past every buffer resource
 template <int SUB>
 constexpr uint32_t kLanes = 64 / (SUB > 1 ? SUB : 1);  // lanes per row of a wave
 template <int R, int SUB>

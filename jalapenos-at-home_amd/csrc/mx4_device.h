@@ -112,6 +112,22 @@ __device__ __forceinline__ void split3x8(const u32x4 a, const u32x4 b, bf16x8& h
     if (__any(bad != bad)) split3_careful(a, b, hi, mid, lo);
 }
 
+// Eight E2M1 weights of a packed word, the block's scale folded in (bytes 2..252:
+// exact in bf16).
+__device__ __forceinline__ bf16x8 decode8(uint32_t word, float sc) {
+    const bf16x2 p0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, sc, 0);
+    const bf16x2 p1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, sc, 1);
+    const bf16x2 p2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, sc, 2);
+    const bf16x2 p3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, sc, 3);
+    bf16x8 r;
+    r[0] = p0[0]; r[1] = p0[1]; r[2] = p1[0]; r[3] = p1[1];
+    r[4] = p2[0]; r[5] = p2[1]; r[6] = p3[0]; r[7] = p3[1];
+    return r;
+}
+
+constexpr uint32_t kPastEnd = 0x80000000u;  // past every buffer resource: a load there returns zeros
+typedef double f64x16 __attribute__((ext_vector_type(16)));
+
 // Values below 2^-110 lose bits as three bf16 terms, whose least is 2^-133. The
 // kernels for any width and for bf16 weights lose none all the same: where a lane
 // holds, in a step of the reduction, only such values (zeros apart), or an inf or

@@ -39,7 +39,6 @@ namespace mx4 {
 namespace {
 
 constexpr int kStreamed = 2;                  // weights are used once: do not keep them in the caches
-constexpr uint32_t kPastEnd = 0x80000000u;    // past every buffer resource: a load there returns zeros
 constexpr int TW = 8;                         // waves per workgroup
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
@@ -71,17 +70,6 @@ __device__ __forceinline__ Pick pick(const Weights& g, uint32_t tile) {
         p.first = in ? g.first[q] : p.first;
     }
     return p;
-}
-
-__device__ __forceinline__ bf16x8 decode8(uint32_t word, float sc) {
-    const bf16x2 p0 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, sc, 0);
-    const bf16x2 p1 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, sc, 1);
-    const bf16x2 p2 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, sc, 2);
-    const bf16x2 p3 = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, sc, 3);
-    bf16x8 r;
-    r[0] = p0[0]; r[1] = p0[1]; r[2] = p1[0]; r[3] = p1[1];
-    r[4] = p2[0]; r[5] = p2[1]; r[6] = p3[0]; r[7] = p3[1];
-    return r;
 }
 
 // Wait states between the last MFMAs and reads of their sums (see gemm.hip).
