@@ -602,6 +602,116 @@ bool gemm_any_supported(uint32_t m, uint32_t n, uint32_t k, bool x_bf16) {
 // partials, the range its picks were measured in.
 constexpr uint64_t kFewRowsSplitBytes = 4ull << 20;
 
+// The arrangement and K split for a shape; part_bytes of scratch for partials.
+static GemmConfig shape_rule(const GemvArgs& a, int cus, uint64_t part_bytes) {
+    // column tiles of width bn over the weight (or over each weight of a group)
+    auto col_tiles = [&](uint32_t bn) -> uint64_t {
+        if (!a.group) return (a.n + bn - 1) / bn;
+        uint64_t t = 0;
+        for (uint32_t s = 0; s < a.group->count; ++s) t += (a.group->n[s] + bn - 1) / bn;
+        return t;
+    };
+    GemmConfig c;
+    // The tile with the least estimated time: whole rounds of workgroups
+    // (one per CU) times the time one round of that tile takes. The round
+    // times (µs at K = 4096, bf16 x) are from a sweep of every instance on
+    // the Qwen3-8B q, gate and down weights at M = 64..2048 on MI355X
+    // (cold weights); with them the pick was the fastest instance, or
+    // within 2% of it, at every M of the sweep: gate at M = 384 / 768 /
+    // 1536 128 x 192 (47 / 90 / 145 us, where the largest tile whose grid
+    // reaches three quarters of the CUs takes 64 / 102 / 157 us), at 2048
+    // 128 x 256 (176 us); q and down at M = 512 64 x 128 (23 / 64 us).
+    // The larger tiles re-read fewer operand bytes per flop, the smaller
+    // ones leave fewer CUs idle in the last round.
+    struct Cand { int wm, wn, tm, tn, bm, bn; double round_us; };
+    const Cand cands[] = {{2, 4, 2, 2, 128, 256, 50.0}, {2, 2, 2, 3, 128, 192, 46.0},
+                          {1, 4, 2, 2, 64, 256, 33.5},  {2, 2, 2, 2, 128, 128, 34.5},
+                          {1, 4, 2, 1, 64, 128, 22.0},  {2, 2, 1, 1, 64, 64, 16.5}};
+    const uint64_t nc = (uint64_t)(cus > 0 ? cus : 256);
+    const uint64_t want = nc * 3 / 4;
+    // 128 x 256 has an instance for bf16 x only
+    auto wide = [&](const Cand& cd) { return cd.bn == 256 && cd.bm == 128 && !a.x_bf16; };
+    // A bf16 group of whole stages runs unsplit even when its tiles leave
+    // CUs idle: one short round of them beats a split and the pass that
+    // adds it (a small model's layer 28.0 against 30.3 us, 4096 wide at 48
+    // rows 89.8 against 90.3), and its weights' separate launches.
+    // A split saves time with K and costs it with the outputs, so that a group
+    // cuts K only while its partials stay below 8 KiB for every element of K
+    // (two weights of 1536 x 512, f32 x, at 64 rows 10.7 -> 8.7 us with 3 MiB in
+    // four slices, at 200 and 300 rows 11.1 and 11.5 -> 13.0 and 20.5 with 5 and
+    // 14 MiB; 2048 + 512 + 512 x 2048 at 300 rows 33.8 -> 30.0 with 14 MiB) and,
+    // where the tiles are few, not into a second round of the CUs (768 + 192 +
+    // 192 x 768 at 300 rows 14.6 -> 15.5 us).
+    const bool may_split = !(a.group && a.x_bf16 && a.k % kBK == 0);
+    if (a.group && part_bytes > 8192ull * a.k) part_bytes = 8192ull * a.k;
+    uint32_t rows = a.n;  // weight rows, of all the group's weights
+    if (a.group) {
+        rows = 0;
+        for (uint32_t s = 0; s < a.group->count; ++s) rows += a.group->n[s];
+    }
+    const Cand* best = nullptr;
+    double best_t = 0.0;
+    for (const Cand& cd : cands) {
+        if (wide(cd)) continue;
+        const uint64_t tiles = (uint64_t)((a.m + cd.bm - 1) / cd.bm) * col_tiles(cd.bn);
+        const double t = (double)((tiles + nc - 1) / nc) * cd.round_us;
+        if (!best || t < best_t) {
+            best = &cd;
+            best_t = t;
+        }
+    }
+    // f32 activations, and bf16 ones on wide K (K >= 8192): the largest
+    // tile whose workgroups, with K cut into 1-4 slices of whole stages,
+    // make one round of at least three quarters of the CUs (the most
+    // workgroups among equal tiles). Measured on the 8B q / gate / down
+    // weights at 64..1024 rows (cold): f32 q at 256 / 512 rows 63.9 /
+    // 113.0 -> 44.2 / 75.8 us, gate at 128 / 256 113.3 / 131.7 -> 53.2 /
+    // 90.9, down at 256 / 512 184 / 329 -> 107 / 201; bf16 down at 384 /
+    // 512 / 1024 60.7 / 66.0 / 101.7 -> 47.5 / 54.1 / 93.3. bf16 at K =
+    // 4096 keeps the round-time pick (its splits measured slower there).
+    if (!a.x_bf16 || a.k >= 8192) {
+        const Cand* sel = nullptr;
+        uint32_t sel_ks = 0;
+        uint64_t sel_area = 0, sel_wgs = 0;
+        for (const Cand& cd : cands) {
+            if (wide(cd)) continue;
+            const uint64_t tiles = (uint64_t)((a.m + cd.bm - 1) / cd.bm) * col_tiles(cd.bn);
+            for (uint32_t ks = 1; ks <= 4; ++ks) {
+                if (!slices_fit(a.k, ks)) continue;
+                if (ks > 1 && (!may_split || (uint64_t)ks * a.m * rows * 4 > part_bytes)) continue;
+                const uint64_t wgs = tiles * ks, area = (uint64_t)cd.bm * cd.bn;
+                if (wgs > nc || wgs < want) continue;
+                if (!sel || area > sel_area || (area == sel_area && wgs > sel_wgs)) {
+                    sel = &cd;
+                    sel_ks = ks;
+                    sel_area = area;
+                    sel_wgs = wgs;
+                }
+            }
+        }
+        if (sel) {
+            c.wm = sel->wm; c.wn = sel->wn; c.tm = sel->tm; c.tn = sel->tn;
+            c.ks = (int)sel_ks;
+            return eight_waves(c, a.x_bf16, a.k % kBK != 0);
+        }
+    }
+    const Cand pick = *best;
+    c.wm = pick.wm; c.wn = pick.wn; c.tm = pick.tm; c.tn = pick.tn;
+    // A grid still short of the CUs (few token rows): split K across up to
+    // four workgroups per tile, each slice whole stages, when the partials
+    // fit the scratch; a second small kernel adds them in slice order.
+    const uint64_t tiles = (uint64_t)((a.m + pick.bm - 1) / pick.bm) * col_tiles(pick.bn);
+    c.ks = 1;
+    for (uint32_t ks = 4; ks >= 2 && tiles < want && may_split; --ks) {
+        if (slices_fit(a.k, ks) && !(a.group && tiles * ks > nc) &&
+            (uint64_t)ks * a.m * rows * 4 <= std::min(part_bytes, kFewRowsSplitBytes)) {
+            c.ks = (int)ks;
+            break;
+        }
+    }
+    return eight_waves(c, a.x_bf16, a.k % kBK != 0);
+}
+
 hipError_t launch_gemm_exact(const GemvArgs& a, int cus, const GemmConfig* forced, float* part, uint64_t part_bytes) {
     if (a.group) {
         // a group: every weight supported, no explicit configuration
@@ -612,13 +722,6 @@ hipError_t launch_gemm_exact(const GemvArgs& a, int cus, const GemmConfig* force
     } else if (!gemm_any_supported(a.m, a.n, a.k, a.x_bf16)) {
         return hipErrorNotSupported;
     }
-    // column tiles of width bn over the weight (or over each weight of a group)
-    auto col_tiles = [&](uint32_t bn) -> uint64_t {
-        if (!a.group) return (a.n + bn - 1) / bn;
-        uint64_t t = 0;
-        for (uint32_t s = 0; s < a.group->count; ++s) t += (a.group->n[s] + bn - 1) / bn;
-        return t;
-    };
     GemmConfig c;
     if (forced && forced->wm) {
         c = *forced;
@@ -629,107 +732,19 @@ hipError_t launch_gemm_exact(const GemvArgs& a, int cus, const GemmConfig* force
                          (uint64_t)c.ks * a.m * a.n * 4 > part_bytes))
             return hipErrorNotSupported;
     } else {
-        // The tile with the least estimated time: whole rounds of workgroups
-        // (one per CU) times the time one round of that tile takes. The round
-        // times (µs at K = 4096, bf16 x) are from a sweep of every instance on
-        // the Qwen3-8B q, gate and down weights at M = 64..2048 on MI355X
-        // (cold weights); with them the pick was the fastest instance, or
-        // within 2% of it, at every M of the sweep: gate at M = 384 / 768 /
-        // 1536 128 x 192 (47 / 90 / 145 us, where the largest tile whose grid
-        // reaches three quarters of the CUs takes 64 / 102 / 157 us), at 2048
-        // 128 x 256 (176 us); q and down at M = 512 64 x 128 (23 / 64 us).
-        // The larger tiles re-read fewer operand bytes per flop, the smaller
-        // ones leave fewer CUs idle in the last round.
-        struct Cand { int wm, wn, tm, tn, bm, bn; double round_us; };
-        const Cand cands[] = {{2, 4, 2, 2, 128, 256, 50.0}, {2, 2, 2, 3, 128, 192, 46.0},
-                              {1, 4, 2, 2, 64, 256, 33.5},  {2, 2, 2, 2, 128, 128, 34.5},
-                              {1, 4, 2, 1, 64, 128, 22.0},  {2, 2, 1, 1, 64, 64, 16.5}};
-        const uint64_t nc = (uint64_t)(cus > 0 ? cus : 256);
-        const uint64_t want = nc * 3 / 4;
-        // 128 x 256 has an instance for bf16 x only
-        auto wide = [&](const Cand& cd) { return cd.bn == 256 && cd.bm == 128 && !a.x_bf16; };
-        // A bf16 group of whole stages runs unsplit even when its tiles leave
-        // CUs idle: one short round of them beats a split and the pass that
-        // adds it (a small model's layer 28.0 against 30.3 us, 4096 wide at 48
-        // rows 89.8 against 90.3), and its weights' separate launches.
-        // A split saves time with K and costs it with the outputs, so that a group
-        // cuts K only while its partials stay below 8 KiB for every element of K
-        // (two weights of 1536 x 512, f32 x, at 64 rows 10.7 -> 8.7 us with 3 MiB in
-        // four slices, at 200 and 300 rows 11.1 and 11.5 -> 13.0 and 20.5 with 5 and
-        // 14 MiB; 2048 + 512 + 512 x 2048 at 300 rows 33.8 -> 30.0 with 14 MiB) and,
-        // where the tiles are few, not into a second round of the CUs (768 + 192 +
-        // 192 x 768 at 300 rows 14.6 -> 15.5 us).
-        const bool may_split = !(a.group && a.x_bf16 && a.k % kBK == 0);
-        if (a.group && part_bytes > 8192ull * a.k) part_bytes = 8192ull * a.k;
-        uint32_t rows = a.n;  // weight rows, of all the group's weights
-        if (a.group) {
-            rows = 0;
-            for (uint32_t s = 0; s < a.group->count; ++s) rows += a.group->n[s];
-        }
-        const Cand* best = nullptr;
-        double best_t = 0.0;
-        for (const Cand& cd : cands) {
-            if (wide(cd)) continue;
-            const uint64_t tiles = (uint64_t)((a.m + cd.bm - 1) / cd.bm) * col_tiles(cd.bn);
-            const double t = (double)((tiles + nc - 1) / nc) * cd.round_us;
-            if (!best || t < best_t) {
-                best = &cd;
-                best_t = t;
-            }
-        }
-        // f32 activations, and bf16 ones on wide K (K >= 8192): the largest
-        // tile whose workgroups, with K cut into 1-4 slices of whole stages,
-        // make one round of at least three quarters of the CUs (the most
-        // workgroups among equal tiles). Measured on the 8B q / gate / down
-        // weights at 64..1024 rows (cold): f32 q at 256 / 512 rows 63.9 /
-        // 113.0 -> 44.2 / 75.8 us, gate at 128 / 256 113.3 / 131.7 -> 53.2 /
-        // 90.9, down at 256 / 512 184 / 329 -> 107 / 201; bf16 down at 384 /
-        // 512 / 1024 60.7 / 66.0 / 101.7 -> 47.5 / 54.1 / 93.3. bf16 at K =
-        // 4096 keeps the round-time pick (its splits measured slower there).
-        if (!a.x_bf16 || a.k >= 8192) {
-            const Cand* sel = nullptr;
-            uint32_t sel_ks = 0;
-            uint64_t sel_area = 0, sel_wgs = 0;
-            for (const Cand& cd : cands) {
-                if (wide(cd)) continue;
-                const uint64_t tiles = (uint64_t)((a.m + cd.bm - 1) / cd.bm) * col_tiles(cd.bn);
-                for (uint32_t ks = 1; ks <= 4; ++ks) {
-                    if (!slices_fit(a.k, ks)) continue;
-                    if (ks > 1 && (!may_split || !part || (uint64_t)ks * a.m * rows * 4 > part_bytes)) continue;
-                    const uint64_t wgs = tiles * ks, area = (uint64_t)cd.bm * cd.bn;
-                    if (wgs > nc || wgs < want) continue;
-                    if (!sel || area > sel_area || (area == sel_area && wgs > sel_wgs)) {
-                        sel = &cd;
-                        sel_ks = ks;
-                        sel_area = area;
-                        sel_wgs = wgs;
-                    }
-                }
-            }
-            if (sel) {
-                c.wm = sel->wm; c.wn = sel->wn; c.tm = sel->tm; c.tn = sel->tn;
-                c.ks = (int)sel_ks;
-                c = eight_waves(c, a.x_bf16, a.k % kBK != 0);
-                return a.x_bf16 ? dispatch<true>(a, c, part) : dispatch<false>(a, c, part);
-            }
-        }
-        const Cand pick = *best;
-        c.wm = pick.wm; c.wn = pick.wn; c.tm = pick.tm; c.tn = pick.tn;
-        // A grid still short of the CUs (few token rows): split K across up to
-        // four workgroups per tile, each slice whole stages, when the partials
-        // fit the scratch; a second small kernel adds them in slice order.
-        const uint64_t tiles = (uint64_t)((a.m + pick.bm - 1) / pick.bm) * col_tiles(pick.bn);
-        c.ks = 1;
-        for (uint32_t ks = 4; ks >= 2 && tiles < want && may_split; --ks) {
-            if (slices_fit(a.k, ks) && part && !(a.group && tiles * ks > nc) &&
-                (uint64_t)ks * a.m * rows * 4 <= std::min(part_bytes, kFewRowsSplitBytes)) {
-                c.ks = (int)ks;
-                break;
-            }
-        }
-        c = eight_waves(c, a.x_bf16, a.k % kBK != 0);
+        c = shape_rule(a, cus, part ? part_bytes : 0);
     }
     return a.x_bf16 ? dispatch<true>(a, c, part) : dispatch<false>(a, c, part);
+}
+
+uint32_t mx4_rule_gemm_exact(const uint32_t* n, uint32_t count, uint32_t m, uint32_t k, bool x_bf16, int cus, uint64_t part_bytes) {
+    GemvGroup g{};
+    g.count = count;
+    for (uint32_t i = 0; i < count; ++i) g.n[i] = n[i];
+    GemvArgs a{nullptr, nullptr, nullptr, nullptr, m, n[0], k, x_bf16, nullptr};
+    if (count > 1) a.group = &g;
+    const GemmConfig c = shape_rule(a, cus, part_bytes);
+    return (uint32_t)(c.wm * 10000 + c.wn * 1000 + c.tm * 100 + c.tn * 10 + c.ks);
 }
 
 }  // namespace mx4

@@ -352,10 +352,12 @@ Plan plan(const uint32_t* n, uint32_t count, uint32_t m, uint32_t k, bool x_bf16
     struct Cand { int bm, bn; double stage_us; };
     const Cand cands[] = {{128, 128, x_bf16 ? 0.65 : 1.64}, {64, 128, x_bf16 ? 0.43 : 1.2}, {128, 64, x_bf16 ? 0.41 : 1.28},
                           {64, 64, x_bf16 ? 0.42 : 1.04}, {128, 256, 1.19}};
-    const int count_c = x_bf16 ? 5 : 4;  // (128 x 256 of f32 activations does not fit the registers)
     const uint64_t nc = (uint64_t)(cus > 0 ? cus : 256);
     Plan best;
-    for (int c = 0; c < count_c; ++c) {
+    for (int c = 0; c < 5; ++c) {
+        // (128 x 256 of f32 activations does not fit the registers; 64 x 64 of bf16
+        // ones takes as long as 128 x 64)
+        if (c == (x_bf16 ? 3 : 4)) continue;
         uint64_t tiles = 0;
         for (uint32_t q = 0; q < count; ++q) tiles += (n[q] + cands[c].bn - 1) / cands[c].bn;
         tiles *= (m + cands[c].bm - 1) / cands[c].bm;
@@ -374,12 +376,14 @@ template <bool XBF16>
 hipError_t dispatch(const Weights& g, const void* x, uint32_t m, uint32_t k, int cus, float* part, uint64_t part_bytes,
                     hipStream_t s) {
     const Plan p = plan(g.n, g.count, m, k, XBF16, cus, part ? part_bytes : 0);
-    if constexpr (XBF16)
+    if constexpr (XBF16) {
         if (p.tile == 4) return go<XBF16, 2, 4, 2, 2>(g, x, m, k, p.ks, part, s);
+    } else {
+        if (p.tile == 3) return go<XBF16, 2, 2, 1, 1>(g, x, m, k, p.ks, part, s);
+    }
     if (p.tile == 0) return go<XBF16, 4, 2, 1, 2>(g, x, m, k, p.ks, part, s);
     if (p.tile == 1) return go<XBF16, 2, 4, 1, 1>(g, x, m, k, p.ks, part, s);
-    if (p.tile == 2) return go<XBF16, 4, 2, 1, 1>(g, x, m, k, p.ks, part, s);
-    return go<XBF16, 2, 2, 1, 1>(g, x, m, k, p.ks, part, s);
+    return go<XBF16, 4, 2, 1, 1>(g, x, m, k, p.ks, part, s);
 }
 
 }  // namespace
@@ -388,6 +392,12 @@ hipError_t dispatch(const Weights& g, const void* x, uint32_t m, uint32_t k, int
 // weights at 33 .. 300 rows 1024 x 64 10.7 / 9.2 f32, 12288 x 64 27.2 / 26.5 bf16).
 double gemm_bf16_us(const uint32_t* n, uint32_t count, uint32_t m, uint32_t k, bool x_bf16, int cus, uint64_t part_bytes) {
     return plan(n, count, m, k, x_bf16, cus, part_bytes).us - 1.2;
+}
+
+uint32_t mx4_rule_gemm_bf16(const uint32_t* n, uint32_t count, uint32_t m, uint32_t k, bool x_bf16, int cus, uint64_t part_bytes) {
+    static const uint32_t tiles[] = {42120, 24110, 42110, 22110, 24220};
+    const Plan p = plan(n, count, m, k, x_bf16, cus, part_bytes);
+    return tiles[p.tile] + p.ks;
 }
 
 bool gemm_bf16_supported(uint32_t m, uint32_t n, uint32_t k, bool x_bf16) {

@@ -131,6 +131,15 @@ double gemm_bf16_us(const uint32_t* n, uint32_t count, uint32_t m, uint32_t k, b
 // y = sum over ks slices of part[s] (count floats each), in slice order.
 hipError_t launch_split_sum(const float* part, uint32_t ks, uint32_t count, float* y, hipStream_t s);
 
+// What the shape rules pick, for tests that have to reach every instance: the
+// GEMMs' waves along M and N, tiles a wave along M and N and K slices as decimal
+// digits, skinny_any's chunks a wave and tiles a workgroup.
+extern "C" uint32_t mx4_rule_gemm_exact(const uint32_t* n, uint32_t count, uint32_t m, uint32_t k, bool x_bf16, int cus,
+                                    uint64_t part_bytes);
+extern "C" uint32_t mx4_rule_gemm_bf16(const uint32_t* n, uint32_t count, uint32_t m, uint32_t k, bool x_bf16, int cus,
+                                   uint64_t part_bytes);
+extern "C" uint32_t mx4_rule_skinny_any(bool fp4, bool x_bf16, uint32_t m, uint32_t k, uint32_t tiles, int cus);
+
 // Block-scaled MFMA prefill on requantized activations. Both operands are in
 // the fragment-native layout of prefill.hip (launch_to_fragments, or the
 // quantizers' fragment output).

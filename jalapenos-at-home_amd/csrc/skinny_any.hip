@@ -495,31 +495,40 @@ hipError_t go(const Weights& g, const void* x, uint32_t m, uint32_t k, uint32_t 
 //    with two of each; two of each with two token tiles;
 //  * f32 x: one (two spill), the second token tile counted as tiles of their
 //    own: 1600 x 1600 at 7 rows 6.1, 18432 x 3264 at 7 / 29 rows 29 / 59.
-template <bool FP4, bool XBF16, int MT>
-hipError_t go_shape(const Weights& g, const void* x, uint32_t m, uint32_t k, uint32_t tiles, int cus, hipStream_t s) {
+struct Shape {
+    uint32_t t, chunks, grid;
+};
+Shape shape_rule(bool fp4, bool x_bf16, uint32_t m, uint32_t k, uint32_t tiles, int cus) {
     const uint32_t nc = (uint32_t)(cus > 0 ? cus : 256);
+    const uint32_t mt = x_bf16 && m > 16 ? 2 : 1;               // token tiles of a workgroup
     const uint32_t per_wave = ((k + 127) / 128 + TW - 1) / TW;  // chunks of a row for each wave
     // the activations of a slice take 16 MT XP NC registers, the weights 5 NC (FP4) or 16 NC a tile
-    constexpr int kMost = XBF16 ? 4 / MT : 1;
-    const uint32_t halves = (m + 16 * MT - 1) / (16 * MT);
+    const uint32_t most = x_bf16 ? 4 / mt : 1;
+    const uint32_t halves = (m + 16 * mt - 1) / (16 * mt);
     uint32_t t = tiles * halves <= nc ? 1 : tiles * halves <= 2 * nc ? 2 : 4;
     uint32_t chunks = per_wave >= 3 ? 4u : per_wave;
-    if (chunks > (uint32_t)kMost) chunks = (uint32_t)kMost;
+    if (chunks > most) chunks = most;
     if (chunks > 2 && t == 1) chunks = 2;
-    if (!FP4 && XBF16) {
-        chunks = MT == 2 && t > 1 ? chunks : 1;
-        t = MT == 1 && tiles <= 4 * nc ? 1 : t > 2 ? 2 : t;
+    if (!fp4 && x_bf16) {
+        chunks = mt == 2 && t > 1 ? chunks : 1;
+        t = mt == 1 && tiles <= 4 * nc ? 1 : t > 2 ? 2 : t;
     }
-    if (chunks == 4 || (chunks == 2 && MT == 1)) t = t > 2 ? 2 : t;
+    if (chunks == 4 || (chunks == 2 && mt == 1)) t = t > 2 ? 2 : t;
     uint32_t grid = (tiles + t - 1) / t;
-    if (t > 1 && grid > (XBF16 ? nc : 2 * nc)) grid = XBF16 ? nc : 2 * nc;
+    if (t > 1 && grid > (x_bf16 ? nc : 2 * nc)) grid = x_bf16 ? nc : 2 * nc;
     // the same number of sets for every workgroup
     const uint32_t sets = (tiles + grid * t - 1) / (grid * t);
-    grid = (tiles + sets * t - 1) / (sets * t);
+    return {t, chunks, (tiles + sets * t - 1) / (sets * t)};
+}
+
+template <bool FP4, bool XBF16, int MT>
+hipError_t go_shape(const Weights& g, const void* x, uint32_t m, uint32_t k, uint32_t tiles, int cus, hipStream_t s) {
+    constexpr int kMost = XBF16 ? 4 / MT : 1;
+    const Shape r = shape_rule(FP4, XBF16, m, k, tiles, cus);
 #define MX4_SKINNY_ANY(C, T_)                                            \
     if constexpr (C <= kMost && (FP4 || !XBF16 || (T_ <= 2 && C == 1) || (T_ == 2 && MT == 2)) && \
                   (C == 1 || T_ <= 2 || MT == 2))                         \
-        if (chunks == C && t == T_) return go<FP4, XBF16, MT, C, T_>(g, x, m, k, tiles, grid, s);
+        if (r.chunks == C && r.t == T_) return go<FP4, XBF16, MT, C, T_>(g, x, m, k, tiles, r.grid, s);
     MX4_SKINNY_ANY(1, 1) MX4_SKINNY_ANY(1, 2) MX4_SKINNY_ANY(1, 4) MX4_SKINNY_ANY(2, 1) MX4_SKINNY_ANY(2, 2)
     MX4_SKINNY_ANY(2, 4) MX4_SKINNY_ANY(4, 2)
 #undef MX4_SKINNY_ANY
@@ -553,6 +562,11 @@ bool skinny_any_faster(uint32_t m, uint32_t k, uint32_t tiles, bool x_bf16, int 
     // (the ring: two tiles for each of the workgroups of eight waves a CU)
     const uint32_t ring = k == 2048 ? 4 * nc : 2 * nc;
     return m > 16 && (k == 2048 || k == 4096) && tiles > nc && tiles < ring;
+}
+
+uint32_t mx4_rule_skinny_any(bool fp4, bool x_bf16, uint32_t m, uint32_t k, uint32_t tiles, int cus) {
+    const Shape r = shape_rule(fp4, x_bf16, m, k, tiles, cus);
+    return r.chunks * 10 + r.t;
 }
 
 hipError_t launch_skinny_any(const GemvArgs& a, const uint16_t* const* bf16, int cus) {

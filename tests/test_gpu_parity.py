@@ -929,7 +929,8 @@ GROUP_EXACT = [
 @pytest.mark.parametrize("k,shapes,ms", GROUP_EXACT, ids=[f"k{k}-{'_'.join(map(str, s))}" for k, s, _ in GROUP_EXACT])
 def test_group_exact_gemm_against_oracle(mx4, ctx, oracle, k, shapes, ms):
     """More than 32 token rows through mx4_matmul_group: one exact-GEMM launch
-    over every weight's column tiles, K unsplit. Each weight's outputs against the
+    over every weight's column tiles (f32 activations: K cut where the tiles are
+    few). Each weight's outputs against the
     oracle (first and last 16 rows and 48 drawn on weights wider than 1024)
     and against separate mx4_matmul calls, bf16 and f32 activations, outputs
     NaN-filled first."""

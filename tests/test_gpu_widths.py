@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 from test_gpu_parity import assert_close, ctx, f32_bits, mx4  # noqa: F401  (ctx, mx4: fixtures)
+from test_launch_rules import GEMM_SHAPES, SKINNY_SHAPES
 
 pytestmark = pytest.mark.gpu
 
@@ -97,8 +98,9 @@ def check_any_width(mx4, ctx, oracle, seed, m, ns, k, shift):
 
 
 # more than 32 token rows: K below, at and past a 128-element stage and with 1
-# to 3 blocks left in the last one; rows and columns around the 64, 128 and
-# 192-wide tiles; enough stages that the K split's last slice is short
+# to 3 blocks left in the last one; rows and columns around 64; enough stages that
+# the K split's last slice is short. (All but a few on 64 x 64 tiles; the other
+# instances: test_any_width_gemm_instances)
 @pytest.mark.parametrize("m,ns,k,shift", [
     (33, (1, 65, 31), 32, 0), (64, (64, 192), 96, 1), (65, (129, 3), 160, 2), (77, (320, 64, 64), 416, 3),
     (129, (50, 257), 352, 0), (40, (193, 33, 7, 64), 1600, 1), (200, (640, 96), 544, 2), (260, (2100,), 288, 3),
@@ -287,9 +289,8 @@ def test_bf16_nonfinite(mx4, ctx, oracle, m, k):
             w.release()
 
 
-# rows of one and two a wave, K of one turn and several with lanes past its end,
-# K past the LDS copy of x (24576 f32: the row-per-wave kernel) and K of no
-# whole pieces
+# K of one turn and several with lanes past its end, K past the LDS copy of x
+# (24576 f32: the row-per-wave kernel) and K of no whole pieces
 @pytest.mark.parametrize("ns,k", [
     ((1, 3), 8), ((33, 5), 520), ((50, 64, 7), 1024), ((130, 2), 1608), ((70, 9), 2056), ((5000, 1), 264),
     ((9000, 4000, 3), 136), ((40, 41), 12296), ((20, 3), 20480), ((17, 5), 24576), ((40, 20), 1604)])
@@ -297,9 +298,10 @@ def test_bf16_decode(mx4, ctx, oracle, ns, k):
     check_bf16_weights(mx4, ctx, oracle, ns[0] + k, 1, ns, k)
 
 
-# tiles of 64 and 128 rows and columns, each full, one short and one over; K below,
-# at and past a 64-element stage, odd and even stage counts, K splits with a
-# short last slice, and K of no whole pieces
+# rows and columns around 64 and 128; K below, at and past a 64-element stage, odd
+# and even stage counts, K splits with a short last slice, and K of no whole pieces
+# (small weights run the row-per-wave kernel, the others the smallest tiles; every
+# tile: test_bf16_gemm_instances)
 @pytest.mark.parametrize("m,ns,k", [
     (33, (1, 65), 8), (64, (64, 128, 2), 64), (65, (127, 33), 72), (129, (130, 5), 200), (40, (300, 7, 64, 1), 1032),
     (200, (257, 64), 2056), (500, (1100, 40), 328), (70, (60, 9), 4100), (1000, (520,), 136)])
@@ -325,19 +327,25 @@ def test_explicit_team_keeps_a_default_that_fits(mx4, ctx, oracle, team):
     w.release()
 
 
-# Largest distance of a row of outputs from the sum in 64 bits, relative to the
-# row's length. Products are exact and a chain of 32-bit additions is at most 24
-# long (three terms of eight MFMAs), then continues in 64 bits: measured 0.5 to
-# 1.3e-7 (2^-24 is 0.6e-7). One chain over K or a lost third term shows as 4e-7
-# and more.
-ROW_TOL = 2.5e-7
+# Distance from the sum in 64 bits, relative to its length: of all outputs and of
+# one token row's. Products are exact, and a chain of 32-bit additions is at most
+# 24 long (three terms of eight MFMAs) before it continues in 64 bits: 24 roundings
+# of at most 2^-24 of a partial sum walk to about 24^0.5 2^-24 / 3^0.5 = 1.7e-7 of
+# its size (measured 0.5 to 1.3e-7), a single row of few large outputs to three
+# times that. One chain over all of K or a lost third term shows as 4e-7 and more
+# over all outputs.
+ALL_TOL, ROW_TOL = 2.5e-7, 6e-7
 
 
-def check_rows(out, x, w, what, tol=ROW_TOL):
-    """Every token row of out against x . w^T in 64 bits."""
+def check_rows(out, x, w, what, alike=True):
+    """Every token row of out, and all of them (if they are of one size), against
+    x . w^T in 64 bits."""
     ref = x.astype(np.float64) @ w.astype(np.float64).T
-    err = np.linalg.norm(out.astype(np.float64) - ref, axis=1) / np.linalg.norm(ref, axis=1)
-    assert np.all(err <= tol), f"{what}: row {int(np.argmax(err))} of {len(err)}: {np.max(err):.2e}"
+    diff, size = np.linalg.norm(out.astype(np.float64) - ref, axis=1), np.linalg.norm(ref, axis=1)
+    err = diff / size
+    assert np.all(err <= ROW_TOL), f"{what}: row {int(np.argmax(err))} of {len(err)}: {np.max(err):.2e}"
+    whole = np.linalg.norm(diff) / np.linalg.norm(size) if alike else np.sqrt(np.mean(err * err))
+    assert whole <= ALL_TOL, f"{what}: {whole:.2e} over all outputs"
 
 
 def tiny_rows(rng, m, k, exponent):
@@ -366,7 +374,7 @@ def test_tiny_f32_activations(mx4, ctx, oracle, m, n, k, exponent):
     for what, w, values in (("mxfp4", wrapped(ctx, packed, scales, 1), oracle.dequantize(packed, scales)),
                             ("bf16", ctx.upload_weight_bf16(bits, n, k), oracle.bf16_to_f32(bits))):
         ctx.matmul(xb, mx4.F32, m, w, y)
-        check_rows(y.download(np.float32).reshape(m, n), x, values, f"{what} m={m} n={n} k={k} 2^{exponent}")
+        check_rows(y.download(np.float32).reshape(m, n), x, values, f"{what} m={m} n={n} k={k} 2^{exponent}", alike=False)
         w.release()
 
 
@@ -483,3 +491,85 @@ def test_group_split_pays(mx4, ctx):
     assert group <= 0.75 * apart, (group, apart)
     for w in ws:
         w.release()
+
+
+def some(rng, count, most):
+    """All of range(count), or its first and last few and a draw."""
+    if count <= most:
+        return np.arange(count)
+    third = most // 3
+    return np.unique(np.r_[0:third, count - third:count, rng.choice(count, third)])
+
+
+def run_instance(mx4, ctx, oracle, fp4, x_bf16, m, rows, k):
+    """One call (a group's for more than one weight) against sums in 64 bits:
+    every output written, none past the end, sampled ones within ROW_TOL, once on
+    plain activations of full mantissas and once, f32, with an inf in one token
+    row and a NaN in another (which show there and nowhere else)."""
+    rng = np.random.default_rng(m + sum(rows) + k)
+    ws, values = [], []
+    for n in rows:
+        cols = some(rng, n, 96)
+        if fp4:
+            packed, scales = planted(rng, n, k)
+            ws.append(wrapped(ctx, packed, scales, n % 4))
+            values.append((cols, oracle.dequantize(packed[cols], scales[cols])))
+        else:
+            bits = rng.integers(0x3c00, 0x3f80, (n, k), dtype=np.uint16) | (rng.integers(0, 2, (n, k), dtype=np.uint16) << 15)
+            ws.append(ctx.upload_weight_bf16(bits, n, k))
+            values.append((cols, oracle.bf16_to_f32(bits[cols])))
+    xt = mx4.BF16 if x_bf16 else mx4.F32
+    ys = [ctx.buffer((m * n + 64) * 4) for n in rows]
+    for odd in (False, True) if xt == mx4.F32 else (False,):
+        xb, x = activations(mx4, ctx, rng, m, k, xt)
+        toks = some(rng, m, 48)
+        if odd:
+            x[toks[1], k // 2], x[toks[-2], k - 1] = np.inf, np.nan
+            xb = ctx.to_device(np.concatenate([x.reshape(-1), np.full(2 * k, np.nan, np.float32)]))
+        for y, n in zip(ys, rows):
+            y.upload(np.full(m * n + 64, 7.0, np.float32))
+        if len(rows) == 1:
+            ctx.matmul(xb, xt, m, ws[0], ys[0])
+        else:
+            ctx.matmul_group(xb.ptr, xt, m, ws, [y.ptr for y in ys])
+        for y, n, (cols, w) in zip(ys, rows, values):
+            out = y.download(np.float32)
+            what = f"fp4={fp4} x_bf16={x_bf16} m={m} rows={rows} n={n} k={k} odd={odd}"
+            assert np.all(out[m * n:] == 7.0), f"{what}: written past the output"
+            out = out[:m * n].reshape(m, n)
+            got = out[np.ix_(toks, cols)]
+            plain = np.ones(len(toks), bool)
+            if odd:
+                plain[[1, -2]] = False
+                assert np.all(np.isnan(got[-2])), what
+                with np.errstate(all="ignore"):
+                    ref = (x[toks[1]].astype(np.float64) * w.astype(np.float64)).sum(1)
+                assert np.array_equal(np.isnan(got[1]), np.isnan(ref)) and np.array_equal(np.isposinf(got[1]), np.isposinf(ref)), what
+                bad = np.delete(out, [toks[1], toks[-2]], 0)
+            else:
+                bad = out
+            assert np.all(np.isfinite(bad)) and np.count_nonzero(bad == 7.0) <= 2, what
+            check_rows(got[plain], x[toks][plain], w, what)
+    for w in ws:
+        w.release()
+
+
+@pytest.mark.parametrize("m,rows,k", sorted({s for (kind, _), shapes in GEMM_SHAPES.items() if kind == "exact" for s in shapes}))
+def test_any_width_gemm_instances(mx4, ctx, oracle, m, rows, k):
+    """Every any-width instance of the exact GEMM, alone and over a group, unsplit
+    and split with short last slices, at ragged rows and columns."""
+    for x_bf16 in (True, False):
+        if (m, rows, k) in GEMM_SHAPES["exact", x_bf16]:
+            run_instance(mx4, ctx, oracle, True, x_bf16, m, rows, k)
+
+
+@pytest.mark.parametrize("m,rows,k", sorted({s for (kind, _), shapes in GEMM_SHAPES.items() if kind == "bf16" for s in shapes}))
+def test_bf16_gemm_instances(mx4, ctx, oracle, m, rows, k):
+    for x_bf16 in (True, False):
+        if (m, rows, k) in GEMM_SHAPES["bf16", x_bf16]:
+            run_instance(mx4, ctx, oracle, False, x_bf16, m, rows, k)
+
+
+@pytest.mark.parametrize("fp4,x_bf16,m,rows,k", list(SKINNY_SHAPES))
+def test_any_width_skinny_instances(mx4, ctx, oracle, fp4, x_bf16, m, rows, k):
+    run_instance(mx4, ctx, oracle, fp4, x_bf16, m, rows, k)
