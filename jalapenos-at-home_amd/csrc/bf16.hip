@@ -98,6 +98,57 @@ __global__ __launch_bounds__(256) void bf16_matmul_kernel(const uint16_t* __rest
     }
 }
 
+// bf16 element e of a 16-byte piece, as f32 bits.
+__device__ __forceinline__ uint32_t half_up(const u32x4& v, int e) { return e % 2 ? v[e / 2] & 0xffff0000u : v[e / 2] << 16; }
+
+// The same for token rows of small weights, which the matrix cores would take
+// longer for: four chains of at most eight products a token row, then sums in 64
+// bits, so that the outputs come out as near to the exact sums as theirs (bf16 x
+// 0.33e-7 relative, f32 0.66e-7 at any K; one chain per lane 0.9e-7 to 1.3e-7 and
+// 1.0e-7 at K = 1024 to 2.6e-7 at 12288). What binds are loads and launch: with all
+// loads of a turn on their way at once it takes no longer than one chain does (1024 x
+// 4096 at 8 rows of f32 7.8 us, 16 x 1024 2.8 or, bf16 x, 2.7 for 2.9).
+template <bool XBF16>
+__global__ __launch_bounds__(256) void bf16_matmul_fine_kernel(const uint16_t* __restrict__ w, const void* __restrict__ x,
+                                                               float* __restrict__ y, uint32_t m, uint32_t n,
+                                                               uint32_t k) {
+    const uint32_t lane = threadIdx.x % 64;
+    const uint32_t row = blockIdx.x * 4 + threadIdx.x / 64;
+    const uint32_t m0 = blockIdx.y * 4;
+    if (row >= n) return;
+    double acc[4] = {};
+    for (uint32_t c0 = lane; c0 < k / 8; c0 += 4 * 64) {
+        float part[4][4] = {};
+        for (uint32_t c = c0; c < k / 8 && c < c0 + 4 * 64; c += 64) {
+            u32x4 xw[4][XBF16 ? 1 : 2];
+            const u32x4 ww = load_u32x4(reinterpret_cast<const uint8_t*>(w) + 2 * ((uint64_t)row * k + 8 * (uint64_t)c));
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const uint32_t tok = m0 + q < m ? m0 + q : m - 1;
+                const uint8_t* xp = static_cast<const uint8_t*>(x) + (XBF16 ? 2 : 4) * ((uint64_t)tok * k + 8 * (uint64_t)c);
+#pragma unroll
+                for (int h = 0; h < (XBF16 ? 1 : 2); ++h) xw[q][h] = load_u32x4(xp + 16 * h);
+            }
+            __builtin_amdgcn_sched_barrier(0);  // every load on its way before the first is waited for
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const float xv = __uint_as_float(XBF16 ? half_up(xw[q][0], e) : xw[q][XBF16 ? 0 : e / 4][e % 4]);
+                    part[q][e % 4] = __builtin_fmaf(xv, __uint_as_float(half_up(ww, e)), part[q][e % 4]);
+                }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            acc[q] += (double)(part[q][0] + part[q][1]);
+            acc[q] += (double)(part[q][2] + part[q][3]);
+        }
+    }
+    const uint32_t q = lane / 16;
+    const double v = wave_sum4(acc, lane);
+    if (lane % 16 == 0 && m0 + q < m) y[(uint64_t)(m0 + q) * n + row] = (float)v;
+}
+
 // One token row. A wave takes a row at a time, U x 512 elements of it per turn
 // (U loads of 1 KiB), the next turn's loads (of this row or its next one) issued
 // before this turn's products; x lies in LDS once per workgroup, filled by
@@ -305,11 +356,19 @@ double bf16_matmul_us(uint32_t m, uint32_t n, uint32_t k, bool x_bf16, int cus) 
 }
 
 hipError_t launch_bf16_matmul(const uint16_t* w, const void* x, bool x_bf16, float* y, uint32_t m, uint32_t n,
-                              uint32_t k, hipStream_t s) {
+                              uint32_t k, bool fine, hipStream_t s) {
     if (m == 0 || n == 0 || k == 0) return hipSuccess;
     // 16-byte pieces need every row (weights and activations) to start 16-byte aligned
     const uint32_t xalign = x_bf16 ? 8 : 4;
     const bool vec = k % 8 == 0 && k % xalign == 0 && ((uintptr_t)w & 15) == 0 && ((uintptr_t)x & 15) == 0;
+    if (vec && fine && m > 1) {
+        dim3 grid((n + 3) / 4, (m + 3) / 4);
+        if (x_bf16)
+            hipLaunchKernelGGL((bf16_matmul_fine_kernel<true>), grid, dim3(256), 0, s, w, x, y, m, n, k);
+        else
+            hipLaunchKernelGGL((bf16_matmul_fine_kernel<false>), grid, dim3(256), 0, s, w, x, y, m, n, k);
+        return hipGetLastError();
+    }
     if (m == 1) return x_bf16 ? go<true, 1>(w, x, y, m, n, k, vec, s) : go<false, 1>(w, x, y, m, n, k, vec, s);
     return x_bf16 ? go<true, 4>(w, x, y, m, n, k, vec, s) : go<false, 4>(w, x, y, m, n, k, vec, s);
 }

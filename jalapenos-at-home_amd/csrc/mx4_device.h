@@ -245,6 +245,19 @@ __device__ __forceinline__ float wave_sum(float v) {
     for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, kWave);
     return v;
 }
+// Wave64 sums of four values at once: every quarter of 16 lanes receives the sum
+// of one, lane/16 its index. Half of what is left goes over with each of the first
+// two steps, 7 exchanges for 24.
+__device__ __forceinline__ double wave_sum4(const double (&v)[4], uint32_t lane) {
+    const bool up = lane & 32u, odd = lane & 16u;
+    double t[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) t[i] = (up ? v[2 + i] : v[i]) + __shfl_xor(up ? v[i] : v[2 + i], 32, kWave);
+    double r = (odd ? t[1] : t[0]) + __shfl_xor(odd ? t[0] : t[1], 16, kWave);
+#pragma unroll
+    for (int off = 8; off >= 1; off >>= 1) r += __shfl_xor(r, off, kWave);
+    return r;
+}
 
 __device__ __forceinline__ u32x4 load_u32x4(const uint8_t* p) {
     return *reinterpret_cast<const u32x4*>(p);

@@ -52,7 +52,8 @@ hipError_t launch_gemv_m1_group(const GemvGroup& g, int cus, const M1Config* for
 bool gemv_mt_supported(uint32_t m, uint32_t k, bool x_bf16);
 // teams / tpw (teams per workgroup): 0 = the default launch shape.
 hipError_t launch_gemv_mt(const GemvArgs& a, int cus, uint32_t teams = 0, uint32_t tpw = 0);
-hipError_t launch_gemv_generic(const GemvArgs& a);
+// fine: m > 1, short chains summed in 64 bits.
+hipError_t launch_gemv_generic(const GemvArgs& a, bool fine);
 // One weight of a width off the tuned ones, m >= 2: does it beat the kernels on the
 // matrix cores that take any width?
 bool generic_faster(uint32_t m, uint32_t n, uint32_t k, bool x_bf16, int cus);
@@ -107,8 +108,9 @@ bool gemm_any_supported(uint32_t m, uint32_t n, uint32_t k, bool x_bf16);
 hipError_t launch_gemm_exact(const GemvArgs& a, int cus, const GemmConfig* forced, float* part, uint64_t part_bytes);
 
 // bf16 weights [n][k] (engine/src/lib.rs:255, None arm), any m, f32 accumulation.
+// fine: m > 1, short chains summed in 64 bits.
 hipError_t launch_bf16_matmul(const uint16_t* w, const void* x, bool x_bf16, float* y, uint32_t m, uint32_t n,
-                              uint32_t k, hipStream_t s);
+                              uint32_t k, bool fine, hipStream_t s);
 // 2 <= m <= 32 over one weight: does it beat launch_skinny_any? And its
 // estimated time in microseconds, for more rows (beside gemm_bf16_us).
 bool bf16_rows_faster(uint32_t m, uint32_t n, uint32_t k, bool x_bf16, int cus);

@@ -357,6 +357,10 @@ mx4_status run_matmul(mx4_context* ctx, const void* x, mx4_dtype xt, uint32_t m,
         // engine/src/lib.rs:255 `None` arm
         if (path != MX4_PATH_AUTO && path != MX4_PATH_GENERIC)
             return fail(MX4_ERR_UNSUPPORTED, "bf16 weights run on the generic path only");
+        // small weights that the row-per-wave kernel takes from the matrix cores are
+        // summed as closely there
+        const bool fine = path == MX4_PATH_AUTO && m >= 2 &&
+                          (bf16_skinny(w, m) || mx4::gemm_bf16_supported(m, w->rows, w->cols, xt == MX4_BF16));
         hipError_t e;
         if (path == MX4_PATH_AUTO && m == 1 && mx4::bf16_gemv_supported(w->cols, xt == MX4_BF16)) {
             e = mx4::launch_bf16_gemv(&w->bf16, &y, &w->rows, 1, x, xt == MX4_BF16, w->cols, ctx->cus, ctx->stream);
@@ -368,14 +372,14 @@ mx4_status run_matmul(mx4_context* ctx, const void* x, mx4_dtype xt, uint32_t m,
             mx4::GemvArgs a{nullptr, nullptr, x, y, m, w->rows, w->cols, xt == MX4_BF16, ctx->stream};
             e = mx4::launch_skinny_any(a, &w->bf16, ctx->cus);
         } else {
-            e = mx4::launch_bf16_matmul(w->bf16, x, xt == MX4_BF16, y, m, w->rows, w->cols, ctx->stream);
+            e = mx4::launch_bf16_matmul(w->bf16, x, xt == MX4_BF16, y, m, w->rows, w->cols, fine, ctx->stream);
         }
         if (e != hipSuccess) return fail(MX4_ERR_DEVICE, "kernel launch failed: %s", hipGetErrorString(e));
         return MX4_OK;
     }
     mx4::GemvArgs a{w->packed, w->scales, x, y, m, w->rows, w->cols, xt == MX4_BF16, ctx->stream};
     const bool chosen = path == MX4_PATH_AUTO;
-    bool any_skinny = false;
+    bool any_skinny = false, fine = false;
     if (chosen) {
         // 2..4 bf16 token rows: the few-token GEMV where it measured faster
         // than the skinny kernel on the Qwen3 1.7B/8B shapes: 2 tokens below
@@ -398,8 +402,10 @@ mx4_status run_matmul(mx4_context* ctx, const void* x, mx4_dtype xt, uint32_t m,
         }
         else if (!small && m > 32 && mx4::gemm_any_supported(m, w->rows, w->cols, xt == MX4_BF16) && scales_foldable(w))
             path = MX4_PATH_GEMM;  // (asked for by name, the path takes K % 128 == 0 only)
-        else
+        else {
             path = MX4_PATH_GENERIC;
+            fine = small && scales_foldable(w);  // what the matrix cores would sum as closely
+        }
     }
     hipError_t e;
     switch (path) {
@@ -431,7 +437,7 @@ mx4_status run_matmul(mx4_context* ctx, const void* x, mx4_dtype xt, uint32_t m,
             e = mx4::launch_gemm_exact(a, ctx->cus, nullptr, ctx->split_part, kSplitPartBytes);
             break;
         case MX4_PATH_GENERIC:
-            e = mx4::launch_gemv_generic(a);
+            e = mx4::launch_gemv_generic(a, fine);
             break;
         default:
             return fail(MX4_ERR_ARGUMENT, "bad path %d", (int)path);

@@ -478,6 +478,61 @@ def test_any_width_small_weights_speed(mx4, ctx, m, n, k):
     w.release()
 
 
+# The same distance on small weights, which kernels without matrix cores take: chains
+# of at most eight products and one 32-bit sum of two of them, then 64 bits. The
+# partial sums' rounding, (1 + .. + 8) / 8 + 1 = 5.5 in units of the last one's
+# variance (2.5e-8 squared: uniform over half a unit of 24 bits, mantissas from 1 to
+# 2), and that of the output make 2.5e-8 6.5^0.5 = 0.65e-7 (measured 0.25 to
+# 0.7e-7); one chain per lane at these K 1.2e-7 and more for f32 activations.
+SMALL_TOL = 0.9e-7
+
+
+@pytest.mark.parametrize("fp4,m,n,k", [(True, 14, 64, 1600), (True, 28, 128, 1600), (True, 16, 256, 8992),
+                                       (True, 32, 128, 8992), (True, 33, 64, 1600), (True, 64, 64, 8992),
+                                       (True, 77, 64, 1056), (False, 2, 512, 8192), (False, 3, 1001, 4096),
+                                       (False, 8, 333, 4096), (False, 24, 64, 12296), (False, 33, 64, 4096),
+                                       (False, 77, 64, 4104)])
+def test_small_weights_precision(mx4, ctx, oracle, fp4, m, n, k):
+    rng = np.random.default_rng(m + n + k)
+    if fp4:
+        packed, scales = planted(rng, n, k)
+        scales = np.full_like(scales, 120)
+        weight, w = ctx.upload_weight(packed, scales, n, k), oracle.dequantize(packed, scales)
+    else:
+        bits = (f32_bits(rng.standard_normal((n, k)).astype(np.float32)) >> 16).astype(np.uint16)
+        weight, w = ctx.upload_weight_bf16(bits, n, k), oracle.bf16_to_f32(bits)
+    for xt in (mx4.BF16, mx4.F32):
+        xb, x = activations(mx4, ctx, rng, m, k, xt)
+        x = x.reshape(m, k).astype(np.float64)
+        y = ctx.to_device(np.full(m * n + 64, 7.0, np.float32))
+        ctx.matmul(xb, xt, m, weight, y)
+        out = y.download(np.float32)
+        assert np.all(out[m * n:] == 7.0)
+        ref = x @ w.astype(np.float64).T
+        err = np.linalg.norm(out[:m * n].reshape(m, n) - ref) / np.linalg.norm(ref)
+        print(f"fp4={fp4} m={m} n={n} k={k} xt={xt}: {err:.2e}", flush=True)
+        assert err <= SMALL_TOL, (fp4, m, n, k, xt, err)
+    weight.release()
+
+
+@pytest.mark.parametrize("m", [1, 3, 5, 29, 77])
+@pytest.mark.parametrize("tiny", ["x", "w"])
+def test_subnormal_bf16_operands(mx4, ctx, oracle, tiny, m):
+    """bf16 activations and bf16 weights, one of them below the normal range: the
+    dot products and matrix cores keep subnormal values."""
+    rng = np.random.default_rng(m)
+    n, k = 200, 1608
+    bits = {}
+    for name, rows in (("x", m), ("w", n)):
+        values = np.ldexp(rng.standard_normal((rows, k)), -130 if name == tiny else 100).astype(np.float32)
+        bits[name] = (f32_bits(values) >> 16).astype(np.uint16)
+    weight, y = ctx.upload_weight_bf16(bits["w"], n, k), ctx.buffer(m * n * 4)
+    ctx.matmul(ctx.to_device(bits["x"]), mx4.BF16, m, weight, y)
+    check_rows(y.download(np.float32).reshape(m, n), oracle.bf16_to_f32(bits["x"]), oracle.bf16_to_f32(bits["w"]),
+               f"tiny {tiny}, m={m}")
+    weight.release()
+
+
 def test_group_split_pays(mx4, ctx):
     """A group of short rows and many outputs is not cut along K, where adding
     the slices would cost more than it saves: well below its members, which are
