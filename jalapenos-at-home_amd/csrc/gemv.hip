@@ -1228,27 +1228,34 @@ static hipError_t launch_generic_t(const GemvArgs& a) {
 // matrix cores' (skinny_any.hip up to 32 token rows, gemm.hip's any-width form
 // beyond)? They take the same time for one tile of weight rows as for a chip full
 // of them; its time is that of its waves, one for each weight row and four token
-// rows, in steps of 2048 of K. From a sweep of 16 to 8192 rows, K = 96 .. 12320, 1
-// to 300 token rows on MI355X (cold weights, recorded passes), us, this kernel /
-// the matrix cores:
-//  * bf16 x, 17 to 32 rows, K > 1024: 256 x 1600 at 32 rows 5.7 / 6.1, 256 x 8992
-//    18.1 / 20.5; 512 x 1600 7.5 / 6.2, 512 x 8992 25.5 / 21; beyond 32 rows 64 x
-//    1600 at 64 4.9 / 7.3, 256 x 1600 7.5 / 7.5, 64 x 8992 at 128 18.2 / 21.5, 256 x
-//    3264 at 64 11.8 / 10.8, 64 x 96 at 33 6.0 / 3.0;
-//  * f32 x, 12 to 32 rows, K > 1024: 256 x 1056 at 16 rows 6.2 / 7.5, 256 x 8992
-//    26 / 29; 512 x 8992 42 / 30 (rows that leave most of the last of several steps
-//    idle gain nothing: 256 x 4288 16.5 / 16.7, 16 x 4288 16.6 / 12.2); beyond 32 rows 64 x
-//    1600 at 33 6.8 / 11.0, 128 x 1600 at 64 9.7 / 11.5, 64 x 8992 at 64 26 / 39,
-//    128 x 8992 at 33 42 / 39.
+// rows, in steps of 64 blocks of K, and a step that is nearly empty takes longer
+// than a full one. From a sweep of 16 to 768 rows, K = 480 .. 8992, 12 to 300 token
+// rows on MI355X (cold weights, recorded passes; no call that comes here is more
+// than 3% slower than the other kernel would be, none that does not more than 10%),
+// us, this kernel / the matrix cores:
+//  * bf16 x: 128 x 1600 at 20 rows 4.7 / 4.8, at 32 4.7 / 5.6, 256 x 1600 at 20
+//    5.4 / 4.9, at 28 5.5 / 5.4; 128 x 3264 at 20 7.4 / 7.5, at 32 7.4 / 9.2, 256 x
+//    5152 at 28 12.2 / 11.3; few blocks in the last step: 128 x 1248 at 28 4.7 /
+//    4.3, 128 x 2592 at 28 7.4 / 6.6. Beyond 32 rows 64 x 1600 at 64 4.8 / 7.3, 256 x
+//    1600 at 64 7.3 / 7.6, 256 x 1056 at 64 7.1 / 6.7; 64 x 8992 at 128 18.8 /
+//    21.5, 256 x 3264 at 64 12.2 / 10.7; 16 x 2080 at 33 9.5 / 7.8;
+//  * f32 x: 256 x 1600 at 14 rows 6.5 / 6.8, at 12 6.5 / 6.1, at 17 9.2 / 7.5; 256 x
+//    8992 at 16 25.9 / 29.1, at 14 25.9 / 26.2; 128 x 8992 at 24 25.9 / 22.5, at 32
+//    25.9 / 26.5; 128 x 2592 at 16 10.2 / 9.5. Beyond 32 rows 64 x 1600 at 33 6.4 /
+//    11.2, 128 x 1600 at 64 9.4 / 11.5, at 100 15.1 / 11.5; 64 x 8992 at 64 25.9 /
+//    39, 128 x 8992 at 33 39 / 39.
 bool generic_faster(uint32_t m, uint32_t n, uint32_t k, bool x_bf16, int cus) {
     const uint64_t waves = (uint64_t)n * ((m + 3) / 4) * 256 / (uint64_t)(cus > 0 ? cus : 256);
     const uint32_t blocks = k / 32, steps = (blocks + 63) / 64;
+    const bool full = 4 * blocks >= 3 * 64 * steps, one = steps == 1;
     if (m <= 32) {
-        if (k <= 1024) return false;
-        return x_bf16 ? m > 16 && waves <= 2048 : m > 11 && waves <= 1024 && (steps == 1 || 4 * blocks >= 3 * 64 * steps);
+        if (k <= 1024 || (!full && (x_bf16 || !one))) return false;
+        if (x_bf16) return one ? m > 16 && waves <= (m > 24 ? 2048u : 1024u) : m > 24 && waves <= 1024;
+        return m > (one ? 13u : 14u) && waves <= (one || m <= 16 || m > 28 ? 1024u : 512u);
     }
-    const bool one_full_step = k > 1024 && k <= 2048;
-    return k >= 448 && waves <= (x_bf16 ? 2048u : 1024u) * (one_full_step ? 2u : 1u);
+    if (k < 448 || (x_bf16 && !one && blocks - 64 * (steps - 1) < 16)) return false;
+    if (one && k > 1024) return waves <= (!x_bf16 ? 2048u : full ? 4096u : 3072u);
+    return waves <= (x_bf16 ? 2048u : 1024u);
 }
 
 hipError_t launch_gemv_generic(const GemvArgs& a, bool fine) {
