@@ -478,6 +478,19 @@ def test_any_width_small_weights_speed(mx4, ctx, m, n, k):
     w.release()
 
 
+@pytest.mark.parametrize("n,k,few,more", [(100, 2080, 16, 20), (256, 1056, 16, 32), (64, 1056, 16, 20), (16, 4288, 16, 17)])
+def test_small_weights_stay_on_matrix_cores(mx4, ctx, n, k, few, more):
+    """Nearly empty steps along K: going from 16 bf16 token rows to the next tile
+    of them costs what it costs on the matrix cores (1.2 to 1.35 times the call),
+    not what the generic kernel would take (1.5 to 1.9)."""
+    w = ctx.synth_weight(n + k, n, k)
+    x, y = ctx.to_device(np.full(more * k, 0x3f80, np.uint16)), ctx.buffer(more * n * 4)
+    a, b = (call_us(ctx, lambda: ctx.matmul(x, mx4.BF16, m, w, y)) for m in (few, more))
+    print(f"n={n} k={k}: m={few} {a:.2f} us, m={more} {b:.2f}", flush=True)
+    assert b <= 1.43 * a, (n, k, a, b)
+    w.release()
+
+
 # The same distance on small weights, which kernels without matrix cores take: chains
 # of at most eight products and one 32-bit sum of two of them, then 64 bits. The
 # partial sums' rounding, (1 + .. + 8) / 8 + 1 = 5.5 in units of the last one's
