@@ -190,7 +190,10 @@ mx4_status mx4_weight_drop_stored(mx4_weight *w);
  * tiled GEMM on bf16 MFMA (MX4_PATH_GEMM) beyond -- the analogue of the
  * reference's M > 32 GEMM (engine/src/matmul.metal:65-97), each in a form for
  * the tuned widths and one for any K % 32 == 0; bf16 weights have a GEMV, a
- * skinny form and a GEMM of their own (K % 8 == 0). Weights with scale bytes
+ * skinny form and a GEMM of their own (K % 8 == 0). Small bf16 weights, and
+ * small ones off the tuned widths, run a kernel without matrix cores where that
+ * is faster (for more than 32 rows also where a group could share a launch, one
+ * weight after the other). Weights with scale bytes
  * outside 2..252 run the exact generic kernel. f32 activations meet the matrix
  * cores as three bf16 terms: every bit of every f32 on the any-width and bf16
  * kernels; on the tuned widths' own (beyond 32 rows K % 128 == 0, and the tuned
