@@ -18,8 +18,8 @@ one by one.
 Algorithmic bytes of one GEMV: N*K/2 (nibbles) + N*K/32 (scales) + M*K*2 (bf16
 x) + M*N*4 (f32 y). value = bytes per step / wall time per step.
 
-stdout is one JSON line, the result; further figures ("extra") go to stderr, a
-line `extra.<name>: {...}` each.
+stdout is one JSON line, the result; further figures ("extra") go to the file
+that --extra names, if any.
 
 Timing protocol of every figure in `extra` (engine/src/model.rs:259-264,
 engine/src/main.rs:70): a recorded pass of distinct weight copies totalling at
@@ -101,12 +101,12 @@ def log(msg: str) -> None:
     print(msg, file=sys.stderr, flush=True)
 
 
-def report(out: dict, extra: dict) -> None:
-    """The result as the one line of stdout, and each entry of `extra` as a line
-    of stderr before it: with the per-shape figures in it the line was 22 KB,
-    more than a reader that keeps the end of the output has left of it."""
-    for name, entry in extra.items():
-        log(f"extra.{name}: {json.dumps(entry)}")
+def report(out: dict, extra: dict, path: str | None = None) -> None:
+    """The result as the one line of stdout, and `extra` as a JSON object in the
+    file `path`, if given: with the per-shape figures the output was 22 KB, more
+    than a reader that keeps the end of it (stdout and stderr alike) has left."""
+    if path:
+        Path(path).write_text(json.dumps(extra, indent=1) + "\n")
     print(json.dumps(out), flush=True)
 
 
@@ -1259,6 +1259,7 @@ def main() -> int:
     ap.add_argument("--profile-verify", action="store_true",
                     help="for kernel traces: only the speculative-verify shapes (each 8B projection and the lm_head "
                          "at M = 1..32 through AUTO over cold copies, enqueued 4 times)")
+    ap.add_argument("--extra", metavar="FILE", help="write the further figures to this file")
     ap.add_argument("--stamp", help="profile modes: also write the stamp (library sha256, workload) to this file")
     ap.add_argument("--summarize", nargs="+", metavar=("KIND", "DIR"),
                     help="print the markdown summary of rocprofv3 CSV output: trace DIR | traffic FETCH_DIR "
@@ -1565,7 +1566,7 @@ def main() -> int:
         "cpu_baseline": cpu,
         "prefill": prefill_top,
     }
-    report(out, extra)
+    report(out, extra, args.extra)
     ctx.synchronize()
     arena.release()
     ctx.close()

@@ -181,15 +181,14 @@ def test_prefill_summary_is_compact_and_reads_the_stamped_counters(tmp_path, mon
     assert len(json.dumps(top)) < 1500
 
 
-def test_result_is_one_short_line(capsys):
-    """stdout holds the result alone, short enough to be read whole from the
-    end of a log; the further figures are lines of stderr."""
+def test_result_is_one_short_line(capsys, tmp_path):
+    """The output is the result alone, short enough to be read whole from the
+    end of a log; the further figures go to a file."""
     out = {"metric": "m", "value": 4250.0, "unit": "GB/s", "ms_per_step": 0.94, "prefill": {"q": [1.0] * 150}}
     extra = {f"section{i}": {f"shape{j}": {"us": 12.345, "GBps": 1234.5} for j in range(60)} for i in range(12)}
-    bench.report(out, extra)
-    got = capsys.readouterr()
-    assert got.out.count("\n") == 1 and len(got.out) < 4096
-    assert json.loads(got.out) == out
-    lines = got.err.splitlines()
-    assert [line.split(": ", 1)[0] for line in lines] == [f"extra.{name}" for name in extra]
-    assert [json.loads(line.split(": ", 1)[1]) for line in lines] == list(extra.values())
+    for path in (None, str(tmp_path / "extra.json")):
+        bench.report(out, extra, path)
+        got = capsys.readouterr()
+        assert got.out.count("\n") == 1 and len(got.out) < 4096 and not got.err
+        assert json.loads(got.out) == out
+    assert json.loads((tmp_path / "extra.json").read_text()) == extra
